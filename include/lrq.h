@@ -240,6 +240,19 @@ int lrq_coo_compact(const void* o, int64_t B, int64_t M, int64_t N, int64_t* ind
 /* Workspace bytes of lrq_coo_compact (>= 0), or a negative LRQ_ERR_*.  Host only. */
 int64_t lrq_coo_workspace(int64_t B, int64_t M, int64_t N);
 
+/* piece_ptr (as lrq_coo_compact writes it, int64 [B*M*ceil(N/64) + 1]) of a coalesced COO tensor
+ * from elsewhere: indices int64 [ndim, n_entries], rows ld_idx apart, the last ndim of (b, m, n) in
+ * row-major order (1 <= ndim <= 3; a missing dimension is 0).  Every pointer lies in [0, n_entries]
+ * whatever the indices hold; entries outside the tensor belong to no piece. */
+int lrq_coo_pieces(const int64_t* indices, int64_t ld_idx, int32_t ndim, int64_t n_entries, int64_t B, int64_t M,
+                   int64_t N, int64_t* piece_ptr, void* stream);
+
+/* The COO invariants of the first min(*nnz, cap) entries (indices as for lrq_coo_pieces): out[0] =
+ * *nnz, and out[1 .. n_out - 1] are all 0 exactly when every entry lies in the tensor and follows its
+ * predecessor in row-major order.  n_out >= 2 sets how many workgroups check. */
+int lrq_coo_check(const int64_t* indices, int64_t ld_idx, int32_t ndim, int64_t cap, const int64_t* nnz, int64_t B,
+                  int64_t M, int64_t N, int64_t* out, int32_t n_out, void* stream);
+
 /* lrq_legacy_encode followed by lrq_coo_compact of its outliers: the reference's encode plus
  * o.to_sparse() (low_rank_extraction_fuse_compression_quantization.py:118-150), without its host
  * synchronisation; codes q, indices, values, *nnz and piece_ptr as the two calls give them.  On the

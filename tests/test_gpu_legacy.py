@@ -553,3 +553,45 @@ def test_legacy_encode_coo_many_chunks(pkg, dev):
     assert torch.equal(q, q2)
     assert torch.equal(oc.piece_ptr, c2.piece_ptr)
     assert torch.equal(oc.indices[:, :n], c2.indices[:, :n]) and torch.equal(oc.values[:n], c2.values[:n])
+
+
+@pytest.mark.parametrize("shape,n", [((1, 1, 1), 0), ((1, 1, 70), 1), ((3, 17, 96), 5), ((2, 33, 4096), 2048 * 33),
+                                     ((2, 33, 4096), 3), ((4, 600, 1000), 50_000), ((1, 2, 65536), 131072)])
+def test_coo_pieces_of_a_sparse_tensor(pkg, dev, shape, n):
+    """Piece pointers rebuilt from a coalesced COO tensor's indices: the number of entries before each
+    64-column piece (chunks of 2048 pieces: none, one, whole, many; rows of 1 to 3 dimensions)."""
+    B, M, N = shape
+    g = torch.Generator().manual_seed(n + M)
+    flat = torch.sort(torch.randperm(B * M * N, generator=g)[:n]).values
+    ind = torch.stack([flat // (M * N), flat // N % M, flat % N])
+    npc = (N + 63) // 64
+    pid = (ind[0] * M + ind[1]) * npc + ind[2] // 64
+    want = torch.searchsorted(pid, torch.arange(B * M * npc + 1))
+    for nd in ([3] if B > 1 else [3, 2, 1] if M == 1 else [3, 2]):
+        sp = torch.sparse_coo_tensor(ind[3 - nd:].to(dev), torch.ones(n, dtype=torch.bfloat16, device=dev),
+                                     shape[3 - nd:], is_coalesced=True)
+        ptr, cols, vals, cnt = pkg.legacy._coo_pieces(sp, B, M, N)
+        assert cnt == n and torch.equal(ptr.cpu(), want) and torch.equal(cols.cpu(), ind[2])
+
+
+@pytest.mark.parametrize("nd,at,row,value", [(3, 4, 2, 64), (3, 0, 0, -1), (3, 70_000, 1, 500), (3, 9, 2, 0),
+                                              (2, 5, 1, 500), (1, 3, 2, 64), (1, 4, 2, -3)])
+def test_sparse_outliers_are_checked(pkg, dev, nd, at, row, value):
+    """to_sparse refuses entries outside the shape, repeated or out of order (one planted, at the
+    first, a middle and the last entry, in rows of 1 to 3 dimensions) and takes the unplanted ones."""
+    B, M, N = (2, 500, 64) if nd == 3 else (1, 500, 64) if nd == 2 else (1, 1, 64)
+    flat = torch.sort(torch.randperm(B * M * N, generator=torch.Generator().manual_seed(1))[:60_000 if nd == 3 else 50]).values
+    n = flat.numel()
+    ind = torch.stack([flat // (M * N), flat // N % M, flat % N]).to(dev)
+    mk = lambda i: pkg.LegacyOutliers(i, torch.ones(n, dtype=torch.bfloat16, device=dev),  # noqa: E731
+                                      torch.tensor([n], device=dev), torch.zeros(1, dtype=torch.int64, device=dev),
+                                      (B, M, N)[3 - nd:])
+    sp = mk(ind).to_sparse()
+    assert sp.is_coalesced() and torch.equal(sp.indices(), ind[3 - nd:])
+    at = min(at, n - 1)
+    bad = ind.clone()
+    bad[row, at] = value if value != 0 else bad[row, at - 1]
+    if value == 0:
+        bad[:, at] = bad[:, at - 1]  # a repeated entry
+    with pytest.raises(RuntimeError):
+        mk(bad).to_sparse()

@@ -76,6 +76,9 @@ SIGNATURES = {
     "lrq_coo_compact": (c_int32, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_int64,
                                   c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "lrq_coo_workspace": (c_int64, [c_int64, c_int64, c_int64]),
+    "lrq_coo_pieces": (c_int32, [c_void_p, c_int64, c_int32, c_int64, c_int64, c_int64, c_int64, c_void_p, c_void_p]),
+    "lrq_coo_check": (c_int32, [c_void_p, c_int64, c_int32, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p,
+                                c_int32, c_void_p]),
     "lrq_legacy_encode_coo": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_int64, c_int64,
                                         c_int64, c_int64, c_void_p, c_int64, c_int32, c_float, c_void_p,
                                         c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,

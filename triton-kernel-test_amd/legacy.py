@@ -62,6 +62,7 @@ __all__ = [
 ]
 
 _OP_STORE, _OP_SILU, _OP_MUL = 0, 1, 2
+_CHECK_WGS = 256  # workgroups of lrq_coo_check (one verdict word each)
 
 
 def _factors(l: torch.Tensor, r: torch.Tensor):
@@ -120,15 +121,46 @@ class LegacyOutliers:
         """Raise if the compaction dropped entries (nnz > capacity); one host synchronisation."""
         n = int(self.nnz.item())
         if n > self.capacity:
-            raise RuntimeError(f"{n} outliers exceed the capacity {self.capacity}; compact again with a larger one")
+            self._overflow(n)
         return self
 
     def to_sparse(self) -> torch.Tensor:
-        """The coalesced sparse COO tensor (one host synchronisation, for the entry count)."""
-        n = int(self.check().nnz.item())
+        """The coalesced sparse COO tensor (one host synchronisation, for the entry count and the
+        check that the entries lie in the tensor in row-major order)."""
+        n, valid = self._count_valid()
+        if n > self.capacity:
+            self._overflow(n)
+        return self._sparse(n, valid)
+
+    def _sparse(self, n: int, valid: Optional[bool]) -> torch.Tensor:
         nd = len(self.shape)
+        # (what _count_valid could not check on the device, torch checks)
+        if valid is False:
+            raise RuntimeError("the outlier indices are not a coalesced COO tensor's: outside the shape or out of order")
         return torch.sparse_coo_tensor(self.indices[3 - nd:, :n], self.values[:n], self.shape, is_coalesced=True,
-                                       check_invariants=True)
+                                       check_invariants=valid is None)
+
+    def _overflow(self, n: int):
+        raise RuntimeError(f"{n} outliers exceed the capacity {self.capacity}; compact again with a larger one")
+
+    def _count_valid(self) -> tuple:
+        """(entry count, whether the entries are a coalesced COO tensor's — None where only torch can
+        tell) in one synchronisation."""
+        ix, nd = self.indices, len(self.shape)
+        dims = _bmn(self.shape) if nd in (1, 2, 3) else (0, 0, 0)
+        plain = (ix.dtype == torch.int64 and ix.is_cuda and ix.dim() == 2 and ix.shape[0] == 3 and ix.stride(1) == 1
+                 and ix.shape[1] >= self.capacity and ix.stride(0) >= ix.shape[1] and self.nnz.dtype == torch.int64
+                 and self.nnz.device == ix.device and self.values.device == ix.device and self.values.dim() == 1
+                 and 0 < dims[1] < 1 << 31 and 0 < dims[2] < 1 << 31 and 1 <= nd <= 3)
+        if not plain:
+            return int(self.nnz.item()), None
+        rows = ix[3 - nd:]
+        out = torch.empty((_CHECK_WGS + 1,), dtype=torch.int64, device=ix.device)
+        with torch.cuda.device(ix.device):
+            call("lrq_coo_check", _p(rows), rows.stride(0), nd, self.capacity, _p(self.nnz), *dims, _p(out),
+                 out.numel(), _stream(ix.device))
+        count, *bad = out.tolist()
+        return count, not any(bad)
 
 
 def _bmn(shape) -> tuple:
@@ -167,17 +199,22 @@ def compact_outliers(o: torch.Tensor, capacity: Optional[int] = None) -> LegacyO
     return LegacyOutliers(bf["idx"], bf["vals"], bf["nnz"], bf["ptr"], tuple(o.shape))
 
 
+def _sparse_or_grow(c: LegacyOutliers, again) -> torch.Tensor:
+    """c.to_sparse(), or that of ``again(n)`` when c's buffers were too small for its n entries."""
+    n, valid = c._count_valid()
+    if n > c.capacity:
+        c = again(n)
+        return c.to_sparse()
+    return c._sparse(n, valid)
+
+
 def _to_sparse(o: torch.Tensor) -> torch.Tensor:
     """``o.to_sparse()`` through the GPU compaction (one synchronisation, as to_sparse has).
     Tensors of more than 3 dimensions are compacted as [prod(leading), M, N] and their leading
     index unravelled afterwards (row-major order is the same)."""
     shape = tuple(o.shape)
     o3 = o.reshape((-1,) + shape[-2:]) if len(shape) > 3 else o
-    c = compact_outliers(o3)
-    n = int(c.nnz.item())
-    if n > c.capacity:
-        c = compact_outliers(o3, capacity=n)
-    sp = c.to_sparse()
+    sp = _sparse_or_grow(compact_outliers(o3), lambda n: compact_outliers(o3, capacity=n))
     if len(shape) <= 3:
         return sp
     lead, rest = sp.indices()[0], []
@@ -194,11 +231,13 @@ def _coo_pieces(o, B: int, M: int, N: int):
         return o.piece_ptr, o.indices[2], o.values, o.capacity
     o = o.coalesce()
     ind = o.indices()
-    b, m, n = ([torch.zeros_like(ind[0])] * (3 - ind.shape[0])) + list(ind)
-    npc = (N + 63) // 64
-    pid = (b * M + m) * npc + torch.div(n, 64, rounding_mode="floor")
-    ptr = torch.searchsorted(pid, torch.arange(B * M * npc + 1, device=pid.device, dtype=torch.int64))
-    return ptr, n.contiguous(), o.values().to(torch.bfloat16).contiguous(), int(n.numel())
+    if not 1 <= ind.shape[0] <= 3:
+        raise ValueError("sparse outliers have 1 to 3 dimensions")
+    if ind.stride(1) != 1 or ind.stride(0) < ind.shape[1]:
+        ind = ind.contiguous()
+    ptr = torch.empty((B * M * ((N + 63) // 64) + 1,), dtype=torch.int64, device=ind.device)
+    call("lrq_coo_pieces", _p(ind), ind.stride(0), ind.shape[0], ind.shape[1], B, M, N, _p(ptr), _stream(ind.device))
+    return ptr, ind[-1], o.values().to(torch.bfloat16).contiguous(), int(ind.shape[1])
 
 
 def _encode_coo(l, r, x, s, bits: int, outlier: float, capacity: Optional[int]):
@@ -235,10 +274,8 @@ def low_rank_addition_fuse_compression_quantization(l, r, x, s, quantize_bit=8, 
     assert r.is_contiguous(), "Matrix B must be contiguous"
     bits = _bits(quantize_bit)
     oc, q = _encode_coo(l, r, x, s, bits, outlier, None)
-    n = int(oc.nnz.item())  # the host synchronisation to_sparse has too
-    if n > oc.capacity:  # more entries than the default buffers hold: again, with room for all
-        oc, q = _encode_coo(l, r, x, s, bits, outlier, n)
-    return oc.to_sparse(), q
+    # more entries than the default buffers hold: again, with room for all (the codes are the same)
+    return _sparse_or_grow(oc, lambda n: _encode_coo(l, r, x, s, bits, outlier, n)[0]), q
 
 
 def legacy_encode_coo(l, r, x, s, quantize_bit=8, outlier=5., capacity: Optional[int] = None):
