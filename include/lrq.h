@@ -194,6 +194,13 @@ int lrq_colmax(const void* x, int64_t ldx, int64_t rows, int64_t hidden, float* 
 /* idx = the k columns with the largest colmax, ascending; ties toward the lower index. */
 int lrq_topk(const float* colmax, int64_t hidden, int32_t k, int32_t* idx, void* stream);
 
+/* The outlier_idx list of an encode, sanitised on the device: out[i] = idx[i] when it lies in
+ * [0, hidden) and no earlier entry has the same value, else -1 (which every kernel skips), and the
+ * side columns [rows, k] (fp16, row stride ld_side) of the -1 entries zeroed.  out may not be idx.
+ * LRQ_ERR_UNSUPPORTED when 4 * (hidden + k) bytes exceed a workgroup's LDS (160 KB). */
+int lrq_outlier_index(const int32_t* idx, int32_t k, int64_t hidden, int32_t* out, int64_t rows, void* side,
+                      int64_t ld_side, void* stream);
+
 /* dst[cols, rows] = src[rows, cols]^T for bf16 (builds Vt from V, and V-layout from the
  * reference's r[K, N] factor). */
 int lrq_transpose_bf16(const void* src, int64_t rows, int64_t cols, void* dst, void* stream);

@@ -41,3 +41,25 @@ def test_colmax_matches_oracle(pkg, dev, rows, hidden):
     torch.cuda.synchronize()
     ref = O.colmax_abs(bits16(x))
     assert np.array_equal(cm.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("k,hidden,rows", [(1, 64, 1), (41, 4096, 300), (257, 512, 16400), (700, 16000, 64),
+                                           (50, 40000, 3), (60, 50000, 70)])
+def test_outlier_index_is_sanitized(pkg, dev, k, hidden, rows):
+    """The device-held channel list: -1 for entries out of range and for repeats of an earlier entry,
+    their side columns zeroed and no other (one and several workgroups, the LDS tables up to and past
+    their limit)."""
+    g = torch.Generator().manual_seed(k)
+    idx = torch.randint(-3, hidden + 3, (k,), generator=g, dtype=torch.int32)
+    idx[k // 2:] = idx[: k - k // 2].clone()  # repeats
+    seen, want = set(), []
+    for c in idx.tolist():
+        want.append(c if 0 <= c < hidden and c not in seen else -1)
+        seen.add(c)
+    side = torch.ones((rows, k), dtype=torch.float16, device=dev)
+    out = pkg.api._sanitize_index(idx.to(dev), hidden, side)
+    assert out.tolist() == want
+    drop = torch.tensor(want) < 0
+    assert not side[:, drop.to(dev)].any()
+    if hidden <= 40000:
+        assert (side[:, ~drop.to(dev)] == 1).all()

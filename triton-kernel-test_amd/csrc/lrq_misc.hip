@@ -263,6 +263,45 @@ extern "C" int lrq_transpose_bf16(const void* src, int64_t rows, int64_t cols, v
   return LRQ_OK;
 }
 
+// The outlier-channel list of an encode, sanitised on the device: out[i] = in[i] when it lies in
+// [0, hidden) and no earlier entry repeats it, else -1, and the side columns of the -1 entries
+// zeroed (the encode writes the others).  Every workgroup finds each column's first entry in LDS
+// (an atomic min per entry) and the dropped entries, workgroup 0 writes the list, and each zeroes
+// its rows' dropped columns.  A launch-bound step: as elementwise passes and a stable sort over k
+// entries it took 15 launches, about 50 us of the host's and the GPU's time per encode; this takes
+// about 4 us.
+constexpr int kIndexThreads = 256;
+__global__ __launch_bounds__(kIndexThreads) void k_outlier_index(const int32_t* __restrict__ in, int k, int hidden,
+                                                                 int32_t* __restrict__ out, int64_t rows,
+                                                                 uint16_t* __restrict__ side, int64_t ldside) {
+  extern __shared__ int32_t first[];  // hidden entries: the first position of each column; then k dropped
+  int32_t* const dropped = first + hidden;
+  __shared__ int ndrop;
+  for (int c = threadIdx.x; c < hidden; c += kIndexThreads) first[c] = INT32_MAX;
+  if (threadIdx.x == 0) ndrop = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < k; i += kIndexThreads) {
+    const int32_t c = in[i];
+    if (c >= 0 && c < hidden) atomicMin(&first[c], i);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < k; i += kIndexThreads) {
+    const int32_t c = in[i];
+    const bool keep = c >= 0 && c < hidden && first[c >= 0 && c < hidden ? c : 0] == i;
+    if (!keep) dropped[atomicAdd(&ndrop, 1)] = i;
+    if (blockIdx.x == 0) out[i] = keep ? c : -1;
+  }
+  __syncthreads();
+  const int nd = ndrop;
+  if (nd == 0) return;  // workgroup-uniform
+  const int64_t per = (rows + gridDim.x - 1) / gridDim.x, r0 = per * blockIdx.x;
+  const int64_t n = max((int64_t)0, min(per, rows - r0)) * nd;
+  for (int64_t i = threadIdx.x; i < n; i += kIndexThreads) {
+    const int64_t r = i / nd;
+    side[(r0 + r) * ldside + dropped[i - r * nd]] = 0;
+  }
+}
+
 // k_colmax launch shape: one workgroup of 8 waves per CU (c3 shape, colmax entry: 36.1 us;
 // 4 waves x 4 per CU 39.3, 8 x 2 40.0, 16 x 1 39.5, 16 x 2 37.6)
 static constexpr int kColmaxPhases = 8, kColmaxWgPerCu = 1;
@@ -303,6 +342,24 @@ extern "C" int lrq_topk(const float* colmax, int64_t hidden, int32_t k, int32_t*
   if (k == 0) return LRQ_OK;
   LRQ_TRY(launch(k_topk, dim3(1), dim3(1024), shm, (hipStream_t)stream, colmax, (int)hidden, (int)k, idx));
   return LRQ_OK;
+}
+
+extern "C" int lrq_outlier_index(const int32_t* idx, int32_t k, int64_t hidden, int32_t* out, int64_t rows, void* side,
+                                 int64_t ld_side, void* stream) {
+  if (idx == nullptr || out == nullptr || (rows > 0 && side == nullptr)) return LRQ_ERR_NULL;
+  if (k < 0 || hidden <= 0 || rows < 0 || ld_side < k) return LRQ_ERR_SHAPE;
+  if (!aligned(idx, 4) || !aligned(out, 4) || !aligned(side, 2)) return LRQ_ERR_ALIGN;
+  // LDS: a word per column and per entry
+  const int64_t shm = 4 * (hidden + (int64_t)k);
+  if (shm + 64 > 160 * 1024) return LRQ_ERR_UNSUPPORTED;
+  if (k == 0) return LRQ_OK;
+  if (shm > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)k_outlier_index, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+    if (e != hipSuccess) return (int)e;
+  }
+  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>((rows + 255) / 256, 64));
+  return launch(k_outlier_index, dim3((unsigned)wgs), dim3(kIndexThreads), (size_t)shm, (hipStream_t)stream, idx, (int)k,
+                (int)hidden, out, rows, (uint16_t*)side, ld_side);
 }
 
 extern "C" const char* lrq_status_string(int status) {
