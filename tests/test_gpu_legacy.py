@@ -595,3 +595,38 @@ def test_sparse_outliers_are_checked(pkg, dev, nd, at, row, value):
         bad[:, at] = bad[:, at - 1]  # a repeated entry
     with pytest.raises(RuntimeError):
         mk(bad).to_sparse()
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+def test_legacy_encode_non_finite_and_huge(pkg, dev, bits):
+    """Infinite and very large activations are outliers of their own and leave every other code and
+    outlier as it is (the encode's matrix steps sum over four elements), in planes with tiny scales
+    too; a NaN changes only its own code."""
+    B, M, N, K, tau = 1, 50, 1024, 16, 5.0
+    l, r, x, s = _inputs(77 + bits, B, M, N, K, 1)
+    s = s.float()
+    s[0, ::7] = 2.0 ** -90
+    s = s.to(torch.bfloat16)
+    x = x.float()
+    nan = [(0, 9, 131), (0, 49, 1023)]
+    for i, (m, n) in enumerate([(3, 5), (3, 6), (17, 700), (31, 64), (49, 0)]):
+        x[0, m, n] = [float("inf"), -float("inf"), 3e38, -3e38, 1e30][i]
+    x = x.to(torch.bfloat16)
+    o_ref, q_ref = O.legacy_encode(bits16(l), bits16(r), bits16(x), bits16(s), bits, tau)
+    xn = x.clone()
+    for i in nan:
+        xn[i] = float("nan")
+    ld, rd, sd = l.to(dev), r.to(dev), s.to(dev)
+    inf = [(0, 3, 5), (0, 3, 6)]  # their own codes come of inf - inf
+    for xi, skip in ((x, inf), (xn, inf + nan)):
+        o_sp, q = pkg.low_rank_addition_fuse_compression_quantization(ld, rd, xi.to(dev), sd, quantize_bit=bits, outlier=tau)
+        qg, og = q.cpu().numpy(), bits16(o_sp.to_dense())
+        ref_q, ref_o = q_ref.copy(), o_ref.copy()
+        for b, m, n in skip:
+            NB = N * bits // 8
+            mask = ((1 << bits) - 1) << (bits * (n // NB))
+            ref_q[b, m, n % NB] = (ref_q[b, m, n % NB] & (0xFF ^ mask)) | (qg[b, m, n % NB] & mask)
+            if (b, m, n) in nan:
+                ref_o[b, m, n] = og[b, m, n]
+        assert np.array_equal(qg, ref_q)
+        assert np.array_equal(O.bf16_to_f32(og), O.bf16_to_f32(ref_o))

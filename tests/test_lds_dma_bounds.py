@@ -1,8 +1,9 @@
 """CPU replay of the direct global-to-LDS loads (ld16_to_lds, csrc/lrq_common.h).
 
-Four kernels move 16 bytes per lane from global memory straight into LDS with
+Five kernels move 16 bytes per lane from global memory straight into LDS with
 __builtin_amdgcn_global_load_lds: k_encode_rows and k_encode_tiles (csrc/lrq_encode.hip),
-k_softmax_rows (csrc/lrq_rowops.hip) and k_wht_rows (csrc/lrq_wht.hip).  This file restates, in numpy, the
+k_softmax_rows (csrc/lrq_rowops.hip), k_wht_rows (csrc/lrq_wht.hip) and k_legacy_encode
+(csrc/lrq_legacy.hip).  This file restates, in numpy, the
 host launch arithmetic (grid, row blocks per workgroup) and each kernel's source and
 destination address arithmetic, and checks for every instance and launch shape that the
 library's callers use (bench.py's configurations and the GPU tests' shapes) that
@@ -268,6 +269,62 @@ def test_wht_rows_direct_loads_stay_in_bounds(cus):
     for rows, N, extra in [(16384, 5120, 0), (20000, 512, 0), (64, 1024, 0), (33, 2048, 0), (100, 4096, 8),
                            (1, 512, 0), (5000, 5120, 0)]:
         n += wht_rows_replay(rows, N, N + extra, cus)
+    assert n > 0
+
+
+# ----------------------------------------------------------------------------- k_legacy_encode
+def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits):
+    """k_legacy_encode<bits, ...> as legacy_launch() launches it: every request of every wave, and the
+    read-back of every slot (lane (j, g): columns 16g .. 16g + 15 of row j)."""
+    NP = 8 // bits
+    NB = N // NP
+    RING, SLOT = 4, 16 * 128
+    WAVE = RING * SLOT + NP * 64 * 4 + 16 * NP * 8
+    nrb, nu = (M + 15) // 16, NB // 64
+    ug = (nu + 3) // 4
+    rbw = max(1, min(16, B * ug * nrb // (4 * cus)))
+    nrun = (nrb + rbw - 1) // rbw
+    lane = np.arange(64)
+    j, g = lane & 15, lane >> 4
+    checked = 0
+    assert 4 * WAVE <= LDS_BYTES
+    for t in range(nrun * ug * B):
+        run, b = (t // ug) % nrun, t // (ug * nrun)
+        rb0 = run * rbw
+        nblk = min(rbw, nrb - rb0)
+        assert nblk >= 1
+        for w in range(4):
+            u = (t % ug) * 4 + w
+            if u * 64 >= NB:
+                continue
+            steps = [(min(st // NP, nblk - 1), st % NP, st) for st in range(RING)]
+            steps += [(min(i + (p + RING) // NP, nblk - 1), (p + RING) % NP, (i * NP + p) % RING)
+                      for i in range(nblk) for p in range(NP)]
+            held = {}
+            for n, (i, p, slot) in enumerate(steps):
+                col = np.empty((16, 8), dtype=np.int64)  # chunk held at each position of each row
+                for k in range(2):
+                    r = 8 * k + lane // 8
+                    row = np.minimum((rb0 + i) * 16 + r, M - 1)
+                    c = u * 64 + 8 * ((lane & 7) ^ (lane >> 3)) + p * NB
+                    gsrc = (b * ldx_b + row * ldx_m + c) * 2
+                    ldst = w * WAVE + slot * SLOT + 1024 * k + 16 * lane
+                    _check(gsrc, ldst, gbytes=((B - 1) * ldx_b + (M - 1) * ldx_m + N) * 2, lds_alloc=4 * WAVE,
+                           lo=w * WAVE + slot * SLOT, hi=w * WAVE + (slot + 1) * SLOT, what=f"k_legacy_encode {M}x{N} {bits}")
+                    col[r, lane & 7] = (c - u * 64 - p * NB) // 8
+                    checked += 64
+                held[slot] = (n, col)
+                for h in range(2):
+                    assert (col[j, (2 * g + h) ^ (j & 7)] == 2 * g + h).all()
+    return checked
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("cus", CU_COUNTS)
+def test_legacy_encode_direct_loads_stay_in_bounds(cus, bits):
+    n = 0
+    for B, M, N, extra in [(1, 1, 512, 0), (2, 100, 1024, 8), (1, 40, 1536, 0), (3, 37, 2048, 0), (1, 2100, 512, 0)]:
+        n += legacy_encode_replay(B, M, N, N + extra, M * (N + extra), cus, bits)
     assert n > 0
 
 

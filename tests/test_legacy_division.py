@@ -18,6 +18,7 @@ import shutil
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 HERE = Path(__file__).resolve().parent
@@ -36,3 +37,37 @@ def test_code_step_forms_give_the_reference_codes(tmp_path):
     # 65280 finite bf16 values
     assert pairs == 2 * (200 * 128 + 1) * 65280
     assert (e1, e2, e4, e8) == (0, 0, 0, 0)
+
+
+def _bf16(f: np.ndarray) -> np.ndarray:
+    """fp32 rounded to bf16 (nearest even), as fp32."""
+    u = f.astype(np.float32).view(np.uint32).astype(np.uint64)
+    u = (u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000
+    return u.astype(np.uint32).view(np.float32)
+
+
+def test_two_term_quotient_gives_the_reference_codes():
+    """The encode's matrix-step quotient: 1/s as two bf16 terms r1 + r2, a r1 (exact) and then a r2
+    added with one fp32 rounding (at 1 bit the threshold 0.5 + 2^-9 enters with a r1, and the sign is
+    the code): its code is the IEEE quotient's for every pair of bf16 mantissas and signs at every
+    exponent difference that can reach a code boundary (|q| from 2^-4 to 2^9; beyond, both clamp)."""
+    man = np.arange(128, 256, dtype=np.float32)
+    a0 = np.concatenate([man, -man])[:, None]
+    for es in (-100, -7, 0, 3, 92):
+        for sg in (1.0, -1.0):
+            s = (sg * man * 2.0 ** es).astype(np.float32)[None, :]
+            rc = (np.float32(1.0) / s).astype(np.float32)
+            r1 = _bf16(rc)
+            r2 = _bf16(rc - r1)
+            for ea in range(-5, 10):
+                a = (a0 * np.float32(2.0) ** (es + ea)).astype(np.float32)
+                q = (a / s).astype(np.float32)
+                p1, p2 = a.astype(np.float64) * r1.astype(np.float64), a.astype(np.float64) * r2.astype(np.float64)
+                t = (p1 + p2).astype(np.float32)
+                for bits in (2, 4, 8):
+                    half = 1 << (bits - 1)
+                    ref = np.clip(np.rint(_bf16(q)), -half, half - 1)
+                    assert np.array_equal(np.clip(np.rint(_bf16(t)), -half, half - 1), ref), (es, ea, bits)
+                one = ((p1 + (0.5 + 2.0 ** -9)).astype(np.float32).astype(np.float64) + p2).astype(np.float32)
+                ref = np.clip(np.rint(_bf16(q)), -1, 0) + 1
+                assert np.array_equal((~np.signbit(one)).astype(np.float32), ref), (es, ea, 1)

@@ -22,8 +22,8 @@
 // (what an fp32-accumulating GEMM returns up to the order of its additions).
 //
 // Two implementations with identical results:
-//   * k_legacy_mfma — when every plane is a whole number of 64-column units and the operands
-//     are 16-byte aligned.  The unit layout of lrq_common.h (lane (j, g) owns 16 consecutive
+//   * k_legacy_encode / k_legacy_mfma — when every plane is a whole number of 64-column units and the
+//     operands are 16-byte aligned.  The unit layout of lrq_common.h (lane (j, g) owns 16 consecutive
 //     columns of its row in every plane) with l @ r rebuilt on MFMA exactly like the
 //     group-mode reconstruction (V = rt).
 //   * k_legacy_scalar — any shape: one thread per packed byte, l @ r summed in fp64 (the
@@ -79,11 +79,10 @@ __device__ __forceinline__ uint32_t legacy_code(float x, float lr, float sc, flo
 }
 
 // The MFMA encode's forms of legacy_code, with the same codes:
-// - the quotient: for scales with 2^-100 <= |sc| <= 2^100 (rc_scale_ok) the one-multiply
-//   estimate a * rc, rc = 1/sc rounded once, instead of the IEEE division: its code equals the
-//   IEEE quotient's at every bit width for every finite bf16 numerator a (a and sc are bf16
-//   values, so a / sc never comes near a code boundary within the estimate's error); other
-//   scales take the IEEE division;
+// - the quotient: for scales with 2^-100 <= |sc| <= 2^100 (rc_scale_ok) a product with 1/sc as two
+//   bf16 terms (legacy_codes_mfma) instead of the IEEE division: its code equals the IEEE quotient's at
+//   every bit width for every finite bf16 numerator a (a and sc are bf16 values, so a / sc never comes
+//   near a code boundary within the product's error); other scales take the IEEE division;
 // - bf16_roundtrip2 rounds two values to bf16 with one conversion;
 // - the code of a bf16 quotient d is legacy_code_biased(d) - kCodeBias + half, where
 //   legacy_code_biased(d) = bits(d + 1.5 * 2^23) clamped to [kCodeBias - half, kCodeBias + half - 1]:
@@ -97,9 +96,9 @@ __device__ __forceinline__ uint32_t legacy_code(float x, float lr, float sc, flo
 // - at 1 bit the code is 1 exactly when bf16(q) >= -0.5, i.e. when q >= -(0.5 + 2^-9) (below
 //   -0.5 the bf16 spacing is 2^-8, and the tie at -0.5 - 2^-9 rounds to the even -0.5): one
 //   compare of the quotient, no rounding.
-// The host check tests/legacy_code_check.c compares the code forms with the reference's over
-// every fp32 quotient but NaN, and the estimate's codes with the IEEE quotient's at 1, 2, 4 and
-// 8 bits over every finite bf16 numerator and every scale the estimate serves.
+// The host checks compare the code forms with the reference's over every fp32 quotient but NaN
+// (tests/legacy_code_check.c) and the two-term product's codes with the IEEE quotient's over every pair
+// of bf16 mantissas (tests/test_legacy_division.py).
 constexpr uint32_t kCodeBias = 0x4B400000u;  // bits of 1.5 * 2^23
 template <int BITS>
 __device__ __forceinline__ uint32_t legacy_code_biased(float d) {
@@ -110,19 +109,18 @@ __device__ __forceinline__ uint32_t legacy_code_biased(float d) {
 constexpr float kOneBitLow = -(0.5f + 0x1p-9f);
 template <int BITS>
 constexpr uint32_t legacy_code_base() {
-  if (BITS == 1) return 0u;  // the 1-bit codes are or-ed in
+  if (BITS == 1) return 0u;  // the complements of the 1-bit codes are or-ed in
   uint32_t k = 0;
   for (int p = 0; p < 8 / BITS; ++p) k += ((1u << (BITS - 1)) - kCodeBias) << (BITS * p);
   return k;
 }
 
-// legacy_code of two elements for the MFMA encode, in the forms above (RC: the estimate of the
-// quotient, else the IEEE division), with one bf16 conversion per rounding step of the pair: at
-// 1 bit the code itself (an outlier leaves a = 0, whose code is 1; otherwise a = xr), at 2, 4
-// and 8 bits biased (legacy_code_biased).
-template <int BITS, bool RC>
-__device__ __forceinline__ void legacy_code_mfma2(const float* x, const float* lr, const float* sc, const float* rc,
-                                                  float tau, float* o, bool* big, uint32_t* code) {
+// legacy_code of two elements in the forms above, with the IEEE division and one bf16 conversion per
+// rounding step of the pair: at 1 bit the code itself (an outlier leaves a = 0, whose code is 1;
+// otherwise a = xr), at 2, 4 and 8 bits biased (legacy_code_biased).
+template <int BITS>
+__device__ __forceinline__ void legacy_code_mfma2(const float* x, const float* lr, const float* sc, float tau, float* o,
+                                                  bool* big, uint32_t* code) {
   float xr[2] = {x[0] - lr[0], x[1] - lr[1]}, q[2];
   bf16_roundtrip2(xr[0], xr[1]);
   if constexpr (BITS == 1) {
@@ -130,8 +128,7 @@ __device__ __forceinline__ void legacy_code_mfma2(const float* x, const float* l
     for (int k = 0; k < 2; ++k) {
       big[k] = fabsf(xr[k]) > tau;
       o[k] = big[k] ? xr[k] : 0.f;
-      const float qk = RC ? xr[k] * rc[k] : xr[k] / sc[k];  // (IEEE division when !RC)
-      code[k] = (big[k] || qk >= kOneBitLow) ? 1u : 0u;
+      code[k] = (big[k] || xr[k] / sc[k] >= kOneBitLow) ? 1u : 0u;
     }
     return;
   }
@@ -139,16 +136,16 @@ __device__ __forceinline__ void legacy_code_mfma2(const float* x, const float* l
   for (int k = 0; k < 2; ++k) {
     big[k] = fabsf(xr[k]) > tau;
     o[k] = big[k] ? xr[k] : 0.f;
-    const float a = xr[k] - o[k];
-    q[k] = RC ? a * rc[k] : a / sc[k];  // (IEEE division when !RC)
+    q[k] = (xr[k] - o[k]) / sc[k];
   }
   bf16_roundtrip2(q[0], q[1]);
   code[0] = legacy_code_biased<BITS>(q[0]);
   code[1] = legacy_code_biased<BITS>(q[1]);
 }
+// (At 1 bit the code comes as a word whose sign bit is its complement, gathered complemented.)
 template <int BITS>
 __device__ __forceinline__ void legacy_accumulate(uint32_t& byte, uint32_t code, int p) {
-  if constexpr (BITS == 1) byte |= code << p;
+  if constexpr (BITS == 1) byte |= (code >> (31 - p)) & (1u << p);
   else byte += code << (BITS * p);
 }
 
@@ -159,6 +156,133 @@ __device__ __forceinline__ uint32_t bf16_at(const u32x4& w0, const u32x4& w1, ui
   const uint32_t lo = (i & 2u) ? w[1] : w[0], hi = (i & 2u) ? w[3] : w[2];
   const uint32_t d = (i & 4u) ? hi : lo;
   return (d >> (16u * (i & 1u))) & 0xffffu;
+}
+
+// The encode's element work on the matrix pipe.  Per element the VALU only rounds, tests and packs:
+// every widening, subtraction and product goes through 4x4x4 MFMA steps (16 blocks of 4 lanes each),
+// whose B operand is 4 elements of the lane itself and whose A operand is diagonal (lane l holds row
+// l % 4, the coefficient of element l % 4), which makes them elementwise:
+//   x - bf16(l r)       A = I on x, then A = -I on bf16(l r) with that as C: one fp32 rounding
+//   q = a r1 + a r2     A = diag r1, then diag r2; 1/s = r1 + r2 to 2^-18 (legacy_rc_split), a r1 exact
+//   d + 1.5 * 2^23      A = I, C = 1.5 * 2^23: the code's biased bits (legacy_code_biased)
+//   q + (0.5 + 2^-9)    at 1 bit the threshold is the first product's C operand, the sign bit the code
+//                       (rounding 17-bit sums to fp32 changes no sign)
+// A sum of two bf16 values (or of two products with a common bf16 factor) is rounded once, so every
+// value is the one the VALU forms above give.  The bf16 tests and masks are packed 16-bit integer
+// operations (two elements each).  An infinite or NaN x would spread over its 4 elements through the
+// zeros of A, and a residual so large that a r2 overflows would meet a r1's infinity: the wave redoes
+// a plane with such a magnitude (mag_limit) with legacy_code_mfma2.  tau >= 0 here.
+// (The packed operations are asm: written as vector code the compiler splits a saturated difference
+// and its test into per-half compares and selects.)
+__device__ __forceinline__ uint32_t pk_sub_sat_u16(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_sub_u16 %0, %1, %2 clamp" : "=v"(r) : "v"(a), "s"(b));
+  return r;
+}
+__device__ __forceinline__ uint32_t pk_min1_u16(uint32_t a, uint32_t one2) {
+  uint32_t r;
+  asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(a), "s"(one2));
+  return r;
+}
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_max_u16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ uint32_t pk_neg_u16(uint32_t a) {
+  uint32_t r;
+  asm("v_pk_sub_u16 %0, 0, %1" : "=v"(r) : "v"(a));
+  return r;
+}
+
+// D(4x4) += A(4x4) * B(4x4) in each of 16 blocks of 4 lanes, bf16 inputs, fp32 accumulate: lane l holds
+// row l % 4 of A, column l % 4 of B and of D.
+__device__ __forceinline__ f32x4 mfma_4x4x4(u32x2 a, u32x2 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+}
+// The diagonal A operand of that step with bf16 bits `v` in this lane's row.
+__device__ __forceinline__ u32x2 diag4_aop(int lane, uint32_t v) {
+  const uint32_t d = v << (16u * (lane & 1));
+  return (lane & 2) ? u32x2{0u, d} : u32x2{d, 0u};
+}
+// Selectors (v_perm_b32) that place the low (hi = 0) or high half of a dword as diag4_aop does.
+__device__ __forceinline__ u32x2 diag4_sel(int lane, int hi) {
+  const uint32_t h = hi ? 0x0302u : 0x0100u, d = (lane & 1) ? (h << 16) | 0x0c0cu : 0x0c0c0000u | h;
+  return (lane & 2) ? u32x2{0x0c0c0c0cu, d} : u32x2{d, 0x0c0c0c0cu};
+}
+// 1/s as the sum of two bf16 terms (relative error at most 2^-18 + 2^-24: a quotient of two bf16
+// values is at least 2^-17 from a code boundary, relative).
+__device__ __forceinline__ void legacy_rc_split(float sc, uint32_t& r1, uint32_t& r2) {
+  const float rc = 1.0f / sc;
+  r1 = pack_bf16x2(rc, 0.f);
+  r2 = pack_bf16x2(rc - __uint_as_float(r1 << 16), 0.f);
+}
+
+// fp32(l r) of the lane's 16 columns of one plane (step q: elements 4q .. 4q + 3).
+template <int K>
+__device__ __forceinline__ void legacy_lowrank_mfma(const u32x2 (&vop)[4][K / 16], const u32x2* lop, f32x4 (&t)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (K == 16) {
+      t[q] = mfma_16x16x16(vop[q][0], lop[0], zero4());
+    } else {
+      t[q] = mfma_16x16x32(u32x4{vop[q][0][0], vop[q][0][1], vop[q][1][0], vop[q][1][1]},
+                           u32x4{lop[0][0], lop[0][1], lop[1][0], lop[1][1]}, zero4());
+    }
+  }
+}
+
+// The plane's outlier test and codes from the packed residuals w (w[k]: elements 2k, 2k + 1): hm bit e =
+// element e is an outlier, w becomes the outlier values (0 elsewhere), code[16] the codes
+// (legacy_code_biased; at 1 bit a word whose sign bit is the code's complement).  Returns whether some
+// magnitude of the lane reaches mag_limit (bf16 bits): hm, w and code are then unspecified.  aq: the LDS table of the plane's quotient operands (step q's two terms at aq[128 q],
+// aq[128 q + 64]).
+template <int BITS>
+__device__ __forceinline__ bool legacy_codes_mfma(uint32_t (&w)[8], uint32_t tau2, uint32_t mag_limit, u32x4 rc, int lane,
+                                                  uint32_t (&code)[16], uint32_t& hm) {
+  uint32_t a[8], mag[8], h2 = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) mag[k] = w[k] & 0x7fff7fffu;
+  const uint32_t t0 = pk_max_u16(pk_max_u16(mag[0], mag[1]), pk_max_u16(mag[2], mag[3]));
+  const uint32_t t1 = pk_max_u16(pk_max_u16(mag[4], mag[5]), pk_max_u16(mag[6], mag[7]));
+  const uint32_t top = pk_max_u16(t0, t1);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t one = pk_min1_u16(pk_sub_sat_u16(mag[k], tau2), 0x00010001u);  // 1 where |xr| > tau
+    h2 |= one << (2 * k);  // bits 2k (element 2k) and 16 + 2k (element 2k + 1)
+    const uint32_t m = pk_neg_u16(one);
+    a[k] = w[k] & ~m;
+    w[k] &= m;
+  }
+  hm = (h2 & 0xffffu) | (h2 >> 15);
+  f32x4 t[4];
+  constexpr float c0 = BITS == 1 ? -kOneBitLow : 0.f;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const u32x2 sel = diag4_sel(lane, h);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const u32x2 ra = u32x2{__builtin_amdgcn_perm(rc[q], rc[q], sel[0]), __builtin_amdgcn_perm(rc[q], rc[q], sel[1])};
+      t[q] = mfma_4x4x4(ra, u32x2{a[2 * q], a[2 * q + 1]}, h == 0 ? f32x4{c0, c0, c0, c0} : t[q]);
+    }
+  }
+  if constexpr (BITS == 1) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) code[e] = __float_as_uint(t[e >> 2][e & 3]);
+  } else {
+    constexpr float mg = 0x1.8p23f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      t[q] = mfma_4x4x4(diag4_aop(lane, 0x3f80u), u32x2{pack_bf16x2(t[q][0], t[q][1]), pack_bf16x2(t[q][2], t[q][3])},
+                        f32x4{mg, mg, mg, mg});
+    constexpr int half = 1 << (BITS - 1);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int v = (int)__float_as_uint(t[e >> 2][e & 3]);
+      code[e] = (uint32_t)min(max(v, (int)kCodeBias - half), (int)kCodeBias + half - 1);
+    }
+  }
+  return (top >> 16) >= mag_limit || (top & 0xffffu) >= mag_limit;
 }
 
 // Scales whose reciprocal estimate gives legacy_code's codes (NaN fails the test).
@@ -284,8 +408,7 @@ __device__ __forceinline__ void coo_tile(const LegacyArgs& a, int64_t (&s0)[NP],
 // entries (a piece's entries do not start on a line boundary), of the code rows and of the output
 // rows.  Wave w walks row blocks (bx * rb + i) * 64 + w * 16, i < rb, of unit u.  OSRC, decode: outliers
 // absent (0), dense (1) or COO pieces (2: looked up per lane, for sparse outliers; 3: gathered
-// per wave into an LDS tile, for denser ones); encode: 1 writes each 64-column piece's staged
-// record (a.pcnt; lrq_coo.h) and the dense outliers only of the pieces it cannot hold.
+// per wave into an LDS tile, for denser ones).
 template <int MODE, int BITS, int K, int OSRC>
 __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
   constexpr int NP = (MODE == kAdd || MODE == kHist) ? 1 : 8 / BITS, G = 64, E = 16, RT = K / 16;
@@ -316,34 +439,12 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
   for (int p = 0; p < NP; ++p) load_vops<G, K>(a.rt, unit_base(p, u, N, NP, G), j, g, vop[p]);
   const float zero[E] = {};
 
-  // the unit's scales in LDS for every row block of the workgroup (the same columns throughout),
-  // and for the encode their reciprocals (one IEEE division per column); rc_ok: every scale is
-  // the reciprocal estimate serves exactly
+  // the unit's scales in LDS for every row block of the workgroup (the same columns throughout)
   constexpr bool kScales = MODE != kAdd && MODE != kHist;
-  __shared__ __attribute__((aligned(16))) float stab[MODE == kEncode ? 2 * NP * G : (kScales ? NP * G : 4)];
-  bool rc_ok = false;
+  __shared__ __attribute__((aligned(16))) float stab[kScales ? NP * G : 4];
   if constexpr (kScales) {
-    int ok = 1;
-    for (int i = threadIdx.x; i < NP * G; i += 256) {
-      const int p = i / G, c = i % G;
-      const float sv = bf_lo(srow[unit_base(p, u, N, NP, G) + c]);
-      stab[i] = sv;
-      if constexpr (MODE == kEncode) {
-        stab[NP * G + i] = 1.0f / sv;
-        ok &= rc_scale_ok(sv) ? 1 : 0;
-      }
-    }
-    if constexpr (MODE == kEncode) {
-      // every thread's ok, as __syncthreads_and (whose device-library reduction is not inlined
-      // here): one ballot per wave, the 4 waves' results through LDS
-      __shared__ uint32_t wave_ok[4];
-      const bool all = __builtin_amdgcn_ballot_w64(ok == 0) == 0;
-      if (lane == 0) wave_ok[w] = all ? 1u : 0u;
-      __syncthreads();
-      rc_ok = (wave_ok[0] & wave_ok[1] & wave_ok[2] & wave_ok[3]) != 0;
-    } else {
-      __syncthreads();
-    }
+    for (int i = threadIdx.x; i < NP * G; i += 256) stab[i] = bf_lo(srow[unit_base(i / G, u, N, NP, G) + i % G]);
+    __syncthreads();
   }
 
   // decode from the COO tile: the next row block's L operand, codes and COO piece bounds are
@@ -363,24 +464,6 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
     if constexpr (MODE == kDecode && OSRC == 3) coo_bounds<NP>(a, (int64_t)b * M + rn, u, N, ns0, ns1);
   };
   if constexpr (kPre) fetch_next(0);
-  // encode at 2 bits and more: the next row block's x (and L operand) is requested before the
-  // current block is computed (nx carries it over; at 1 bit its 64 registers would halve the
-  // waves per SIMD)
-  constexpr bool kPreX = MODE == kEncode && NP <= 4;
-  u32x4 nx[kPreX ? NP : 1][2];
-  auto fetch_x = [&](int i) __attribute__((always_inline)) {
-    const int64_t rn = min((bx * a.rb + i) * 64 + w * 16 + j, M - 1);
-#pragma unroll
-    for (int t = 0; t < RT; ++t) nl[t] = ld8(a.l + rn * K + 16 * t + 4 * g);
-#pragma unroll
-    for (int p = 0; p < (kPreX ? NP : 1); ++p) {
-      const uint16_t* xp = a.x + (int64_t)b * a.ldx_b + rn * a.ldx_m + unit_base(p, u, N, NP, G) + E * g;
-      nx[p][0] = ld16(xp);
-      nx[p][1] = ld16(xp + 8);
-    }
-  };
-  if constexpr (kPreX) fetch_x(0);
-
   for (int i = 0; i < a.rb; ++i) {
     const int row0 = (bx * a.rb + i) * 64 + w * 16;  // wave-uniform: a scalar exit
     if (row0 >= M) break;  // whole 16-row block past the end
@@ -400,26 +483,11 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
         s1[q] = ns1[q];
       }
       fetch_next(min(i + 1, a.rb - 1));  // (the last block fetches itself again: unused)
-    } else if constexpr (kPreX) {
-#pragma unroll
-      for (int t = 0; t < RT; ++t) lop[t] = nl[t];
     } else {
 #pragma unroll
       for (int t = 0; t < RT; ++t) lop[t] = ld8(a.l + rr * K + 16 * t + 4 * g);
       if constexpr (kCodes) qb = ld16(a.qin + ((int64_t)b * M + rr) * NB + u * G + E * g);
     }
-    u32x4 cx[kPreX ? NP : 1][2];
-    if constexpr (kPreX) {
-#pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        cx[p][0] = nx[p][0];
-        cx[p][1] = nx[p][1];
-      }
-      fetch_x(min(i + 1, a.rb - 1));  // (the last block fetches itself again: unused)
-    }
-    uint32_t byte[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) byte[e] = MODE == kEncode ? legacy_code_base<BITS>() : 0u;
     uint16_t* ot = otile + (size_t)w * 16 * coo_row_stride<NP>();
     if constexpr (MODE == kDecode && OSRC == 3) coo_tile<NP, kCooEntriesPerLane>(a, s0, s1, u, N, j, g, ot);
 
@@ -430,20 +498,8 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
       residual_unit<G, K>(vop[p], lop, zero, lr);
 #pragma unroll
       for (int e = 0; e < E; e += 2) bf16_roundtrip2(lr[e], lr[e + 1]);
-      float sc[E], rc[E];
-      if constexpr (MODE == kEncode) {
-        const float* sp = stab + p * G + E * g;
-#pragma unroll
-        for (int k = 0; k < E; k += 4) {
-          const f32x4 v = *reinterpret_cast<const f32x4*>(sp + k);
-          const f32x4 w = *reinterpret_cast<const f32x4*>(sp + NP * G + k);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sc[k + e] = v[e];
-            rc[k + e] = w[e];
-          }
-        }
-      } else if constexpr (kScales) {
+      float sc[E];
+      if constexpr (kScales) {
         const float* sp = stab + p * G + E * g;
 #pragma unroll
         for (int k = 0; k < E; k += 4) {
@@ -464,80 +520,16 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
             if (bin >= 0) atomicAdd(&lh[bin], 1u);
           }
         }
-      } else if constexpr (MODE == kEncode || MODE == kAdd) {
+      } else if constexpr (MODE == kAdd) {
+        const uint16_t* xp = a.x + (int64_t)b * a.ldx_b + rr * a.ldx_m + c0;
         float xv[E];
-        if constexpr (kPreX) {
-          unpack8(cx[p][0], xv);
-          unpack8(cx[p][1], xv + 8);
-        } else {
-          const uint16_t* xp = a.x + (int64_t)b * a.ldx_b + rr * a.ldx_m + c0;
-          unpack8(ld16(xp), xv);
-          unpack8(ld16(xp + 8), xv + 8);
-        }
-        if constexpr (MODE == kEncode) {
-          // legacy_code of each element in the forms above, two at a time (legacy_code_mfma2)
-          float ov[E];
-          uint32_t hm = 0;  // bit e: element e is an outlier entry
-          if (rc_ok) {  // workgroup-uniform
+        unpack8(ld16(xp), xv);
+        unpack8(ld16(xp + 8), xv + 8);
+        float ov[E];
 #pragma unroll
-            for (int e = 0; e < E; e += 2) {
-              bool hit[2];
-              uint32_t cd[2];
-              legacy_code_mfma2<BITS, true>(xv + e, lr + e, sc + e, rc + e, a.tau, ov + e, hit, cd);
-              legacy_accumulate<BITS>(byte[e], cd[0], p);
-              legacy_accumulate<BITS>(byte[e + 1], cd[1], p);
-              hm |= (hit[0] ? 1u << e : 0u) | (hit[1] ? 2u << e : 0u);
-            }
-          } else {
-#pragma unroll
-            for (int e = 0; e < E; e += 2) {
-              bool hit[2];
-              uint32_t cd[2];
-              legacy_code_mfma2<BITS, false>(xv + e, lr + e, sc + e, rc + e, a.tau, ov + e, hit, cd);
-              legacy_accumulate<BITS>(byte[e], cd[0], p);
-              legacy_accumulate<BITS>(byte[e + 1], cd[1], p);
-              hm |= (hit[0] ? 1u << e : 0u) | (hit[1] ? 2u << e : 0u);
-            }
-          }
-          const u32x4 ow0 = pack8(ov), ow1 = pack8(ov + 8);
-          if constexpr (OSRC == 1) {
-            // the piece's staged record (lrq_coo.h): its count and first kCooSlots entries, over
-            // the row's four lanes (lane g holds the piece's columns 16g .. 16g+15); its dense
-            // values only when the record cannot hold them
-            const uint32_t n = __builtin_popcount(hm);
-            uint32_t pre, total;
-            row_prefix4(n, g, pre, total);
-            const uint32_t i0 = __builtin_ctz(hm | 0x10000u) & 15u, h1 = hm & (hm - 1u);
-            const uint32_t i1 = __builtin_ctz(h1 | 0x10000u) & 15u;
-            const uint32_t e0 = ((uint32_t)(16 * g) + i0) | (bf16_at(ow0, ow1, i0) << 16);
-            const uint32_t e1 = ((uint32_t)(16 * g) + i1) | (bf16_at(ow0, ow1, i1) << 16);
-            static_assert(kCooSlots == 2, "two entries per record");
-            uint32_t d0 = pre == 0u && n >= 1u ? e0 : 0u;
-            uint32_t d1 = pre == 0u && n >= 2u ? e1 : pre == 1u && n >= 1u ? e0 : 0u;
-            d0 = row_or4(d0);
-            d1 = row_or4(d1);
-            // lane g = 0 of each row stores the record through a range-checked store (the other
-            // lanes' offsets fall outside the range: no branch)
-            int64_t* prow = a.pcnt + ((int64_t)b * M + row0) * a.npc;  // the block's first row
-            st8_pred(prow, (uint32_t)(16 * a.npc * 8),
-                     (uint32_t)(((rr - row0) * a.npc + unit_base(p, u, N, NP, G) / 64) * 8),
-                     u32x2{d0 | total << 8, d1}, g == 0 && row < M);
-            uint16_t* orow = a.oout + ((int64_t)b * M + row0) * N;
-            const uint32_t olen = (uint32_t)(16 * N * 2), ooff = (uint32_t)(((rr - row0) * N + c0) * 2);
-            const bool dense = total > (uint32_t)kCooSlots && row < M;
-            st16_pred(orow, olen, ooff, ow0, dense);
-            st16_pred(orow, olen, ooff + 16, ow1, dense);
-          } else {
-            st16(a.oout + erow + c0, ow0);
-            st16(a.oout + erow + c0 + 8, ow1);
-          }
-        } else {
-          float ov[E];
-#pragma unroll
-          for (int e = 0; e < E; ++e) ov[e] = xv[e] + lr[e];  // fp32 add, then bf16 (pack8), as torch
-          st16(a.out + erow + c0, pack8(ov));
-          st16(a.out + erow + c0 + 8, pack8(ov + 8));
-        }
+        for (int e = 0; e < E; ++e) ov[e] = xv[e] + lr[e];  // fp32 add, then bf16 (pack8), as torch
+        st16(a.out + erow + c0, pack8(ov));
+        st16(a.out + erow + c0 + 8, pack8(ov + 8));
       } else {
         float ov[E], oo[E], yv[E];
         if constexpr (MODE == kDecode && OSRC == 1) {
@@ -564,17 +556,239 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
         st16(a.out + erow + c0 + 8, pack8(ov + 8));
       }
     }
-    if constexpr (MODE == kEncode) {
-      uint32_t word[E / 4];
-#pragma unroll
-      for (int k = 0; k < E / 4; ++k) word[k] = gather_bytes(byte[4 * k], byte[4 * k + 1], byte[4 * k + 2], byte[4 * k + 3]);
-      st16(a.qout + ((int64_t)b * M + rr) * NB + u * G + E * g, u32x4{word[0], word[1], word[2], word[3]});
-    }
   }
   if constexpr (MODE == kHist) {
     __syncthreads();
     if (lh[threadIdx.x] != 0u) atomicAdd(&a.hist[threadIdx.x], lh[threadIdx.x]);
   }
+}
+
+// ------------------------------------------------------------------ MFMA encode
+// Independent waves (no barrier), four to a workgroup on four neighbouring units of the same rows: wave
+// w of tile (batch, run, unit group), unit groups fastest, in XCD order (xcd_tile), takes unit 4 * group +
+// w over RBW 16-row blocks.  x streams through a private LDS ring of four (row block, plane) slots,
+// 16 rows x 128 bytes each, straight from HBM (two 1 KB loads of eight whole lines; slot position c of
+// row r holds chunk c ^ (r % 8), so that reading it back in the MFMA layout spreads over the banks); a
+// slot is requested again, four planes on, as soon as the wave has read it.  A skeleton with these
+// accesses and stores moves the 604 MB of [4, 8192, 8192] at 2 bits in 126 us; loads in the MFMA
+// layout, four row blocks of one unit per workgroup, took 162 - 176 us.  The encode itself runs 152 us
+// there (218 us in that layout with the element work on the VALU; 184 us with it on the matrix pipe),
+// 155 us at 1 bit (202 us).
+// STAGED: each 64-column piece's record (lrq_coo.h) goes to a.pcnt and the dense outliers only of the
+// pieces it cannot hold; else the dense outliers.  A block's 16 NP records are gathered in LDS, each
+// lane writing the entries it holds (usually none or one: the or of its masked values), and leave
+// as one 8-byte store per record.
+template <int BITS>
+struct LegacyEnc {
+  static constexpr int NP = 8 / BITS, NW = 4, RING = 4, SLOT = 16 * 128, NREC = 16 * NP;
+  static constexpr int TAB = NP * 64 * 4, WAVE = RING * SLOT + TAB + NREC * 8;  // bytes per wave
+  static constexpr int kStepOps = 4;  // memory operations per step: two loads, two (dense outlier) stores
+};
+template <int BITS, int K, bool STAGED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1 : BITS >= 2 && K == 16 ? 3 : 2))) void k_legacy_encode(
+    LegacyArgs a, int RBW, int ug) {
+  using Le = LegacyEnc<BITS>;
+  constexpr int NP = Le::NP, G = 64, E = 16, RT = K / 16, RING = Le::RING, SLOT = Le::SLOT, NREC = Le::NREC;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[Le::NW][Le::WAVE];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int j = lane & 15, g = lane >> 4;
+  const int M = (int)a.M, N = (int)a.N, nrb = (M + 15) / 16, nrun = (nrb + RBW - 1) / RBW;
+  const int t = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x));
+  const int u = __builtin_amdgcn_readfirstlane(t % ug) * Le::NW + w;
+  const int run = __builtin_amdgcn_readfirstlane((t / ug) % nrun), b = __builtin_amdgcn_readfirstlane(t / (ug * nrun));
+  const int64_t NB = N / NP;  // bytes per code row
+  if (u * G >= NB) return;    // the group's last units (this wave only)
+  const int rb0 = run * RBW, nblk = min(RBW, nrb - rb0);
+  unsigned char* const ring = lds[w];
+  uint32_t* const rtab = reinterpret_cast<uint32_t*>(ring + RING * SLOT);  // [NP][16 (g, j % 4)][4 steps]
+  u32x2* const recs = reinterpret_cast<u32x2*>(ring + RING * SLOT + Le::TAB);
+  const uint16_t* srow = a.s + (a.s_rows == 1 ? 0 : (int64_t)b * N);
+
+  // step st = (block st / NP, plane st % NP): slot st % RING.  Load k covers rows 8k .. 8k + 7 of the
+  // block (rows past the end clamp to the last), lane l chunk (l % 8) ^ (row % 8) of row 8k + l / 8.
+  const uint16_t* const xbase = a.x + (int64_t)b * a.ldx_b + u * G + 8 * ((lane & 7) ^ (lane >> 3));
+  auto request = [&](int i, int p, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int64_t row = min((rb0 + i) * 16 + 8 * k + (lane >> 3), M - 1);
+      ld16_to_lds(xbase + row * a.ldx_m + p * NB, ring + slot * SLOT + 1024 * k);
+    }
+  };
+#pragma unroll
+  for (int st = 0; st < RING; ++st) request(min(st / NP, nblk - 1), st % NP, st);
+  u32x2 nl[RT];
+  auto fetch_l = [&](int i) __attribute__((always_inline)) {
+    const int64_t rn = min((rb0 + i) * 16 + j, M - 1);
+#pragma unroll
+    for (int k = 0; k < RT; ++k) nl[k] = ld8(a.l + rn * K + 16 * k + 4 * g);
+  };
+  fetch_l(0);
+  u32x2 vop[NP][4][RT];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) load_vops<G, K>(a.rt, unit_base(p, u, N, NP, G), j, g, vop[p]);
+  // fast: the estimate serves every scale of the unit and the threshold is not negative
+  int ok = a.tau >= 0.f ? 1 : 0;
+  float smin = INFINITY;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const float sv = bf_lo(srow[unit_base(p, u, N, NP, G) + lane]);
+    smin = fminf(smin, fabsf(sv));
+    uint32_t r1, r2;
+    legacy_rc_split(sv, r1, r2);
+    // column c = 16g' + 4q + v of the unit: entry [g'][v][q]
+    rtab[p * 64 + ((lane >> 4) * 4 + (lane & 3)) * 4 + ((lane >> 2) & 3)] = r1 | (r2 << 16);
+    ok &= rc_scale_ok(sv) ? 1 : 0;
+  }
+  const bool fast = __builtin_amdgcn_ballot_w64(ok == 0) == 0;  // wave-uniform
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) smin = fminf(smin, __shfl_xor(smin, d));
+  // magnitudes below 2^118 min |s| keep every quotient below 2^119 (at most the bits of infinity)
+  const uint32_t mag_limit = __builtin_amdgcn_readfirstlane(__float_as_uint(smin * 0x1p118f) >> 16);
+  const u32x2 ida = diag4_aop(lane, 0x3f80u), idn = diag4_aop(lane, 0xbf80u);  // I, -I
+  const uint32_t tau2 = (__float_as_uint(a.tau) >> 16) * 0x10001u;
+  // the prologue's loads have landed (the counted waits below start from none outstanding)
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  __builtin_amdgcn_sched_barrier(0);
+
+#pragma unroll 1
+  for (int i = 0; i < nblk; ++i) {
+    const int row0 = (rb0 + i) * 16;
+    const int row = row0 + j;
+    const int64_t rr = min(row, M - 1);
+    u32x2 lop[RT];
+#pragma unroll
+    for (int k = 0; k < RT; ++k) lop[k] = nl[k];
+    fetch_l(min(i + 1, nblk - 1));
+    uint32_t byte[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) byte[e] = legacy_code_base<BITS>();
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int k = 0; k < (NREC + 63) / 64; ++k)
+        if (64 * k + lane < NREC) recs[64 * k + lane] = u32x2{0u, 0u};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, NP>([&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+      const int c0 = unit_base(p, u, N, NP, G) + E * g;
+      const int slot = (i * NP + p) % RING;
+      // The slot's loads were issued RING steps ago; the RING - 1 steps between issued kStepOps memory
+      // operations each (and the blocks' own loads and stores besides), and memory operations retire
+      // in issue order.
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 1) * Le::kStepOps));
+      __builtin_amdgcn_sched_barrier(0);
+      const unsigned char* xs = ring + slot * SLOT + 128 * j;
+      const u32x4 x0 = *reinterpret_cast<const u32x4*>(xs + 16 * ((2 * g) ^ (j & 7)));
+      const u32x4 x1 = *reinterpret_cast<const u32x4*>(xs + 16 * ((2 * g + 1) ^ (j & 7)));
+      const u32x4 rc = *reinterpret_cast<const u32x4*>(rtab + p * 64 + (g * 4 + (j & 3)) * 4);
+      f32x4 tl[4], tx[4];
+      legacy_lowrank_mfma<K>(vop[p], lop, tl);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slot is read
+      __builtin_amdgcn_sched_barrier(0);
+      // (past the run the last block is requested again: unused)
+      request(min(i + (p + RING) / NP, nblk - 1), (p + RING) % NP, slot);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 x = q < 2 ? x0 : x1;
+        tx[q] = mfma_4x4x4(ida, u32x2{x[2 * (q & 1)], x[2 * (q & 1) + 1]}, zero4());
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        tx[q] = mfma_4x4x4(idn, u32x2{pack_bf16x2(tl[q][0], tl[q][1]), pack_bf16x2(tl[q][2], tl[q][3])}, tx[q]);
+      uint32_t ow[8];   // the residuals, then the outlier values, packed
+      uint32_t hm = 0;  // bit e: element e is an outlier entry
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        ow[2 * q] = pack_bf16x2(tx[q][0], tx[q][1]);
+        ow[2 * q + 1] = pack_bf16x2(tx[q][2], tx[q][3]);
+      }
+      uint32_t code[E];
+      bool slow = true;
+      if (fast) slow = __builtin_amdgcn_ballot_w64(legacy_codes_mfma<BITS>(ow, tau2, mag_limit, rc, lane, code, hm)) != 0;
+      if (slow) {
+        // scales the estimate does not serve, a negative threshold, or an x (or residual) that is not
+        // finite in the wave's plane: legacy_code of each element, two at a time
+        float lr[E], xv[E], ov[E];
+        const uint16_t* xp = a.x + (int64_t)b * a.ldx_b + rr * a.ldx_m + c0;
+        unpack8(ld16(xp), xv);
+        unpack8(ld16(xp + 8), xv + 8);
+        legacy_lowrank_mfma<K>(vop[p], lop, tl);
+        hm = 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) lr[e] = tl[e >> 2][e & 3];
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+          const uint32_t sw = ld4(srow + c0 + e);
+          const float sc[2] = {bf_lo(sw), bf_hi(sw)};
+          bool hit[2];
+          uint32_t cd[2];
+          bf16_roundtrip2(lr[e], lr[e + 1]);
+          legacy_code_mfma2<BITS>(xv + e, lr + e, sc, a.tau, ov + e, hit, cd);
+          code[e] = BITS == 1 ? (cd[0] ^ 1u) << 31 : cd[0];
+          code[e + 1] = BITS == 1 ? (cd[1] ^ 1u) << 31 : cd[1];
+          hm |= (hit[0] ? 1u << e : 0u) | (hit[1] ? 2u << e : 0u);
+          ow[e / 2] = pack_bf16x2(ov[e], ov[e + 1]);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        legacy_accumulate<BITS>(byte[e], code[e], p);
+        asm("" : "+v"(byte[e]));  // accumulated here, not kept as a code per plane until the end
+      }
+      const u32x4 ow0 = u32x4{ow[0], ow[1], ow[2], ow[3]}, ow1 = u32x4{ow[4], ow[5], ow[6], ow[7]};
+      if constexpr (STAGED) {
+        // the lane's entries: hits pre .. pre + n - 1 of its row's piece (lane g: columns 16g .. 16g + 15)
+        static_assert(kCooSlots == 2, "two entries per record");
+        const uint32_t n = __builtin_popcount(hm);
+        uint32_t pre, total;
+        row_prefix4(n, g, pre, total);
+        uint32_t* rec = reinterpret_cast<uint32_t*>(&recs[p * 16 + j]);
+        const uint32_t col = (uint32_t)(16 * g);
+        if (__builtin_amdgcn_ballot_w64(n > 1u) != 0) {  // (wave-uniform)
+          const uint32_t i0 = __builtin_ctz(hm | 0x10000u) & 15u, h1 = hm & (hm - 1u);
+          const uint32_t i1 = __builtin_ctz(h1 | 0x10000u) & 15u;
+          if (n > 0u && pre < 2u) rec[pre] = (col + i0) | (bf16_at(ow0, ow1, i0) << 16) | (pre == 0u ? total << 8 : 0u);
+          if (n > 1u && pre == 0u) rec[1] = (col + i1) | (bf16_at(ow0, ow1, i1) << 16);
+        } else {
+          // at most one hit in the lane: its value is the or of the masked ones
+          const uint32_t o = (ow[0] | ow[1] | ow[2]) | (ow[3] | ow[4] | ow[5]) | (ow[6] | ow[7]);
+          const uint32_t v = (o & 0xffff0000u) | (o << 16);
+          if (n > 0u && pre < 2u) rec[pre] = (col + __builtin_ctz(hm)) | v | (pre == 0u ? total << 8 : 0u);
+        }
+        uint16_t* orow = a.oout + ((int64_t)b * M + row0) * N;
+        const uint32_t olen = (uint32_t)(16 * N * 2), ooff = (uint32_t)(((rr - row0) * N + c0) * 2);
+        const bool dense = total > (uint32_t)kCooSlots && row < M;
+        st16_pred(orow, olen, ooff, ow0, dense);
+        st16_pred(orow, olen, ooff + 16, ow1, dense);
+      } else {
+        uint16_t* op = a.oout + ((int64_t)b * M + rr) * N + c0;
+        st16(op, ow0);
+        st16(op + 8, ow1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    uint32_t word[E / 4];
+#pragma unroll
+    for (int k = 0; k < E / 4; ++k) {
+      word[k] = gather_bytes(byte[4 * k], byte[4 * k + 1], byte[4 * k + 2], byte[4 * k + 3]);
+      if constexpr (BITS == 1) word[k] = ~word[k];
+    }
+    st16(a.qout + ((int64_t)b * M + rr) * NB + u * G + E * g, u32x4{word[0], word[1], word[2], word[3]});
+    if constexpr (STAGED) {
+      // record 64 k + lane: plane (64 k + lane) / 16, row lane % 16 (range-checked stores: no branch)
+      int64_t* prow = a.pcnt + ((int64_t)b * M + row0) * a.npc;  // the block's first row
+#pragma unroll
+      for (int k = 0; k < (NREC + 63) / 64; ++k) {
+        const int q = min(64 * k + lane, NREC - 1);
+        st8_pred(prow, (uint32_t)(16 * a.npc * 8), (uint32_t)((j * a.npc + (q >> 4) * (NB / 64) + u) * 8), recs[q],
+                 64 * k + lane < NREC && row < M);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // the requests past the run have landed before the LDS can go to another workgroup
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 }
 
 // ------------------------------------------------------------------ scalar path
@@ -1251,8 +1465,19 @@ static int legacy_launch(const LegacyArgs& a, int K, int64_t B, bool mfma_ok, hi
     LegacyArgs la = a;
     la.rb = rb;
     const dim3 grid((unsigned)nwg);
-    if (K == 16) LRQ_TRY(launch((k_legacy_mfma<MODE, BITS, 16, OSRC>), grid, dim3(256), 0, st, la));
-    else LRQ_TRY(launch((k_legacy_mfma<MODE, BITS, 32, OSRC>), grid, dim3(256), 0, st, la));
+    if constexpr (MODE == kEncode) {
+      // runs of up to 16 row blocks, shorter where that would leave under four workgroups per CU
+      const int64_t ug = (NB / 64 + 3) / 4, nrb = (a.M + 15) / 16;
+      const int64_t rbw = std::max<int64_t>(1, std::min<int64_t>(16, B * ug * nrb / (4 * (int64_t)cu_count())));
+      const int64_t wgs = (nrb + rbw - 1) / rbw * ug * B;
+      if (wgs > INT32_MAX) return LRQ_ERR_SHAPE;
+      const dim3 eg((unsigned)wgs);
+      if (K == 16) return launch((k_legacy_encode<BITS, 16, OSRC == 1>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
+      return launch((k_legacy_encode<BITS, 32, OSRC == 1>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
+    } else {
+      if (K == 16) return launch((k_legacy_mfma<MODE, BITS, 16, OSRC>), grid, dim3(256), 0, st, la);
+      return launch((k_legacy_mfma<MODE, BITS, 32, OSRC>), grid, dim3(256), 0, st, la);
+    }
   } else {
     const int64_t chunks = (NB + 255) / 256;
     if (B * a.M * chunks > INT32_MAX) return LRQ_ERR_SHAPE;
