@@ -630,3 +630,77 @@ def test_legacy_encode_non_finite_and_huge(pkg, dev, bits):
                 ref_o[b, m, n] = og[b, m, n]
         assert np.array_equal(qg, ref_q)
         assert np.array_equal(O.bf16_to_f32(og), O.bf16_to_f32(ref_o))
+
+
+# the MFMA decode (k_legacy_apply) where it can go wrong: units that do not fill a group of four, one
+# row, ragged last blocks, several runs; densities below and above the entries requested ahead; every
+# bit width and rank
+APPLY = [(1, 1, 512, 16, 1, 0.01), (2, 37, 1024, 32, 1, 0.2), (1, 50, 256, 16, 2, 0.05), (3, 33, 1536, 16, 2, 0.3),
+         (1, 2100, 512, 32, 2, 0.01), (2, 100, 640, 16, 4, 0.1), (1, 47, 384, 32, 4, 0.02), (1, 300, 320, 16, 8, 0.4),
+         (2, 64, 192, 32, 8, 0.01)]
+
+
+def _decode_operands(dev, B, M, N, K, bits, density, seed):
+    g = torch.Generator().manual_seed(seed)
+    l = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    r = torch.randn(K, N, generator=g).to(torch.bfloat16).to(dev)
+    s = (torch.randn(B, N, generator=g) + 2).to(torch.bfloat16).to(dev)
+    q = torch.randint(0, 256, (B, M, N * bits // 8), generator=g, dtype=torch.uint8).to(dev)
+    o = torch.randn(B, M, N, generator=g) * (torch.rand(B, M, N, generator=g) < density)
+    o[0, M // 2, : min(N, 200)] = 3.0  # a row of full pieces
+    return l, r, s, q, o.to(torch.bfloat16).to(dev)
+
+
+@pytest.mark.parametrize("B,M,N,K,bits,density", APPLY)
+def test_legacy_apply_is_the_dense_decode(pkg, dev, B, M, N, K, bits, density):
+    """COO outliers (with buffers below and above 1/16 of the elements) and none give the bits of the
+    decode from dense outliers; the fused consumers give those of the decode and the dense consumer."""
+    dec = pkg.low_rank_addition_fuse_decompression_dequantization
+    l, r, s, q, o = _decode_operands(dev, B, M, N, K, bits, density, N + M)
+    want = dec(l, r, q, o, s, quantize_bit=bits)
+    n = int((o != 0).sum())
+    for cap in {n, max(n, o.numel() // 20), max(n, o.numel() // 8)}:
+        assert torch.equal(dec(l, r, q, pkg.compact_outliers(o, capacity=cap), s, quantize_bit=bits), want), cap
+    plain = dec(l, r, q, torch.zeros_like(o), s, quantize_bit=bits)
+    assert torch.equal(dec(l, r, q, None, s, quantize_bit=bits), plain)
+    y = (torch.randn(B, M, N, generator=torch.Generator().manual_seed(M)) * 0.1).to(torch.bfloat16).to(dev)
+    assert torch.equal(pkg.triton_silu_backward_fuse_extraction(l, r, q, s, y, bits), pkg.triton_silu_backward(plain, y))
+    assert torch.equal(pkg.triton_hadamard_fuse_extraction(l, r, q, s, y, bits), pkg.triton_hadamard(plain, y))
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+def test_legacy_apply_non_finite_and_huge(pkg, dev, bits):
+    """Infinite and huge outliers, factors and scales change no element but their own (the decode's
+    matrix steps sum over four elements): the bits of the decode from dense outliers, and a NaN stays
+    where it is."""
+    dec = pkg.low_rank_addition_fuse_decompression_dequantization
+    l, r, s, q, o = _decode_operands(dev, 1, 70, 1024, 16, bits, 0.02, bits)
+    o[0, 3, 5], o[0, 3, 9], o[0, 20, 700], o[0, 69, 1023] = float("inf"), 3e38, -float("inf"), -3e38
+    l[33] = 1e30
+    r[2, 40], r[3, 41] = 1e30, -3e38
+    s[0, 130], s[0, 900] = 2.0 ** 120, -(2.0 ** 110)
+    want = dec(l, r, q, o, s, quantize_bit=bits)
+    got = dec(l, r, q, pkg.compact_outliers(o), s, quantize_bit=bits)
+    same = (got == want) | (torch.isnan(got) & torch.isnan(want))
+    assert same.all()
+    o[0, 50, 77] = float("nan")
+    got = dec(l, r, q, pkg.compact_outliers(o), s, quantize_bit=bits)
+    same = (got == want) | (torch.isnan(got) & torch.isnan(want))
+    same[0, 50, 77] = torch.isnan(got[0, 50, 77])
+    assert same.all()
+
+
+@pytest.mark.parametrize("bits,K", [(2, 16), (4, 32), (8, 16)])
+def test_legacy_rows_largest_dense_coo(pkg, dev, bits, K):
+    """Dense COO outliers at 2^27 elements (the row-tile decode) give the dense decode's bits."""
+    B, M, N = 4, 8200, 4096
+    dec = pkg.low_rank_addition_fuse_decompression_dequantization
+    g = torch.Generator(device=dev).manual_seed(bits)
+    l = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    r = torch.randn(K, N, generator=g, device=dev).to(torch.bfloat16)
+    s = (torch.randn(B, N, generator=g, device=dev) + 2).to(torch.bfloat16)
+    q = torch.randint(0, 256, (B, M, N * bits // 8), generator=g, device=dev, dtype=torch.uint8)
+    o = torch.randn(B, M, N, generator=g, device=dev).to(torch.bfloat16)
+    o = o * (o > 1)
+    oc = pkg.compact_outliers(o, capacity=o.numel() // 5)
+    assert torch.equal(dec(l, r, q, oc.check(), s, quantize_bit=bits), dec(l, r, q, o, s, quantize_bit=bits))

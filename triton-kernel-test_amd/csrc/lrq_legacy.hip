@@ -316,105 +316,17 @@ __device__ __forceinline__ float legacy_consume(float xh, float yv) {
   else return xh;
 }
 
-// The outlier values of columns c0 .. c0 + E - 1 of row `bm` (b * M + m) from the COO pieces
-// (sparse outliers, OSRC 2): the entries of the piece holding c0 (the E columns never straddle a
-// piece boundary), one at a time.
-template <int E>
-__device__ __forceinline__ void coo_piece_values(const LegacyArgs& a, int64_t bm, int64_t c0, float* oo) {
-#pragma unroll
-  for (int e = 0; e < E; ++e) oo[e] = 0.f;
-  const int64_t pc = bm * a.npc + c0 / 64;
-  const int64_t e1 = min(a.optr[pc + 1], a.ncap);
-  for (int64_t k = max(a.optr[pc], (int64_t)0); k < e1; ++k) {
-    const int64_t d = a.ocol[k] - c0;
-    const float v = __uint_as_float((uint32_t)a.oval[k] << 16);
-#pragma unroll
-    for (int e = 0; e < E; ++e) oo[e] = d == e ? v : oo[e];
-  }
-}
-
-// Denser outliers (OSRC 3): the COO pieces of a wave's 16 rows x one unit (NP pieces of 64
-// columns per row) go into the wave's
-// LDS tile ot[row][plane][64] (bf16 bits).  The four lanes of a row share its pieces: the piece
-// bounds come from coo_bounds (requested a block ahead), then in each pass lane (j, g) requests entries
-// g, g + 4, .. (KL per piece) of each of its row's pieces, all of them before any is used
-// (clamped indices; no load sits under a branch), and writes those that fall in the piece into
-// the tile after the lane has zeroed its own 16 columns of every plane.  Another pass runs only
-// while some piece of the wave has more entries.  Entries of a coalesced COO are unique per
-// position (so no two lanes write the same one), and entries outside the piece are ignored.
-// The piece bounds of row bm's NP pieces of unit u (requested together; coo_tile uses them).
-template <int NP>
-__device__ __forceinline__ void coo_bounds(const LegacyArgs& a, int64_t bm, int u, int N, int64_t (&s0)[NP],
-                                           int64_t (&s1)[NP]) {
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int64_t pc = bm * a.npc + (int64_t)(p * (N / NP) + u * 64) / 64;
-    s0[p] = a.optr[pc];
-    s1[p] = a.optr[pc + 1];
-  }
-}
-
-// Entries each lane requests per piece and pass (4 lanes per row: 4 * KL entries of a piece per pass).
-static constexpr int kCooEntriesPerLane = 2;
-// bf16 of padding after each row of the COO tile: rows 16 bytes apart in the LDS banks, so the
-// 16-byte accesses of 8 consecutive lanes (8 rows) fall in distinct banks.
-static constexpr int kCooRowPad = 8;
-template <int NP>
-constexpr int coo_row_stride() { return NP * 64 + kCooRowPad; }
-template <int NP, int KL>
-__device__ __forceinline__ void coo_tile(const LegacyArgs& a, int64_t (&s0)[NP], int64_t (&s1)[NP], int u, int N,
-                                         int j, int g, uint16_t* __restrict__ ot) {
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    uint16_t* r = ot + j * coo_row_stride<NP>() + p * 64 + 16 * g;
-    st16(r, u32x4{0u, 0u, 0u, 0u});
-    st16(r + 8, u32x4{0u, 0u, 0u, 0u});
-    s0[p] = max(s0[p], (int64_t)0);
-    s1[p] = min(s1[p], a.ncap);
-  }
-  if (a.ncap <= 0) return;  // uniform: no entries at all
-  const uint32_t* col32 = reinterpret_cast<const uint32_t*>(a.ocol);  // low dword of each int64 column
-  for (int pass = 0;; ++pass) {
-    uint32_t cv[NP][KL];
-    uint16_t vv[NP][KL];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-      for (int i = 0; i < KL; ++i) {
-        const int64_t k = min(s0[p] + (int64_t)(4 * KL * pass + g + 4 * i), a.ncap - 1);
-        cv[p][i] = col32[2 * k];
-        vv[p][i] = a.oval[k];
-      }
-    bool more = false;
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int64_t base = p * (N / NP) + u * 64;
-#pragma unroll
-      for (int i = 0; i < KL; ++i) {
-        const int64_t k = s0[p] + (int64_t)(4 * KL * pass + g + 4 * i);
-        const int64_t d = (int64_t)cv[p][i] - base;
-        if (k < s1[p] && d >= 0 && d < 64) ot[j * coo_row_stride<NP>() + p * 64 + (int)d] = vv[p][i];
-      }
-      more |= s1[p] - s0[p] > (int64_t)4 * KL * (pass + 1);
-    }
-    if (!__builtin_amdgcn_ballot_w64(more)) break;  // uniform
-  }
-}
-
 // ------------------------------------------------------------------ MFMA path
 // Grid: ceil(M / (64 * rb)) * (N / (64 * NP)) * B workgroups (one dimension); 4 waves; the
 // workgroup's tile t = (b, bx, u), units fastest, is xcd_tile of its index: the workgroups of one
 // XCD that run together cover neighbouring units of the same rows, which share L2 lines of the COO
 // entries (a piece's entries do not start on a line boundary), of the code rows and of the output
-// rows.  Wave w walks row blocks (bx * rb + i) * 64 + w * 16, i < rb, of unit u.  OSRC, decode: outliers
-// absent (0), dense (1) or COO pieces (2: looked up per lane, for sparse outliers; 3: gathered
-// per wave into an LDS tile, for denser ones).
-template <int MODE, int BITS, int K, int OSRC>
+// rows.  Wave w walks row blocks (bx * rb + i) * 64 + w * 16, i < rb, of unit u.  Decodes from dense
+// outliers, adds and histograms (the other decodes: k_legacy_apply, k_legacy_rows).
+template <int MODE, int BITS, int K>
 __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
   constexpr int NP = (MODE == kAdd || MODE == kHist) ? 1 : 8 / BITS, G = 64, E = 16, RT = K / 16;
   __shared__ uint32_t lh[MODE == kHist ? 256 : 1];
-  // decode from denser COO outliers: each wave's outlier tile (16 rows x NP planes x 64 columns, bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t otile[(MODE == kDecode && OSRC == 3) ? 4 * 16 * coo_row_stride<NP>() : 8];
   int64_t sel = -1;
   if constexpr (MODE == kHist) {
     lh[threadIdx.x] = 0u;
@@ -440,30 +352,13 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
   const float zero[E] = {};
 
   // the unit's scales in LDS for every row block of the workgroup (the same columns throughout)
-  constexpr bool kScales = MODE != kAdd && MODE != kHist;
+  constexpr bool kScales = MODE == kDecode;
   __shared__ __attribute__((aligned(16))) float stab[kScales ? NP * G : 4];
   if constexpr (kScales) {
     for (int i = threadIdx.x; i < NP * G; i += 256) stab[i] = bf_lo(srow[unit_base(i / G, u, N, NP, G) + i % G]);
     __syncthreads();
   }
 
-  // decode from the COO tile: the next row block's L operand, codes and COO piece bounds are
-  // requested before the current block is computed (nl / nq / ns0 / ns1 carry them over; the
-  // other modes measured slower with the carried registers)
-  constexpr bool kCodes = MODE == kDecode || MODE == kFusedStore || MODE == kFusedSilu || MODE == kFusedMul;
-  constexpr bool kPre = MODE == kDecode && OSRC == 3;
-  constexpr int NPB = (MODE == kDecode && OSRC == 3) ? NP : 1;  // COO piece bounds per lane
-  u32x2 nl[RT];
-  u32x4 nq = u32x4{0u, 0u, 0u, 0u};
-  int64_t ns0[NPB], ns1[NPB];
-  auto fetch_next = [&](int i) __attribute__((always_inline)) {  // block i of the workgroup (rows clamped to the last)
-    const int64_t rn = min((bx * a.rb + i) * 64 + w * 16 + j, M - 1);
-#pragma unroll
-    for (int t = 0; t < RT; ++t) nl[t] = ld8(a.l + rn * K + 16 * t + 4 * g);
-    nq = ld16(a.qin + ((int64_t)b * M + rn) * NB + u * G + E * g);
-    if constexpr (MODE == kDecode && OSRC == 3) coo_bounds<NP>(a, (int64_t)b * M + rn, u, N, ns0, ns1);
-  };
-  if constexpr (kPre) fetch_next(0);
   for (int i = 0; i < a.rb; ++i) {
     const int row0 = (bx * a.rb + i) * 64 + w * 16;  // wave-uniform: a scalar exit
     if (row0 >= M) break;  // whole 16-row block past the end
@@ -472,24 +367,9 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
     const int64_t erow = ((int64_t)b * M + rr) * N;  // element offset of the row in [B, M, N] outputs
     u32x2 lop[RT];
     u32x4 qb = u32x4{0u, 0u, 0u, 0u};
-    int64_t s0[NPB], s1[NPB];
-    if constexpr (kPre) {
 #pragma unroll
-      for (int t = 0; t < RT; ++t) lop[t] = nl[t];
-      qb = nq;
-#pragma unroll
-      for (int q = 0; q < NPB; ++q) {
-        s0[q] = ns0[q];
-        s1[q] = ns1[q];
-      }
-      fetch_next(min(i + 1, a.rb - 1));  // (the last block fetches itself again: unused)
-    } else {
-#pragma unroll
-      for (int t = 0; t < RT; ++t) lop[t] = ld8(a.l + rr * K + 16 * t + 4 * g);
-      if constexpr (kCodes) qb = ld16(a.qin + ((int64_t)b * M + rr) * NB + u * G + E * g);
-    }
-    uint16_t* ot = otile + (size_t)w * 16 * coo_row_stride<NP>();
-    if constexpr (MODE == kDecode && OSRC == 3) coo_tile<NP, kCooEntriesPerLane>(a, s0, s1, u, N, j, g, ot);
+    for (int t = 0; t < RT; ++t) lop[t] = ld8(a.l + rr * K + 16 * t + 4 * g);
+    if constexpr (MODE == kDecode) qb = ld16(a.qin + ((int64_t)b * M + rr) * NB + u * G + E * g);
 
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
@@ -531,26 +411,13 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
         st16(a.out + erow + c0, pack8(ov));
         st16(a.out + erow + c0 + 8, pack8(ov + 8));
       } else {
-        float ov[E], oo[E], yv[E];
-        if constexpr (MODE == kDecode && OSRC == 1) {
-          unpack8(ld16(a.oin + erow + c0), oo);
-          unpack8(ld16(a.oin + erow + c0 + 8), oo + 8);
-        }
-        if constexpr (MODE == kDecode && OSRC == 2) coo_piece_values<E>(a, (int64_t)b * M + rr, c0, oo);
-        if constexpr (MODE == kDecode && OSRC == 3) {
-          const uint16_t* r = ot + j * coo_row_stride<NP>() + p * 64 + 16 * g;
-          unpack8(*reinterpret_cast<const u32x4*>(r), oo);
-          unpack8(*reinterpret_cast<const u32x4*>(r + 8), oo + 8);
-        }
-        if constexpr (MODE == kFusedSilu || MODE == kFusedMul) {
-          unpack8(ld16(a.y + erow + c0), yv);
-          unpack8(ld16(a.y + erow + c0 + 8), yv + 8);
-        }
+        float ov[E], oo[E];
+        unpack8(ld16(a.oin + erow + c0), oo);
+        unpack8(ld16(a.oin + erow + c0 + 8), oo + 8);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
           const uint32_t code = (qb[e >> 2] >> (8 * (e & 3) + BITS * p)) & kMask;
-          const float xh = legacy_value<BITS, MODE == kDecode && OSRC != 0>(code, sc[e], oo[e], lr[e]);
-          ov[e] = legacy_consume<MODE>(xh, yv[e]);
+          ov[e] = legacy_value<BITS, true>(code, sc[e], oo[e], lr[e]);
         }
         st16(a.out + erow + c0, pack8(ov));
         st16(a.out + erow + c0 + 8, pack8(ov + 8));
@@ -791,6 +658,361 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 }
 
+// ------------------------------------------------------------------ MFMA decode and fused consumers
+// x_hat without outliers or with sparse COO outliers (COO), stored (kDecode / kFusedStore) or consumed
+// with y (kFusedSilu, kFusedMul).  Independent waves as in k_legacy_encode (wave w of a tile: unit
+// 4 * group + w, RBW 16-row blocks); a step is one plane of one block.
+// - y streams through the same LDS ring of whole 128-byte lines; the result goes through a private LDS
+//   tile and leaves as two 1 KB stores of whole lines (a skeleton of the MFMA-layout accesses that
+//   these replace reaches 3.9 TB/s, of these 5.1).
+// - Element work on the matrix pipe (diagonal 4x4x4 steps, see legacy_codes_mfma): the codes enter as
+//   the bf16 values 128 + c (a byte permute, no conversion), a = s (128 + c) - s (128 + h) is exact in
+//   fp32 (h = 2^(b-1); at 8 bits c = 16 hi + lo takes two steps); then a's bf16 rounding (4 and 8 bits),
+//   + o and + bf16(l r) are identity steps with one rounding each, as in legacy_value.  About 3.5 vector
+//   instructions per element for x_hat, 11 - 16 before.
+//   2-bit decode of [4, 8192, 8192] with 0.6 % outliers 209 -> 114 us, 1-bit 319 -> 115 us; SiLU gradient
+//   at [4, 4096, 4096] 97 -> 57.6 us a call.
+// - COO: the block's pieces (one per (row, plane)) take LPP lanes each; a lane's piece bounds are
+//   requested two blocks ahead and its SLOTS entries one block ahead, as range-checked loads (an absent
+//   entry reads nothing); they go into the wave's zeroed tile [NP][16][64] at the block's start and are
+//   cleared from it at its end.  Pieces with more entries take further rounds on the spot.
+// A diagonal step sums over four elements, so nothing in it may overflow or be infinite: scales below
+// 2^100, |o| below 2^126 and max |l| max |r| K below 2^120 (legacy_value's sums are then all finite);
+// a block beyond that takes legacy_value element by element.
+template <int MODE, int BITS, int COO>
+struct LegacyApply {
+  static constexpr int NP = 8 / BITS, NW = 4, RING = 4, SLOT = 16 * 128, NREC = 16 * NP;
+  static constexpr bool HASY = MODE == kFusedSilu || MODE == kFusedMul;
+  static constexpr int TAB = NP * 64 * 4;
+  static constexpr int OFF_TAB = HASY ? RING * SLOT : 0, OFF_OUT = OFF_TAB + TAB, OFF_O = OFF_OUT + SLOT;
+  static constexpr int WAVE = OFF_O + (COO ? NP * SLOT : 0);  // bytes per wave
+  static constexpr int kStepOps = 4;                          // with y: two loads, two stores per step
+  static constexpr int LPP = NREC <= 64 ? 64 / NREC : 1, PPL = NREC <= 64 ? 1 : NREC / 64;
+  // entries of a piece per lane and round (2 bits, 16 % outliers: [4, 3072, 3072] 49.7 us at 8, 58.5 at
+  // 12, 61.3 at 20)
+  static constexpr int SLOTS = COO == 2 ? (PPL > 1 ? 4 : LPP == 1 ? 8 : 20 / LPP) : PPL == 1 && LPP < 4 ? 4 : 2;
+};
+template <int MODE, int BITS, int K, int COO>
+__global__ __launch_bounds__(256) void k_legacy_apply(LegacyArgs a, int RBW, int ug) {
+  using La = LegacyApply<MODE, BITS, COO>;
+  constexpr int NP = La::NP, G = 64, E = 16, RT = K / 16, RING = La::RING, SLOT = La::SLOT;
+  constexpr bool HASY = La::HASY;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[La::NW][La::WAVE];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int j = lane & 15, g = lane >> 4;
+  const int M = (int)a.M, N = (int)a.N, nrb = (M + 15) / 16, nrun = (nrb + RBW - 1) / RBW;
+  const int t = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x));
+  const int u = __builtin_amdgcn_readfirstlane(t % ug) * La::NW + w;
+  const int run = __builtin_amdgcn_readfirstlane((t / ug) % nrun), b = __builtin_amdgcn_readfirstlane(t / (ug * nrun));
+  const int64_t NB = N / NP;  // bytes per code row
+  if (u * G >= NB) return;    // the group's last units (this wave only)
+  const int rb0 = run * RBW, nblk = min(RBW, nrb - rb0);
+  const int64_t bm0 = (int64_t)b * M;
+  unsigned char* const ring = lds[w];
+  uint32_t* const stab = reinterpret_cast<uint32_t*>(ring + La::OFF_TAB);  // [NP][16 (g, j % 4)][4 steps]
+  unsigned char* const otile = ring + La::OFF_O;
+  unsigned char* const xtile = ring + La::OFF_OUT;
+  const uint16_t* srow = a.s + (a.s_rows == 1 ? 0 : (int64_t)b * N);
+
+  // y: step st = (block st / NP, plane st % NP) in slot st % RING (see k_legacy_encode)
+  const uint16_t* const ybase = HASY ? a.y + bm0 * N + u * G + 8 * ((lane & 7) ^ (lane >> 3)) : nullptr;
+  auto request = [&](int i, int p, int slot) __attribute__((always_inline)) {
+    if constexpr (HASY) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int64_t row = min((rb0 + i) * 16 + 8 * k + (lane >> 3), M - 1);
+        ld16_to_lds(ybase + row * N + p * NB, ring + slot * SLOT + 1024 * k);
+      }
+    }
+  };
+#pragma unroll
+  for (int st = 0; st < RING; ++st) request(min(st / NP, nblk - 1), st % NP, st);
+  u32x2 nl[RT];
+  u32x4 nq;
+  auto fetch = [&](int i) __attribute__((always_inline)) {  // block i's codes and l operand
+    const int64_t rn = min((rb0 + i) * 16 + j, M - 1);
+#pragma unroll
+    for (int k = 0; k < RT; ++k) nl[k] = ld8(a.l + rn * K + 16 * k + 4 * g);
+    nq = ld16(a.qin + (bm0 + rn) * NB + u * G + E * g);
+  };
+  fetch(0);
+
+  // COO: lane -> piece pi = lane / LPP + 64 q' of the block (plane pi / 16, row pi % 16), place lane % LPP
+  constexpr int LPP = La::LPP, PPL = La::PPL, SL = La::SLOTS;
+  struct Bnd {
+    int64_t s0, s1;
+  };
+  struct Ent {
+    uint32_t col[SL];
+    uint32_t val[SL];
+  };
+  Bnd bnd[PPL], bnd_n[PPL];  // of the block whose entries are in flight, and of the one after
+  Ent ent[PPL];
+  int64_t ebase = 0;  // the entry buffers' first entry (wave-uniform)
+  auto bounds = [&](int i, Bnd (&d)[PPL]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < PPL; ++h) {
+      const int pi = lane / LPP + 64 * h;
+      const int64_t rn = min((rb0 + i) * 16 + (pi & 15), M - 1);
+      const int64_t pc = (bm0 + rn) * a.npc + (pi >> 4) * (NB / G) + u;
+      d[h].s0 = max(a.optr[pc], (int64_t)0);
+      d[h].s1 = min(a.optr[pc + 1], a.ncap);
+    }
+  };
+  // entries s0 + LPP * (SL * round + k) + lane % LPP, k < SL, of the lane's pieces; an entry past the
+  // piece (or 2^24 entries past the block's first) is outside the range and reads as column 0, value 0
+  auto load_entries = [&](const Bnd (&d)[PPL], int round, Ent (&en)[PPL]) __attribute__((always_inline)) {
+    const int64_t left = max(min(a.ncap - ebase, (int64_t)1 << 24), (int64_t)0);
+    const __amdgpu_buffer_rsrc_t rc = uniform_rsrc(const_cast<int64_t*>(a.ocol + ebase), (uint32_t)(left * 8));
+    const __amdgpu_buffer_rsrc_t rv = uniform_rsrc(const_cast<uint16_t*>(a.oval + ebase), (uint32_t)(left * 2));
+#pragma unroll
+    for (int h = 0; h < PPL; ++h)
+#pragma unroll
+      for (int k = 0; k < SL; ++k) {
+        const int64_t e = d[h].s0 + LPP * (SL * round + k) + lane % LPP;
+        const int64_t rel = e - ebase;
+        const bool in = e < d[h].s1 && rel >= 0 && rel < left;
+        en[h].col[k] = __builtin_amdgcn_raw_buffer_load_b32(rc, in ? (uint32_t)rel * 8u : 0x7ffffff0u, 0, 0);
+        en[h].val[k] = __builtin_amdgcn_raw_buffer_load_b16(rv, in ? (uint32_t)rel * 2u : 0x7ffffff0u, 0, 0);
+      }
+  };
+  // writes the entries of a round into the tile (or clears them from it); returns whether an entry's
+  // magnitude is 2^126 or more (or not finite)
+  auto put = [&](const Bnd (&d)[PPL], int round, const Ent (&en)[PPL], bool clear) __attribute__((always_inline)) -> bool {
+    bool big = false;
+#pragma unroll
+    for (int h = 0; h < PPL; ++h) {
+      const int pi = lane / LPP + 64 * h;
+      const int cbase = (pi >> 4) * (int)NB + u * G;
+#pragma unroll
+      for (int k = 0; k < SL; ++k) {
+        const int64_t e = d[h].s0 + LPP * (SL * round + k) + lane % LPP;
+        const int64_t rel = e - ebase;
+        const uint32_t c = en[h].col[k] - (uint32_t)cbase;
+        if (e < d[h].s1 && rel >= 0 && rel < (1 << 24) && c < 64u) {
+          // (chunk c / 8 of row r at position (c / 8) ^ (r % 8))
+          uint16_t* o = reinterpret_cast<uint16_t*>(otile + pi * 128 + 16 * ((c >> 3) ^ (pi & 7)));
+          o[c & 7u] = clear ? (uint16_t)0 : (uint16_t)en[h].val[k];
+          big |= (en[h].val[k] & 0x7fffu) >= 0x7e80u;
+        }
+      }
+    }
+    return big;
+  };
+  auto zero_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2 * NP; ++k) *reinterpret_cast<u32x4*>(otile + 1024 * k + 16 * lane) = u32x4{0u, 0u, 0u, 0u};
+  };
+  auto first_entry = [&](const Bnd (&d)[PPL]) __attribute__((always_inline)) -> int64_t {
+    const uint64_t v = (uint64_t)d[0].s0;  // lane 0: plane 0 of the block's first row, the smallest
+    return (int64_t)(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
+                     (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)v));
+  };
+  if constexpr (COO != 0) {
+    bounds(0, bnd);
+    bounds(min(1, nblk - 1), bnd_n);
+    zero_tile();
+    ebase = first_entry(bnd);
+    load_entries(bnd, 0, ent);
+  }
+
+  u32x2 vop[NP][4][RT];
+  uint32_t rtop = 0;  // the largest magnitude of the lane's r^T operands (bf16 bits, both halves)
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    load_vops<G, K>(a.rt, unit_base(p, u, N, NP, G), j, g, vop[p]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int k = 0; k < RT; ++k)
+        rtop = pk_max_u16(pk_max_u16(rtop, vop[p][q][k][0] & 0x7fff7fffu), vop[p][q][k][1] & 0x7fff7fffu);
+  }
+  bool s_ok = true;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const float sv = bf_lo(srow[unit_base(p, u, N, NP, G) + lane]);
+    s_ok &= fabsf(sv) < 0x1p100f;  // (NaN fails)
+    // bf16(s) | bf16(16 s) << 16: the second term serves the high nibble at 8 bits
+    stab[p * 64 + ((lane >> 4) * 4 + (lane & 3)) * 4 + ((lane >> 2) & 3)] = pack_bf16x2(sv, 16.f * sv);
+  }
+  uint32_t rmax = max(rtop >> 16, rtop & 0xffffu);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) rmax = max(rmax, (uint32_t)__shfl_xor((int)rmax, d));
+  // K max |r| of the unit, infinite or NaN when an operand is
+  const float rbound = (float)K * __uint_as_float(__builtin_amdgcn_readfirstlane(rmax) << 16);
+  const bool unit_ok = __builtin_amdgcn_ballot_w64(!s_ok) == 0;  // wave-uniform
+  const u32x2 ida = diag4_aop(lane, 0x3f80u);
+  constexpr uint32_t kMask = (BITS == 8 ? 0x0fu : (1u << BITS) - 1u) * 0x01010101u;
+  constexpr int kHalf = 1 << (BITS - 1);
+  // -(128 + h) as bf16 pairs (at 8 bits -(16 * 128 + 128 + 128)): exact
+  const uint32_t koff = pack_bf16x2_exact(-(float)(BITS == 8 ? 2304 : 128 + kHalf), -(float)(BITS == 8 ? 2304 : 128 + kHalf));
+  if constexpr (HASY) {
+    // the prologue's loads have landed (the counted waits below start from none outstanding)
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+#pragma unroll 1
+  for (int i = 0; i < nblk; ++i) {
+    const int row0 = (rb0 + i) * 16;
+    u32x2 lop[RT];
+#pragma unroll
+    for (int k = 0; k < RT; ++k) lop[k] = nl[k];
+    const u32x4 qb = nq;
+    bool big = false, rest = false;
+    Bnd cur[PPL];
+    Ent cure[PPL];
+    int64_t cbase_e = ebase;
+    if constexpr (COO != 0) {
+      big = put(bnd, 0, ent, false);
+#pragma unroll
+      for (int h = 0; h < PPL; ++h) {
+        rest |= bnd[h].s1 - bnd[h].s0 > (int64_t)LPP * SL;
+        cur[h] = bnd[h];
+        if constexpr (COO == 1) cure[h] = ent[h];
+        bnd[h] = bnd_n[h];
+      }
+      rest = __builtin_amdgcn_ballot_w64(rest) != 0;  // (wave-uniform)
+      if (rest) {
+        for (int round = 1;; ++round) {
+          bool more = false;
+          Ent en[PPL];
+          load_entries(cur, round, en);
+          big |= put(cur, round, en, false);
+#pragma unroll
+          for (int h = 0; h < PPL; ++h) more |= cur[h].s1 - cur[h].s0 > (int64_t)LPP * SL * (round + 1);
+          if (__builtin_amdgcn_ballot_w64(more) == 0) break;
+        }
+      }
+      ebase = first_entry(bnd);
+      load_entries(bnd, 0, ent);
+      bounds(min(i + 2, nblk - 1), bnd_n);
+    }
+    fetch(min(i + 1, nblk - 1));
+    // max |l| K max |r| < 2^120: every l r is finite and small enough
+    uint32_t lt = 0;
+#pragma unroll
+    for (int k = 0; k < RT; ++k) lt = pk_max_u16(lt, pk_max_u16(lop[k][0] & 0x7fff7fffu, lop[k][1] & 0x7fff7fffu));
+    const float lmax = __uint_as_float(max(lt & 0xffff0000u, lt << 16));
+    const bool fast = unit_ok && __builtin_amdgcn_ballot_w64(!(lmax * rbound < 0x1p120f) || big) == 0;  // wave-uniform
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, NP>([&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+      const int slot = (i * NP + p) % RING;
+      u32x4 yw[2];
+      if constexpr (HASY) {
+        // (the slot's loads: RING steps ago, kStepOps memory operations in each step since)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 1) * La::kStepOps));
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned char* ys = ring + slot * SLOT + 128 * j;
+        yw[0] = *reinterpret_cast<const u32x4*>(ys + 16 * ((2 * g) ^ (j & 7)));
+        yw[1] = *reinterpret_cast<const u32x4*>(ys + 16 * ((2 * g + 1) ^ (j & 7)));
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slot is read
+        __builtin_amdgcn_sched_barrier(0);
+        request(min(i + (p + RING) / NP, nblk - 1), (p + RING) % NP, slot);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      u32x4 ov[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
+      if constexpr (COO != 0) {
+        const unsigned char* os = otile + (p * 16 + j) * 128;
+        ov[0] = *reinterpret_cast<const u32x4*>(os + 16 * ((2 * g) ^ (j & 7)));
+        ov[1] = *reinterpret_cast<const u32x4*>(os + 16 * ((2 * g + 1) ^ (j & 7)));
+      }
+      uint32_t xo[8];  // x_hat, packed
+      f32x4 tl[4], tv[4];
+      legacy_lowrank_mfma<K>(vop[p], lop, tl);
+      if (fast) {
+        const u32x4 st = *reinterpret_cast<const u32x4*>(stab + p * 64 + (g * 4 + (j & 3)) * 4);
+        const u32x2 sel = diag4_sel(lane, 0), selh = diag4_sel(lane, 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x2 sa = u32x2{__builtin_amdgcn_perm(st[q], st[q], sel[0]), __builtin_amdgcn_perm(st[q], st[q], sel[1])};
+          // elements 4q .. 4q + 3: 128 + code as bf16 (bytes code, 0x43)
+          const uint32_t m = BITS == 8 ? qb[q] & kMask : (qb[q] >> (BITS * p)) & kMask;
+          const u32x2 cb = u32x2{__builtin_amdgcn_perm(0x43434343u, m, 0x04010400u), __builtin_amdgcn_perm(0x43434343u, m, 0x04030402u)};
+          f32x4 v = mfma_4x4x4(sa, u32x2{koff, koff}, zero4());
+          v = mfma_4x4x4(sa, cb, v);
+          if constexpr (BITS == 8) {
+            const u32x2 sb = u32x2{__builtin_amdgcn_perm(st[q], st[q], selh[0]), __builtin_amdgcn_perm(st[q], st[q], selh[1])};
+            const uint32_t mh = (qb[q] >> 4) & kMask;
+            v = mfma_4x4x4(sb, u32x2{__builtin_amdgcn_perm(0x43434343u, mh, 0x04010400u), __builtin_amdgcn_perm(0x43434343u, mh, 0x04030402u)}, v);
+          }
+          tv[q] = v;
+        }
+        auto rounded = [&](f32x4 v) __attribute__((always_inline)) {
+          return u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        };
+        if constexpr (BITS > 2) {  // (already a bf16 value at 1 and 2 bits)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) tv[q] = mfma_4x4x4(ida, rounded(tv[q]), zero4());
+        }
+        if constexpr (COO != 0) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const u32x4 o = ov[q >> 1];
+            tv[q] = mfma_4x4x4(ida, u32x2{o[2 * (q & 1)], o[2 * (q & 1) + 1]}, tv[q]);
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) tv[q] = mfma_4x4x4(ida, rounded(tv[q]), zero4());
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) tv[q] = mfma_4x4x4(ida, rounded(tl[q]), tv[q]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x2 r = rounded(tv[q]);
+          xo[2 * q] = r[0];
+          xo[2 * q + 1] = r[1];
+        }
+      } else {
+        const uint16_t* sp = srow + unit_base(p, u, N, NP, G) + E * g;
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+          const uint32_t sw = ld4(sp + e), ow = ov[e >> 3][(e >> 1) & 3];
+          const uint32_t c0 = (qb[e >> 2] >> (8 * (e & 3) + BITS * p)) & ((1u << BITS) - 1u);
+          const uint32_t c1 = (qb[e >> 2] >> (8 * ((e + 1) & 3) + BITS * p)) & ((1u << BITS) - 1u);
+          xo[e / 2] = pack_bf16x2_exact(
+              legacy_value<BITS, COO != 0>(c0, bf_lo(sw), bf_lo(ow), bf16r(tl[e >> 2][e & 3])),
+              legacy_value<BITS, COO != 0>(c1, bf_hi(sw), bf_hi(ow), bf16r(tl[e >> 2][(e + 1) & 3])));
+        }
+      }
+      if constexpr (HASY) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const uint32_t y = yw[k >> 2][k & 3];
+          xo[k] = pack_bf16x2(legacy_consume<MODE>(bf_lo(xo[k]), bf_lo(y)), legacy_consume<MODE>(bf_hi(xo[k]), bf_hi(y)));
+        }
+      }
+      // through the tile (this wave's LDS operations run in order) to two stores of eight whole lines;
+      // rows past the end fall outside the store range
+      unsigned char* xs = xtile + 128 * j;
+      *reinterpret_cast<u32x4*>(xs + 16 * ((2 * g) ^ (j & 7))) = u32x4{xo[0], xo[1], xo[2], xo[3]};
+      *reinterpret_cast<u32x4*>(xs + 16 * ((2 * g + 1) ^ (j & 7))) = u32x4{xo[4], xo[5], xo[6], xo[7]};
+      uint16_t* orow = a.out + (bm0 + row0) * N;
+      const int c = u * G + p * (int)NB + 8 * ((lane & 7) ^ (lane >> 3));
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int r = 8 * k + (lane >> 3);
+        const u32x4 v = *reinterpret_cast<const u32x4*>(xtile + 1024 * k + 16 * lane);
+        st16_pred_stream(orow, (uint32_t)(16 * N * 2), (uint32_t)((r * N + c) * 2), v, row0 + r < M);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (COO != 0) {
+      if (COO == 2 || rest) {
+        zero_tile();
+      } else {
+        const int64_t keep = ebase;
+        ebase = cbase_e;
+        put(cur, 0, cure, true);
+        ebase = keep;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // the requests past the run have landed before the LDS can go to another workgroup
+  if constexpr (HASY) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+}
+
 // ------------------------------------------------------------------ scalar path
 // One thread per packed byte position c of one row; grid.x enumerates (b, m, 256-byte chunk).
 template <int MODE, int BITS, int OSRC>
@@ -847,7 +1069,7 @@ __global__ __launch_bounds__(256) void k_legacy_scalar(LegacyArgs a, int K, int6
 }
 
 // ------------------------------------------------------------------ row-tile decode
-// Decode for large shapes (2, 4 or 8 bits; no outliers, or COO outliers), staged through an LDS
+// Decode from dense COO outliers for the largest shapes (2, 4 or 8 bits), staged through an LDS
 // tile so that the output leaves as whole row segments.  A workgroup of 4 waves owns 4 units
 // (wave w: unit u0 + w, i.e. 64 columns in every plane) of one batch over a run of RBW 16-row
 // blocks, with the unit's r^T operands in registers and the units' scales in LDS for the whole
@@ -862,7 +1084,7 @@ __global__ __launch_bounds__(256) void k_legacy_scalar(LegacyArgs a, int K, int6
 //   a block earlier, into the zeroed tile and request the entries of block b + 2 and the COO
 //   bounds of block b + 4.
 // COO ranges: the entries of one (row, plane) of the workgroup's units are contiguous (row-major
-// COO, 64-column pieces in order): [piece_ptr[pc], piece_ptr[pc + units]).  With outliers the
+// COO, 64-column pieces in order): [piece_ptr[pc], piece_ptr[pc + units]).  The
 // workgroup has 4 more waves, COO workers (their loads and waits stay out of the decoding waves'
 // in-order memory queues): worker w takes ranges w * RPW .. w * RPW + RPW - 1 (range q: row q % 16,
 // plane q / 16), LPR = 64 / RPW lanes each; lane l of range r loads its own bounds and entries
@@ -883,11 +1105,11 @@ struct LegacyRows {
   static_assert(BITS == 2 || BITS == 4 || BITS == 8, "2, 4 or 8 bits");
 };
 
-template <int BITS, int K, bool COO>
-__global__ __launch_bounds__(COO ? 512 : 256) __attribute__((amdgpu_waves_per_eu(4))) void k_legacy_rows(LegacyArgs a, int RBW, int ug) {
+template <int BITS, int K>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_legacy_rows(LegacyArgs a, int RBW, int ug) {
   using Lr = LegacyRows<BITS>;
   constexpr int NP = Lr::NP, NW = Lr::NW, G = 64, E = 16, RT = K / 16, SEG = Lr::SEG, RSTR = Lr::RSTR;
-  constexpr int TILE = Lr::TILE, RPW = Lr::RPW, PD = Lr::PD, T = COO ? 512 : 256;
+  constexpr int TILE = Lr::TILE, RPW = Lr::RPW, PD = Lr::PD, T = 512;
   constexpr uint32_t kMask = BITS == 8 ? 0xffu : (1u << BITS) - 1u;
   extern __shared__ __attribute__((aligned(16))) uint16_t lt[];  // [2][TILE] + dummy[64]
   uint16_t* const dummy = lt + 2 * TILE;
@@ -902,10 +1124,10 @@ __global__ __launch_bounds__(COO ? 512 : 256) __attribute__((amdgpu_waves_per_eu
   const int t = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x, gridDim.x));
   const int ugi = t % ug, run = (t / ug) % nrun, b = t / (ug * nrun);
   const int u0 = ugi * NW, nuw = min(NW, nu - u0), u = min(u0 + w % NW, nu - 1);
-  // with COO outliers, waves NW .. 2 NW - 1 are COO workers: they zero the tiles and write the
+  // waves NW .. 2 NW - 1 are COO workers: they zero the tiles and write the
   // entries into them, so that their loads and waits never hold up the decoding waves' block ring
   // (memory operations retire in issue order, per wave)
-  const bool worker = COO && w >= NW;  // (uniform)
+  const bool worker = w >= NW;  // (uniform)
   const int rb0 = run * RBW, nblk = min(RBW, nrb - rb0);
   const int64_t bm0 = (int64_t)b * M;  // first row of the batch in [B * M] rows
   const uint16_t* srow = a.s + (a.s_rows == 1 ? 0 : (int64_t)b * N);
@@ -1007,10 +1229,8 @@ __global__ __launch_bounds__(COO ? 512 : 256) __attribute__((amdgpu_waves_per_eu
       residual_unit<G, K>(vop[p], d.lop, zero, lr);
       uint16_t* tp = tb + j * RSTR + p * SEG + w * G + E * g;
       u32x4 ov[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
-      if constexpr (COO) {
-        ov[0] = *reinterpret_cast<const u32x4*>(tp);
-        ov[1] = *reinterpret_cast<const u32x4*>(tp + 8);
-      }
+      ov[0] = *reinterpret_cast<const u32x4*>(tp);
+      ov[1] = *reinterpret_cast<const u32x4*>(tp + 8);
       u32x4 xo[2];
       const uint16_t* sp = stab + p * SEG + w * G + E * g;
       const u32x4 scp[2] = {*reinterpret_cast<const u32x4*>(sp), *reinterpret_cast<const u32x4*>(sp + 8)};
@@ -1029,12 +1249,10 @@ __global__ __launch_bounds__(COO ? 512 : 256) __attribute__((amdgpu_waves_per_eu
           av[0] = bf_lo(ap);
           av[1] = bf_hi(ap);
         }
-        if constexpr (COO) {
-          const uint32_t ow = ov[e >> 3][(e >> 1) & 3];
-          const uint32_t ap = pack_bf16x2(av[0] + bf_lo(ow), av[1] + bf_hi(ow));
-          av[0] = bf_lo(ap);
-          av[1] = bf_hi(ap);
-        }
+        const uint32_t ow = ov[e >> 3][(e >> 1) & 3];
+        const uint32_t ao = pack_bf16x2(av[0] + bf_lo(ow), av[1] + bf_hi(ow));
+        av[0] = bf_lo(ao);
+        av[1] = bf_hi(ao);
         xo[e >> 3][(e >> 1) & 3] = pack_bf16x2(av[0] + bf_lo(lp), av[1] + bf_hi(lp));
       }
       *reinterpret_cast<u32x4*>(tp) = xo[0];
@@ -1061,65 +1279,47 @@ __global__ __launch_bounds__(COO ? 512 : 256) __attribute__((amdgpu_waves_per_eu
 
   Blk ring[PD];
   const int npos = (nblk + PD - 1) / PD * PD;  // positions, whole ring rounds
-  if constexpr (COO) {
-    if (worker) {
-      // block 0's entries into tile 0, block 1's requested; per position: zero the next tile
-      // (between the barriers), then write the next block's entries into it and request those
-      // of the block after
-      const Bnd bnd0 = load_bounds(0);
-      Bnd bnd_c = load_bounds(1), bnd_n = load_bounds(2), bnd_nn = load_bounds(3);
-      zero_tile(lt);
-      zero_tile(lt + TILE);
-      int ns = slots(bnd0, 0);
-      load_entries(bnd0, 0, ns);
-      lds_barrier();  // B0: both tiles zeroed
-      scatter(lt, bnd0, 0, ns);
-      scatter_rest(lt, bnd0);
-      int ns_c = slots(bnd_c, 0);
-      load_entries(bnd_c, 0, ns_c);  // block 1's
+  if (worker) {
+    // block 0's entries into tile 0, block 1's requested; per position: zero the next tile
+    // (between the barriers), then write the next block's entries into it and request those
+    // of the block after
+    const Bnd bnd0 = load_bounds(0);
+    Bnd bnd_c = load_bounds(1), bnd_n = load_bounds(2), bnd_nn = load_bounds(3);
+    zero_tile(lt);
+    zero_tile(lt + TILE);
+    int ns = slots(bnd0, 0);
+    load_entries(bnd0, 0, ns);
+    lds_barrier();  // B0: both tiles zeroed
+    scatter(lt, bnd0, 0, ns);
+    scatter_rest(lt, bnd0);
+    int ns_c = slots(bnd_c, 0);
+    load_entries(bnd_c, 0, ns_c);  // block 1's
 #pragma unroll 1
-      for (int bi = 0; bi < npos; ++bi) {
-        uint16_t* tn = lt + ((bi + 1) & 1) * TILE;
-        lds_barrier();  // B1: tn's previous rows have left
-        zero_tile(tn);
-        lds_barrier();  // B2: tn zeroed
-        scatter(tn, bnd_c, 0, ns_c);  // block bi + 1
-        scatter_rest(tn, bnd_c);
-        bnd_c = bnd_n;
-        bnd_n = bnd_nn;
-        ns_c = slots(bnd_c, 0);
-        load_entries(bnd_c, 0, ns_c);  // block bi + 2
-        bnd_nn = load_bounds(bi + 4);
-      }
-    } else {
-      static_for<0, PD>([&](auto kc) { load_blk(decltype(kc)::value, ring[decltype(kc)::value]); });
-      lds_barrier();  // B0
-#pragma unroll 1
-      for (int bb = 0; bb < npos; bb += PD)
-        static_for<0, PD>([&](auto kc) {
-          constexpr int k = decltype(kc)::value;
-          const int bi = bb + k;
-          uint16_t* tc = lt + (bi & 1) * TILE;
-          lds_barrier();  // B1: block bi's outliers are in tc
-          compute(ring[k], tc);
-          lds_barrier();  // B2: x_hat of block bi in tc
-          store_tile(tc, bi);
-          __builtin_amdgcn_sched_barrier(0);
-          load_blk(bi + PD, ring[k]);
-          __builtin_amdgcn_sched_barrier(0);
-        });
+    for (int bi = 0; bi < npos; ++bi) {
+      uint16_t* tn = lt + ((bi + 1) & 1) * TILE;
+      lds_barrier();  // B1: tn's previous rows have left
+      zero_tile(tn);
+      lds_barrier();  // B2: tn zeroed
+      scatter(tn, bnd_c, 0, ns_c);  // block bi + 1
+      scatter_rest(tn, bnd_c);
+      bnd_c = bnd_n;
+      bnd_n = bnd_nn;
+      ns_c = slots(bnd_c, 0);
+      load_entries(bnd_c, 0, ns_c);  // block bi + 2
+      bnd_nn = load_bounds(bi + 4);
     }
   } else {
     static_for<0, PD>([&](auto kc) { load_blk(decltype(kc)::value, ring[decltype(kc)::value]); });
+    lds_barrier();  // B0
 #pragma unroll 1
     for (int bb = 0; bb < npos; bb += PD)
       static_for<0, PD>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
         const int bi = bb + k;
         uint16_t* tc = lt + (bi & 1) * TILE;
-        lds_barrier();  // B1: tc's previous rows have left
+        lds_barrier();  // B1: block bi's outliers are in tc
         compute(ring[k], tc);
-        lds_barrier();  // B2
+        lds_barrier();  // B2: x_hat of block bi in tc
         store_tile(tc, bi);
         __builtin_amdgcn_sched_barrier(0);
         load_blk(bi + PD, ring[k]);
@@ -1413,17 +1613,18 @@ static int legacy_rows_per_wg(int64_t M, int64_t wg_cols) {
   return 1;
 }
 
-// The row-tile decode (k_legacy_rows) for decodes without dense outliers at 2, 4 and 8 bits,
-// when every workgroup of 4 units has whole units and there are enough blocks for about two
-// workgroups per CU (smaller shapes keep k_legacy_mfma, which splits rows more finely); runs of
-// whole ring rounds (PD blocks).  Returns false where it does not apply.
+// The row-tile decode (k_legacy_rows) for dense COO outliers at 2, 4 and 8 bits from 2^27 elements up,
+// where the COO entries outgrow the caches and their longer contiguous ranges pay (16 % outliers, 2
+// bits: [4, 8192, 8192] 340 us against 352 - 370 us for k_legacy_apply; [4, 3072, 3072] 60 against 50).
+// Runs of whole ring rounds (PD blocks).  Returns false where it does not apply.
 template <int MODE, int BITS, int OSRC>
 static bool legacy_rows_launch(const LegacyArgs& a, int K, int64_t B, hipStream_t st, int* status) {
-  if constexpr (MODE != kDecode || OSRC == 1 || BITS == 1) {
+  if constexpr (MODE != kDecode || OSRC != 3 || BITS == 1) {
     return false;
   } else {
     using Lr = LegacyRows<BITS>;
     const int64_t NB = a.N / Lr::NP, nu = NB / 64, nrb = (a.M + 15) / 16;
+    if (B * a.M * a.N < ((int64_t)1 << 27) || a.ncap == 0) return false;
     if (NB % 64 != 0 || nu < Lr::NW || 16 * a.N * 2 >= ((int64_t)1 << 31)) return false;
     const int64_t ug = (nu + Lr::NW - 1) / Lr::NW, tiles = B * ug;
     const int64_t want = 2 * (int64_t)cu_count();
@@ -1434,18 +1635,12 @@ static bool legacy_rows_launch(const LegacyArgs& a, int K, int64_t B, hipStream_
     runs = (nrb + rbw - 1) / rbw;
     const int64_t nwg = tiles * runs;
     if (nwg > INT32_MAX) return false;
-    const bool coo = OSRC != 0 && a.ncap > 0;
     auto go = [&](auto kern) __attribute__((always_inline)) {
       (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Lr::LDS);
-      *status = launch(kern, dim3((unsigned)nwg), dim3(coo ? 512 : 256), Lr::LDS, st, a, (int)rbw, (int)ug);
+      *status = launch(kern, dim3((unsigned)nwg), dim3(512), Lr::LDS, st, a, (int)rbw, (int)ug);
     };
-    if (K == 16) {
-      if (coo) go(k_legacy_rows<BITS, 16, true>);
-      else go(k_legacy_rows<BITS, 16, false>);
-    } else {
-      if (coo) go(k_legacy_rows<BITS, 32, true>);
-      else go(k_legacy_rows<BITS, 32, false>);
-    }
+    if (K == 16) go(k_legacy_rows<BITS, 16>);
+    else go(k_legacy_rows<BITS, 32>);
     return true;
   }
 }
@@ -1460,7 +1655,11 @@ static int legacy_launch(const LegacyArgs& a, int K, int64_t B, bool mfma_ok, hi
   const int64_t NB = a.N / NP;
   const int rb = legacy_rows_per_wg(a.M, NB / 64 * B);
   const int64_t nwg = (a.M + 64 * rb - 1) / (64 * rb) * (NB / 64) * B;
-  if (mfma_ok && NB % 64 == 0 && nwg <= INT32_MAX) {
+  // (the MFMA decode's store and entry ranges cover 16 rows)
+  constexpr bool kApply = (MODE == kDecode && OSRC != 1) || MODE == kFusedStore || MODE == kFusedSilu ||
+                          MODE == kFusedMul;
+  const bool fits = !kApply || 16 * a.N <= ((int64_t)1 << 24);
+  if (mfma_ok && fits && NB % 64 == 0 && nwg <= INT32_MAX) {
     // 4 row blocks per workgroup, fewer where that would leave under two workgroups per CU
     LegacyArgs la = a;
     la.rb = rb;
@@ -1474,9 +1673,23 @@ static int legacy_launch(const LegacyArgs& a, int K, int64_t B, bool mfma_ok, hi
       const dim3 eg((unsigned)wgs);
       if (K == 16) return launch((k_legacy_encode<BITS, 16, OSRC == 1>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
       return launch((k_legacy_encode<BITS, 32, OSRC == 1>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
+    } else if constexpr (kApply) {
+      const int64_t ug = (NB / 64 + 3) / 4, nrb = (a.M + 15) / 16;
+      const int64_t rbw = std::max<int64_t>(1, std::min<int64_t>(16, B * ug * nrb / (4 * (int64_t)cu_count())));
+      const int64_t wgs = (nrb + rbw - 1) / rbw * ug * B;
+      if (wgs > INT32_MAX) return LRQ_ERR_SHAPE;
+      const dim3 eg((unsigned)wgs);
+      constexpr int kMode = MODE == kFusedStore ? (int)kDecode : MODE;
+      constexpr int kCoo = OSRC >= 2 ? OSRC - 1 : 0;
+      if (kCoo != 0 && a.ncap > 0) {
+        if (K == 16) return launch((k_legacy_apply<kMode, BITS, 16, kCoo>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
+        return launch((k_legacy_apply<kMode, BITS, 32, kCoo>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
+      }
+      if (K == 16) return launch((k_legacy_apply<kMode, BITS, 16, 0>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
+      return launch((k_legacy_apply<kMode, BITS, 32, 0>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
     } else {
-      if (K == 16) return launch((k_legacy_mfma<MODE, BITS, 16, OSRC>), grid, dim3(256), 0, st, la);
-      return launch((k_legacy_mfma<MODE, BITS, 32, OSRC>), grid, dim3(256), 0, st, la);
+      if (K == 16) return launch((k_legacy_mfma<MODE, BITS, 16>), grid, dim3(256), 0, st, la);
+      return launch((k_legacy_mfma<MODE, BITS, 32>), grid, dim3(256), 0, st, la);
     }
   } else {
     const int64_t chunks = (NB + 255) / 256;
@@ -1707,8 +1920,8 @@ extern "C" int lrq_legacy_decode_coo(const void* l, const void* rt, int32_t K, c
   a.qin = (const uint8_t*)q, a.out = (uint16_t*)out, a.M = M, a.N = N;
   a.optr = piece_ptr, a.ocol = cols, a.oval = (const uint16_t*)vals, a.npc = (N + 63) / 64, a.ncap = n_entries;
   const bool mfma_ok = vec_ok({l, rt, q, s, out}) && N % 8 == 0;
-  // more than about 4 entries per 64-column piece (1/16 of the elements): the wave gathers its
-  // pieces' entries cooperatively (an LDS tile); sparser: each lane reads its piece's few entries
+  // more than about 4 entries per 64-column piece (1/16 of the elements): more of a piece's entries are
+  // requested ahead (k_legacy_apply), or the row-tile decode (legacy_rows_launch)
   if (mfma_ok && n_entries * 16 > B * M * N) return legacy_bits<kDecode, 3>(a, K, B, bits, mfma_ok, (hipStream_t)stream);
   return legacy_bits<kDecode, 2>(a, K, B, bits, mfma_ok, (hipStream_t)stream);
 }
@@ -1735,8 +1948,8 @@ extern "C" int lrq_legacy_kth_residual(const void* l, const void* rt, int32_t K,
     if (mfma_ok) {
       a.rb = legacy_rows_per_wg(M, N / 64);
       const dim3 grid((unsigned)((M + 64 * a.rb - 1) / (64 * a.rb) * (N / 64)));  // < 2^26 (M * N < 2^32)
-      if (K == 16) LRQ_TRY(launch((k_legacy_mfma<kHist, 8, 16, 0>), grid, dim3(256), 0, hs, a));
-      else LRQ_TRY(launch((k_legacy_mfma<kHist, 8, 32, 0>), grid, dim3(256), 0, hs, a));
+      if (K == 16) LRQ_TRY(launch((k_legacy_mfma<kHist, 8, 16>), grid, dim3(256), 0, hs, a));
+      else LRQ_TRY(launch((k_legacy_mfma<kHist, 8, 32>), grid, dim3(256), 0, hs, a));
     } else {
       const int64_t chunks = (N + 255) / 256;
       if (M * chunks > INT32_MAX) return LRQ_ERR_SHAPE;
