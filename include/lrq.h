@@ -218,6 +218,12 @@ int lrq_wht128(const void* x, int64_t ldx, int64_t rows, int64_t hidden, void* y
  * [B, M, N] bf16 with leading dims (ldx_b, ldx_m); row-major in N.  Arithmetic follows
  * the reference's torch forms, bf16 rounding after each op. */
 
+/* The factor operands of the calls below, zero-padded to KP = 16 or 32 ranks: rt[N, KP] from r[K, N]
+ * (transposed) and, when lout is given, lout[M, KP] from l[M, K] (K <= KP, contiguous bf16; lout and
+ * rt 16-byte aligned).  The K < 16 rule of the reference (…compression_quantization.py:126-129). */
+int lrq_legacy_factors(const void* l, int64_t M, int32_t K, const void* r, int64_t N, int32_t KP, void* lout, void* rt,
+                       void* stream);
+
 /* Replaces low_rank_addition_fuse_compression_quantization
  * (low_rank_extraction_fuse_compression_quantization.py:118-150; torch form :153-171).
  * o[B, M, N] receives the dense outliers (bf16), q[B, M, N*bits/8] the codes. */

@@ -704,3 +704,15 @@ def test_legacy_rows_largest_dense_coo(pkg, dev, bits, K):
     o = o * (o > 1)
     oc = pkg.compact_outliers(o, capacity=o.numel() // 5)
     assert torch.equal(dec(l, r, q, oc.check(), s, quantize_bit=bits), dec(l, r, q, o, s, quantize_bit=bits))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (65, 8, 63), (64, 16, 64), (130, 17, 1000), (3, 32, 65), (200, 31, 8), (5, 0, 70)])
+def test_legacy_factors(pkg, dev, M, K, N):
+    """r transposed and l, r zero-padded to 16 or 32 ranks."""
+    g = torch.Generator().manual_seed(M + N)
+    l = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    r = torch.randn(K, N, generator=g).to(torch.bfloat16).to(dev)
+    lp, rt, kp = pkg.legacy._factors(l, r)
+    assert kp == (16 if K <= 16 else 32) and lp.shape == (M, kp) and rt.shape == (N, kp)
+    assert torch.equal(lp[:, :K], l) and not lp[:, K:].any()
+    assert torch.equal(rt[:, :K], r.T) and not rt[:, K:].any()

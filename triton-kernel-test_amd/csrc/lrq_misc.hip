@@ -24,6 +24,33 @@ __global__ __launch_bounds__(256) void k_transpose_bf16(const uint16_t* __restri
   }
 }
 
+// The legacy kernels' factor operands in one launch: rt[N, KP] = r[K, N]^T with zero columns K .. KP - 1,
+// and (lout given) lout[M, KP] = l[M, K] with the same zero columns.  Workgroups of one wave: the
+// first ceil(N / 64) take 64 columns of r each (a lane reads its column's K values, 128-byte rows of
+// them per load, and writes its rt row), the others 64 rows of l.  Launch-bound; with r in 32x32 LDS
+// tiles it took 4.2 - 5.5 us per call at [16, 4096] .. [32, 4096], and padding l and r four more launches.
+template <int KP>
+__global__ __launch_bounds__(64) void k_legacy_factors(const uint16_t* __restrict__ l, int64_t M, int K,
+                                                       const uint16_t* __restrict__ r, int64_t N,
+                                                       uint16_t* __restrict__ lout, uint16_t* __restrict__ rt) {
+  const int64_t nwg = (N + 63) / 64;
+  const bool left = blockIdx.x >= nwg;  // uniform
+  const int64_t i = (left ? blockIdx.x - nwg : (int64_t)blockIdx.x) * 64 + threadIdx.x;
+  if (i >= (left ? M : N)) return;
+  const uint16_t* src = left ? l + i * K : r + i;
+  const int64_t step = left ? 1 : N;
+  uint16_t v[KP];
+#pragma unroll
+  for (int k = 0; k < KP; ++k) v[k] = src[min(k, K - 1) * step];
+  uint32_t d[KP / 2];
+#pragma unroll
+  for (int k = 0; k < KP / 2; ++k)
+    d[k] = (2 * k < K ? (uint32_t)v[2 * k] : 0u) | (2 * k + 1 < K ? (uint32_t)v[2 * k + 1] << 16 : 0u);
+  uint16_t* dst = (left ? lout : rt) + i * KP;
+#pragma unroll
+  for (int k = 0; k < KP / 8; ++k) st16(dst + 8 * k, u32x4{d[4 * k], d[4 * k + 1], d[4 * k + 2], d[4 * k + 3]});
+}
+
 // colmax[c] = max |x[r, c]| via an unsigned max on the fp32 bit pattern (valid for
 // non-negative floats).  colmax must be zeroed first (done by the host entry).
 // Grid: (ceil(cols / 512), row groups of rows_per rows); PH waves = PH row phases x 64 column
@@ -300,6 +327,19 @@ __global__ __launch_bounds__(kIndexThreads) void k_outlier_index(const int32_t* 
     const int64_t r = i / nd;
     side[(r0 + r) * ldside + dropped[i - r * nd]] = 0;
   }
+}
+
+extern "C" int lrq_legacy_factors(const void* l, int64_t M, int32_t K, const void* r, int64_t N, int32_t KP, void* lout,
+                                  void* rt, void* stream) {
+  if (r == nullptr || rt == nullptr || (lout != nullptr && l == nullptr)) return LRQ_ERR_NULL;
+  if (M < 0 || N < 0 || K < 1 || K > KP) return LRQ_ERR_SHAPE;
+  if (KP != 16 && KP != 32) return LRQ_ERR_UNSUPPORTED;
+  if (!aligned(l, 2) || !aligned(r, 2) || !aligned(lout, 16) || !aligned(rt, 16)) return LRQ_ERR_ALIGN;
+  const int64_t wgs = (N + 63) / 64 + (lout != nullptr ? (M + 63) / 64 : 0);
+  if (wgs > INT32_MAX) return LRQ_ERR_SHAPE;
+  if (wgs == 0) return LRQ_OK;
+  return launch(KP == 16 ? k_legacy_factors<16> : k_legacy_factors<32>, dim3((unsigned)wgs), dim3(64), 0,
+                (hipStream_t)stream, (const uint16_t*)l, M, (int)K, (const uint16_t*)r, N, (uint16_t*)lout, (uint16_t*)rt);
 }
 
 // k_colmax launch shape: one workgroup of 8 waves per CU (c3 shape, colmax entry: 36.1 us;

@@ -75,15 +75,15 @@ def _factors(l: torch.Tensor, r: torch.Tensor):
         raise AssertionError("Incompatible dimensions")
     if K > 32:
         raise ValueError("liblrq supports low-rank factors of rank <= 32")
+    if K == 0:  # no low-rank term: one zero rank
+        l, r, K = l.new_zeros((M, 1)), r.new_zeros((1, N)), 1
     kp = 16 if K <= 16 else 32
-    if kp != K:
-        l = torch.cat([l, torch.zeros((M, kp - K), device=l.device, dtype=l.dtype)], dim=1)
-        r = torch.cat([r, torch.zeros((kp - K, N), device=r.device, dtype=r.dtype)], dim=0)
     l = l.to(torch.bfloat16).contiguous()
     r = r.to(torch.bfloat16).contiguous()
     rt = torch.empty((N, kp), dtype=torch.bfloat16, device=r.device)
-    call("lrq_transpose_bf16", _p(r), kp, N, _p(rt), _stream(r.device))
-    return l, rt, kp
+    lp = l if kp == K else torch.empty((M, kp), dtype=torch.bfloat16, device=l.device)
+    call("lrq_legacy_factors", _p(l), M, K, _p(r), N, kp, _p(None if kp == K else lp), _p(rt), _stream(r.device))
+    return lp, rt, kp
 
 
 def _scale(s: torch.Tensor, B: int, N: int) -> torch.Tensor:
