@@ -147,16 +147,24 @@ def check(code: int, what: str) -> None:
     raise RuntimeError(msg)
 
 
+_bound: dict = {}  # name -> the library's function, bound on its first call
+
+
 def call_raw(name: str, *args) -> int:
     """Call an entry point and return its status without raising."""
-    lib = load()
-    if name in _missing:
-        raise RuntimeError(f"{name} is not exported by {LIB_PATH}")
-    return int(getattr(lib, name)(*args))
+    fn = _bound.get(name)
+    if fn is None:
+        lib = load()
+        if name in _missing:
+            raise RuntimeError(f"{name} is not exported by {LIB_PATH}")
+        fn = _bound[name] = getattr(lib, name)
+    return fn(*args)
 
 
 def call(name: str, *args) -> None:
-    check(call_raw(name, *args), name)
+    st = call_raw(name, *args)
+    if st:
+        check(st, name)
 
 
 __all__ = ["LrqTensors", "load", "call", "call_raw", "check", "status_string", "missing_symbols", "SIGNATURES",

@@ -38,12 +38,37 @@ __all__ = [
 ]
 
 
-def _p(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+# Host time is most of a short sequence's call (encode + decode of [33, 1024]: 28 us a pass for 12 us of
+# kernels), so what every call does is kept lean: plain integers for pointers and streams, one
+# constructor call for a descriptor, and the device guard only where another device is current.
+def _p(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device: torch.device) -> int:
+    """The raw handle of torch's current stream on `device`."""
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
+
+
+class _NoGuard:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_no_guard = _NoGuard()
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing to enter where it is the current one already."""
+    return _no_guard if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def _require_device(*ts):
@@ -92,7 +117,7 @@ class LowRankBasis:
     def Vt(self) -> torch.Tensor:
         if self._vt is None:
             vt = torch.empty((self.rank, self.hidden), dtype=torch.bfloat16, device=self.V.device)
-            with torch.cuda.device(self.V.device):
+            with _on(self.V.device):
                 call("lrq_transpose_bf16", _p(self.V), self.hidden, self.rank, _p(vt), _stream(self.V.device))
             self._vt = vt
         return self._vt
@@ -153,23 +178,21 @@ class CompressedActivation:
         return n
 
     def descriptor(self, for_encode: bool = False) -> LrqTensors:
-        t = LrqTensors()
-        t.rows, t.hidden = self.rows, self.hidden
-        t.rank, t.bits, t.group = self.rank, self.bits, self.group
+        codes, qparams, basis, rank = self.codes, self.qparams, self.basis, self.rank
         # encode sets the flag itself when it hands the library the unrotated activation (see
         # ``encode``); every other entry point sees the flag
-        t.flags = _lib.LRQ_FLAG_HADAMARD if (self.hadamard and not for_encode) else 0
-        if self.rank:
-            t.L, t.ld_L = self.L.data_ptr(), self.L.stride(0)
-            t.V = self.basis.V.data_ptr()
-            if for_encode:
-                t.Vt = self.basis.Vt.data_ptr()
-        t.codes, t.ld_codes = self.codes.data_ptr(), self.codes.stride(0)
-        t.qparams, t.ld_qp = self.qparams.data_ptr(), self.qparams.stride(0)
-        if self.idx is not None and self.idx.numel() > 0:
-            t.outlier_idx, t.n_outlier = self.idx.data_ptr(), self.idx.numel()
-            t.side, t.ld_side = self.side.data_ptr(), self.side.stride(0)
-        return t
+        flags = _lib.LRQ_FLAG_HADAMARD if (self.hadamard and not for_encode) else 0
+        idx, side = self.idx, self.side
+        if idx is not None and idx.numel() > 0:
+            outliers = (idx.data_ptr(), idx.numel(), side.data_ptr(), side.stride(0))
+        else:
+            outliers = (None, 0, None, 0)
+        if rank:
+            low = (self.L.data_ptr(), self.L.stride(0), basis.V.data_ptr(), basis.Vt.data_ptr() if for_encode else None)
+        else:
+            low = (None, 0, None, None)
+        return LrqTensors(codes.shape[0], self.shape[-1], rank, self.bits, self.group, flags, *low, codes.data_ptr(),
+                          codes.stride(0), qparams.data_ptr(), qparams.stride(0), *outliers)
 
 
 def _alloc(rows: int, n: int, bits: int, group: int, rank: int, k: int, device) -> dict:
@@ -208,7 +231,7 @@ def _sanitize_index(idx: torch.Tensor, n: int, side: torch.Tensor) -> torch.Tens
     synchronisation)."""
     k = idx.numel()
     out = torch.empty_like(idx)
-    with torch.cuda.device(idx.device):
+    with _on(idx.device):
         st = _lib.call_raw("lrq_outlier_index", _p(idx), k, n, _p(out), side.shape[0], _p(side), side.stride(0),
                            _stream(idx.device))
     if st != _lib.LRQ_ERR_UNSUPPORTED:
@@ -255,7 +278,7 @@ def encode(x: torch.Tensor, basis: Optional[LowRankBasis | torch.Tensor] = None,
                              basis=basis, side=bufs["side"], idx=outlier_idx if k else None,
                              shape=tuple(x.shape), bits=bits, group=group_size, hadamard=hadamard)
     t = c.descriptor(for_encode=True)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         if hadamard:
             # rotated format: the library rotates x as it reads it where it can (flagged
             # descriptor); otherwise y = bf16(WHT128(x)) into a temporary, then the plain encode
@@ -285,7 +308,7 @@ def wht128(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     o = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if out is None else out
     if o.shape != x.shape or o.dtype != torch.bfloat16 or not o.is_contiguous():
         raise ValueError("out must be a contiguous bf16 tensor of x's shape")
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         call("lrq_wht128", _p(x2), ldx, rows, n, _p(o), n, _stream(x.device))
     return o
 
@@ -310,7 +333,7 @@ def decode(c: CompressedActivation, out: Optional[torch.Tensor] = None) -> torch
     """Reconstruct x_hat (bf16, the activation's shape)."""
     o = _out_like(c, out)
     t = c.descriptor()
-    with torch.cuda.device(c.device):
+    with _on(c.device):
         call("lrq_decode", ctypes.byref(t), _p(o), c.hidden, _stream(c.device))
     return o
 
@@ -323,7 +346,7 @@ def _fused(name: str, c: CompressedActivation, y: torch.Tensor, argname: str) ->
     y2, ldy = _operand(c, y, argname)
     o = _out_like(c, None)
     t = c.descriptor()
-    with torch.cuda.device(c.device):
+    with _on(c.device):
         call(name, ctypes.byref(t), _p(y2), ldy, _p(o), c.hidden, _stream(c.device))
     return o
 
@@ -359,7 +382,7 @@ def dequant_gemm(c: CompressedActivation, a: torch.Tensor, out_dtype=torch.float
         raise ValueError("out_dtype must be float32 or bfloat16")
     o = torch.empty((c.rows, n_out), dtype=out_dtype, device=c.device)
     t = c.descriptor()
-    with torch.cuda.device(c.device):
+    with _on(c.device):
         call("lrq_dequant_gemm", ctypes.byref(t), _p(a), n_out, _p(o), n_out,
              1 if out_dtype == torch.float32 else 0, _stream(c.device))
     return o.reshape(tuple(c.shape[:-1]) + (n_out,))
@@ -383,7 +406,7 @@ def dequant_gemm_t(c: CompressedActivation, g: torch.Tensor, out_dtype=torch.flo
         _lib.check(ws_bytes, "lrq_dequant_gemm_t_workspace")
     ws = torch.empty((max(ws_bytes, 16) + 15) // 16 * 4, dtype=torch.float32, device=c.device)
     o = torch.empty((c.hidden, n_out), dtype=out_dtype, device=c.device)
-    with torch.cuda.device(c.device):
+    with _on(c.device):
         call("lrq_dequant_gemm_t", ctypes.byref(t), _p(g2), n_out, n_out, _p(o), n_out,
              1 if out_dtype == torch.float32 else 0, _p(ws), ws.numel() * 4, _stream(c.device))
     return o
@@ -417,7 +440,7 @@ def lora_grads(c: CompressedActivation, a: torch.Tensor, g: torch.Tensor, xa_dty
     ws = torch.empty((max(ws_bytes, 16) + 15) // 16 * 4, dtype=torch.float32, device=c.device)
     xa = torch.empty((c.rows, n_out), dtype=xa_dtype, device=c.device)
     da = torch.empty((c.hidden, n_out), dtype=da_dtype, device=c.device)
-    with torch.cuda.device(c.device):
+    with _on(c.device):
         call("lrq_lora_grads", ctypes.byref(t), _p(a2), n_out, _p(g2), n_out, n_out, _p(xa), n_out,
              1 if xa_dtype == torch.float32 else 0, _p(da), n_out, 1 if da_dtype == torch.float32 else 0,
              _p(ws), ws.numel() * 4, _stream(c.device))
@@ -437,7 +460,7 @@ def dequant_gemm_t_noalloc(c: CompressedActivation, g: torch.Tensor, out: torch.
             or not out.is_contiguous():
         raise ValueError("out must be a contiguous fp32 or bf16 [N, n]")
     t = c.descriptor()
-    with torch.cuda.device(c.device):
+    with _on(c.device):
         call("lrq_dequant_gemm_t_noalloc", ctypes.byref(t), _p(g), n_out, n_out, _p(out), n_out,
              1 if out.dtype == torch.float32 else 0, _stream(c.device))
     return out
@@ -448,7 +471,7 @@ def column_absmax(x: torch.Tensor) -> torch.Tensor:
     _require_device(x)
     x2, rows, n, ldx = _rows_view(x)
     out = torch.empty((n,), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         call("lrq_colmax", _p(x2), ldx, rows, n, _p(out), _stream(x.device))
     return out
 
@@ -458,7 +481,7 @@ def topk_channels(colmax: torch.Tensor, k: int) -> torch.Tensor:
     _require_device(colmax)
     colmax = colmax.to(torch.float32).contiguous()
     idx = torch.empty((k,), dtype=torch.int32, device=colmax.device)
-    with torch.cuda.device(colmax.device):
+    with _on(colmax.device):
         call("lrq_topk", _p(colmax), colmax.numel(), k, _p(idx), _stream(colmax.device))
     return idx
 

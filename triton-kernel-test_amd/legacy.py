@@ -37,7 +37,7 @@ import torch
 
 from . import _lib
 from ._lib import call
-from .api import _p, _require_device, _stream
+from .api import _on, _p, _require_device, _stream
 
 __all__ = [
     "low_rank_addition_fuse_compression_quantization",
@@ -156,7 +156,7 @@ class LegacyOutliers:
             return int(self.nnz.item()), None
         rows = ix[3 - nd:]
         out = torch.empty((_CHECK_WGS + 1,), dtype=torch.int64, device=ix.device)
-        with torch.cuda.device(ix.device):
+        with _on(ix.device):
             call("lrq_coo_check", _p(rows), rows.stride(0), nd, self.capacity, _p(self.nnz), *dims, _p(out),
                  out.numel(), _stream(ix.device))
         count, *bad = out.tolist()
@@ -193,7 +193,7 @@ def compact_outliers(o: torch.Tensor, capacity: Optional[int] = None) -> LegacyO
     cap = max(1024, o.numel() // 32) if capacity is None else int(capacity)
     dev = o.device
     bf = _coo_buffers(B, M, N, cap, dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         call("lrq_coo_compact", _p(o), B, M, N, _p(bf["idx"]), cap, _p(bf["vals"]), cap, _p(bf["nnz"]),
              _p(bf["ptr"]), _p(bf["ws"]), bf["ws"].numel() * 8, _stream(dev))
     return LegacyOutliers(bf["idx"], bf["vals"], bf["nnz"], bf["ptr"], tuple(o.shape))
@@ -251,7 +251,7 @@ def _encode_coo(l, r, x, s, bits: int, outlier: float, capacity: Optional[int]):
         raise ValueError(f"x must be [B, {M}, {N}]")
     if x.stride(2) != 1:
         x = x.contiguous()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         l2, rt, K = _factors(l, r)
         s2 = _scale(s, B, N)
         o = torch.empty((B, M, N), device=x.device, dtype=torch.bfloat16)
@@ -303,7 +303,7 @@ def low_rank_addition_fuse_decompression_dequantization(l, r, q, o, s, quantize_
         _require_device(o)
         if not coo:
             o = o.to(torch.bfloat16).contiguous()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         l2, rt, K = _factors(l, r)
         s2 = _scale(s, B, N)
         x = torch.empty((B, M, N), device=q.device, dtype=torch.bfloat16)
@@ -331,7 +331,7 @@ def residual_kthvalue(l, r, x, k: int) -> torch.Tensor:
         x = x.contiguous()
     out = torch.empty((), dtype=torch.float32, device=x.device)
     ws = torch.empty((256,), dtype=torch.int64, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         l2, rt, K = _factors(l, r)
         call("lrq_legacy_kth_residual", _p(l2), _p(rt), K, _p(x), M, N, x.stride(0), int(k), _p(out), _p(ws),
              ws.numel() * 8, _stream(x.device))
@@ -356,7 +356,7 @@ def low_rank_addition(l, r, x):
     _, N = r.shape
     B = x.shape[0]
     x = x.contiguous()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         l2, rt, K = _factors(l, r)
         o = torch.empty((B, M, N), device=x.device, dtype=torch.bfloat16)
         call("lrq_lowrank_add", _p(l2), _p(rt), K, _p(x), B, M, N, _p(o), _stream(x.device))
@@ -375,7 +375,7 @@ def _legacy_fused(op, l, r, q, s, b, quantize_bit):
         if tuple(b.shape) != (B, M, N):
             raise ValueError(f"second operand must be [{B}, {M}, {N}]")
         b = b.to(torch.bfloat16).contiguous()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         l2, rt, K = _factors(l, r)
         s2 = _scale(s, B, N)
         c = torch.empty((B, M, N), device=q.device, dtype=torch.bfloat16)
@@ -425,7 +425,7 @@ def triton_matmul_decompress(q, l, r, s, y, quantize_bit=2):
     if npad != n:
         y = torch.nn.functional.pad(y, (0, npad - n))
     y = y.contiguous()
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         l2, rt, K = _factors(l, r)
         s2 = _scale(s, B, N)
         o = torch.empty((B, M, npad), device=q.device, dtype=torch.bfloat16)
@@ -442,7 +442,7 @@ def _dense(op, x, y):
     x = x.to(torch.bfloat16).contiguous()
     y = y.to(torch.bfloat16).contiguous()
     o = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         call("lrq_dense_elementwise", op, _p(x), _p(y), _p(o), x.numel(), _stream(x.device))
     return o
 
@@ -470,7 +470,7 @@ def triton_softmax_backward(y, grad_y):
     y2 = y.to(torch.bfloat16).contiguous()
     g2 = grad_y.to(torch.bfloat16).contiguous()
     o = torch.empty_like(y2)
-    with torch.cuda.device(y.device):
+    with _on(y.device):
         call("lrq_dense_softmax_bwd", _p(y2), _p(g2), _p(o), y2.numel() // n, n, _stream(y.device))
     return o
 
@@ -483,7 +483,7 @@ def torch_extract_unstructured(x, threshold):
     o = torch.empty_like(x2)
     rest = torch.empty_like(x2)
     tau = float(threshold.item() if isinstance(threshold, torch.Tensor) else threshold)
-    with torch.cuda.device(x2.device):
+    with _on(x2.device):
         call("lrq_threshold_split", _p(x2), x2.numel(), tau, _p(o), _p(rest), _stream(x2.device))
     return _to_sparse(o), rest
 
@@ -500,6 +500,6 @@ def torch_extract_channel(x, channel_index):
         raise ValueError("channel_index must not repeat")
     B, M, N = x.shape
     out = torch.empty((B, idx.numel(), N), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         call("lrq_gather_rows_zero", _p(x), B, M, N, _p(idx), idx.numel(), _p(out), _stream(x.device))
     return out, x
