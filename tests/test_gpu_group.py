@@ -84,6 +84,41 @@ def test_encode_decode_formats(pkg, dev, rows, hidden, rank, bits, group):
     assert d.max() <= 1 and (d > 0).mean() <= 1e-3, (d.max(), (d > 0).mean())
 
 
+@pytest.mark.parametrize("rows,hidden,rank,bits,group", [
+    (1, 128, 16, 4, 64),       # one unit
+    (33, 896, 16, 4, 64),      # seven units: a wave without one
+    (40, 1152, 32, 4, 64),     # nine units, rank 32
+    (9000, 384, 16, 4, 64),    # several row blocks per workgroup, two workgroups per CU
+    (5003, 3072, 16, 4, 64),   # 24 units, ragged rows
+    (64, 3072, 32, 4, 64),     # the widest at rank 32
+    (47, 4864, 16, 4, 64),     # 38 units: the widest
+    (4100, 2176, 16, 4, 64),   # 17 units: plane 1 starts in the middle of a tile
+    (50, 1152, 0, 4, 64),      # rank 0, odd
+    (70, 4992, 0, 4, 64),      # rank 0, 39 units
+    (37, 1280, 16, 8, 128),    # int8, ten units
+    (4200, 3328, 16, 8, 128),  # int8, 26 units
+    (33, 4864, 16, 8, 128),
+])
+def test_encode_any_width(pkg, dev, rows, hidden, rank, bits, group):
+    """The single-pass encode of widths without an instantiation of their own (k_encode_any), against
+    the oracle; its L within the accumulation bound, its codes those of its own L."""
+    x = pkg.inputs.activation(rows, hidden, n_outlier=2, outlier_scale=20.0, seed=rows + hidden)
+    V = pkg.inputs.basis(hidden, rank, seed=9) if rank else None
+    _check_encode(pkg, dev, x, V, bits, group)
+
+
+@pytest.mark.parametrize("rows,hidden,rank,bits,group", [(50, 2304, 16, 4, 64), (4100, 3584, 16, 4, 64), (33, 1536, 32, 4, 64),
+                                                         (70, 1280, 16, 8, 128), (40, 4864, 16, 4, 64)])
+def test_encode_any_width_rotated(pkg, dev, rows, hidden, rank, bits, group):
+    """The same kernel rotating its tiles in LDS: the codes of the separate rotation's encode wherever L
+    agrees."""
+    x = pkg.inputs.activation(rows, hidden, n_outlier=2, outlier_scale=20.0, seed=rows).to(dev)
+    V = pkg.inputs.basis(hidden, rank, seed=9).to(dev)
+    a = pkg.encode(x, V, bits=bits, group_size=group, hadamard=True)
+    b = pkg.encode(pkg.wht128(x), V, bits=bits, group_size=group)
+    assert torch.equal(a.L, b.L) and torch.equal(a.codes, b.codes) and torch.equal(a.qparams, b.qparams)
+
+
 @pytest.mark.parametrize("rows,hidden,rank,bits,group,k", [
     (100, 4096, 16, 4, 64, 41),   # row-staged single pass (4 units per wave), config 3's channel count
     (5000, 4096, 16, 4, 64, 8),   # several row blocks per workgroup, ragged

@@ -1,7 +1,7 @@
 """CPU replay of the direct global-to-LDS loads (ld16_to_lds, csrc/lrq_common.h).
 
-Five kernels move 16 bytes per lane from global memory straight into LDS with
-__builtin_amdgcn_global_load_lds: k_encode_rows and k_encode_tiles (csrc/lrq_encode.hip),
+Six kernels move 16 bytes per lane from global memory straight into LDS with
+__builtin_amdgcn_global_load_lds: k_encode_rows, k_encode_tiles and k_encode_any (csrc/lrq_encode.hip),
 k_softmax_rows (csrc/lrq_rowops.hip), k_wht_rows (csrc/lrq_wht.hip) and k_legacy_encode
 (csrc/lrq_legacy.hip).  This file restates, in numpy, the
 host launch arithmetic (grid, row blocks per workgroup) and each kernel's source and
@@ -269,6 +269,59 @@ def test_wht_rows_direct_loads_stay_in_bounds(cus):
     for rows, N, extra in [(16384, 5120, 0), (20000, 512, 0), (64, 1024, 0), (33, 2048, 0), (100, 4096, 8),
                            (1, 512, 0), (5000, 5120, 0)]:
         n += wht_rows_replay(rows, N, N + extra, cus)
+    assert n > 0
+
+
+# ----------------------------------------------------------------------------- k_encode_any
+def encode_any_replay(M, N, ldx, cus, bits, per_cu):
+    """k_encode_any as encode_any_dispatch() launches it, and the read-back of every unit's columns."""
+    TILE, NP, U = 4096, 8 // bits, N // 128
+    alloc = U * TILE
+    nrb = (M + 15) // 16
+    rbw, grid = _rows_per_wg(nrb, cus * per_cu)
+    lane = np.arange(64)
+    lr, lq, j, g = lane >> 4, lane & 15, lane & 15, lane >> 4
+    checked = 0
+    for rbs in _blocks(grid, rbw, nrb):
+        for rb in rbs:
+            lim = M - 1 - rb * 16
+            where = {}  # (tile, row, position) -> chunk of the row
+            dsts = []
+            for w in range(8):
+                for t in range(w, U, 8):
+                    for k in range(4):
+                        r = 4 * k + lr
+                        gsrc = (rb * 16 * ldx) * 2 + 256 * t + np.minimum(r, lim) * ldx * 2 + 16 * (lq ^ r)
+                        ldst = t * TILE + 1024 * k + 16 * lane
+                        _check(gsrc, ldst, gbytes=((M - 1) * ldx + N) * 2, lds_alloc=alloc, lo=t * TILE, hi=(t + 1) * TILE,
+                               what=f"k_encode_any {M}x{N}")
+                        dsts.append(ldst)
+                        checked += 64
+                        for ll in range(0, 64, 7):
+                            where[(t, int(r[ll]), int(lq[ll]))] = int(lq[ll] ^ r[ll])
+            d = np.concatenate(dsts)
+            assert np.unique(d).size == d.size
+            for u in range(U):
+                for p in range(NP):
+                    c = p * U + u if NP == 2 else 2 * u
+                    for k in range(4 // NP):
+                        chunk = 8 * (c & 1) + (4 // NP) * g + k
+                        col = 128 * (c // 2) + 8 * chunk
+                        want = p * (N // NP) + u * (128 // NP) + (32 // NP) * g + 8 * k
+                        assert (col == want).all()
+                        for ll in range(0, 64, 5):
+                            key = (c // 2, int(j[ll]), int(chunk[ll] ^ j[ll]))
+                            if key in where:
+                                assert where[key] == chunk[ll]
+    return checked
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("cus", CU_COUNTS)
+def test_encode_any_direct_loads_stay_in_bounds(cus, bits):
+    n = 0
+    for M, N, extra, per in [(1, 128, 0, 2), (33, 896, 8, 2), (40, 1152, 0, 1), (100, 3072, 0, 1), (47, 4864, 0, 1)]:
+        n += encode_any_replay(M, N, N + extra, cus, bits, per)
     assert n > 0
 
 

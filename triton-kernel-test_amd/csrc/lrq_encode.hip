@@ -812,6 +812,172 @@ __global__ __launch_bounds__(512) void k_encode_tiles(const uint16_t* __restrict
 }
 
 // -------------------------------------------------------------------------------------
+// Single-pass encode for any width whose 16-row block fits the LDS (int4/g64 and int8/g128 at rank 16 up
+// to 38 units of 128 elements, int4/g64 at rank 32 up to 24 units and, for odd unit counts, at rank 0).
+//
+// As in k_encode_tiles the block lives in LDS as N/128 tiles of 16 rows x 128 columns (row r's 16-byte
+// chunk c at position c ^ r), wave w loads (and with ROT rotates) tiles w, w + 8, ... and quantises units
+// w, w + 8, ... (a wave has UPW or UPW - 1 of them); unit u of plane p is the 64-column half (p U + u) % 2
+// of tile (p U + u) / 2 at int4, tile u at int8.  Per block: own tiles landed (and rotated) | barrier |
+// the units' columns into registers | barrier | the next block's tiles requested | projection partials,
+// barrier, L summed in wave order | units quantised.  Up to 8 units two workgroups share a CU (one's
+// loads under the other's work).
+// Against the two slab passes and the slab reduction, which read X twice: [5003, 3072] int4 rank 16
+// 10.2 + 4.0 + 11.9 us.
+template <int BITS, int G, int R, int UPW>
+struct AnyEnc {
+  static constexpr int NW = 8, TILE = 16 * 256, RT = R > 0 ? R / 16 : 1, PART = R > 0 ? NW * RT * 64 * 16 : 0;
+  static constexpr int kPerCu = UPW == 1 && R <= 16 ? 2 : 1;  // workgroups per CU (two would spill from two units a wave up)
+  static size_t bytes(int U) { return (size_t)U * TILE + PART; }
+  static_assert(G * (8 / BITS) == 128, "a unit is 128 elements of a row");
+};
+
+template <int BITS, int G, int R, int UPW, bool ROT>
+__global__ __launch_bounds__(512, (2 * AnyEnc<BITS, G, R, UPW>::kPerCu)) void k_encode_any(
+    const uint16_t* __restrict__ X, int64_t ldx, int M, int N, const uint16_t* __restrict__ V,
+    uint16_t* __restrict__ Lout, int64_t ldl, uint8_t* __restrict__ codes, int64_t ldc, uint16_t* __restrict__ qparams,
+    int64_t ldq, int RBW) {
+  using Ae = AnyEnc<BITS, G, R, UPW>;
+  constexpr int NP = 8 / BITS, CPG = G / 32, RT = Ae::RT, NW = Ae::NW, TILE = Ae::TILE;
+  extern __shared__ __attribute__((aligned(16))) unsigned char shm[];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const int U = N / 128, nrb = (M + 15) / 16;
+  const int rb0 = blockIdx.x * RBW;
+  if (rb0 >= nrb) return;  // whole workgroup (no barrier reached)
+  const int nblk = min(RBW, nrb - rb0);
+  const int nl = U <= w ? 0 : (U - w + NW - 1) / NW;  // this wave's tiles and units (wave-uniform): UPW or UPW - 1
+  f32x4* part = reinterpret_cast<f32x4*>(shm + (size_t)U * TILE);  // [NW][RT][64]
+
+  // tile i of this wave: rows 4k .. 4k + 3 per load; lane l covers row 4k + l / 16, chunk (l % 16) ^ row,
+  // landing at position l % 16 (rows past the end clamp to the last row)
+  const int lr = lane >> 4, lq = lane & 15;
+  const uint32_t ldx2 = (uint32_t)ldx * 2u;
+  auto issue = [&](int rb) __attribute__((always_inline)) {
+    const int lim = M - 1 - rb * 16;  // last row of the block that exists (>= 0)
+#pragma unroll
+    for (int i = 0; i < UPW; ++i) {
+      if (i < nl) {  // (uniform)
+        const int t = w + NW * i;
+        const unsigned char* base = reinterpret_cast<const unsigned char*>(X + (int64_t)rb * 16 * ldx) + 256 * t;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int r = 4 * k + lr;
+          ld16_to_lds(base + ((uint32_t)min(r, lim) * ldx2 + 16u * (uint32_t)(lq ^ r)), shm + (size_t)t * TILE + 1024 * k);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  issue(rb0);
+  u32x2 vop[UPW][NP][G / 16][RT];
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int i = 0; i < UPW; ++i)
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+        if (i < nl) load_vops<G, R>(V, unit_base(p, w + NW * i, N, NP, G), j, g, vop[i][p]);
+  }
+
+#pragma unroll 1
+  for (int b = 0; b < nblk; ++b) {
+    const int rb = __builtin_amdgcn_readfirstlane(rb0 + b);
+    const int row = min(rb * 16 + j, M - 1);
+    // Own tiles landed: after their loads this wave issued the previous block's stores (each unit's, and
+    // the L rows'), which need not complete here; memory operations retire in issue order.
+    constexpr int kUnit = quant_unit_stores<G>(), kL = R > 0 ? RT : 0;
+    if (b == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    else if (nl == UPW) __builtin_amdgcn_s_waitcnt(vmcnt_imm(UPW * kUnit + kL));
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm((UPW - 1) * kUnit + kL));
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ROT) {
+      // the sign operands, formed per block (the empty asm hides that they are loop-invariant, so they
+      // do not stay live across the quantisation)
+      int jj = j;
+      asm volatile("" : "+v"(jj));
+      u32x4 op[2][2];
+      wht_operands_from_pair(wht_sign_dword(jj, g, 0, false, 0), wht_sign_dword(jj, g, 0, false, 1), op);
+#pragma unroll
+      for (int i = 0; i < UPW; ++i)
+        if (i < nl) wht128_lds_swz(shm + (size_t)(w + NW * i) * TILE + 256 * j, g, j, op);
+    }
+    lds_barrier();  // every tile landed and rotated
+    u32x4 x[UPW][NP][CPG];
+#pragma unroll
+    for (int i = 0; i < UPW; ++i)
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        if (i < nl) {
+          const int c = NP == 2 ? p * U + w + NW * i : 2 * (w + NW * i);  // first 64-column half
+          const unsigned char* tr = shm + (size_t)(c / 2) * TILE + 256 * j;
+#pragma unroll
+          for (int k = 0; k < CPG; ++k)
+            x[i][p][k] = *reinterpret_cast<const u32x4*>(tr + 16 * ((8 * (c & 1) + CPG * g + k) ^ j));
+        }
+      }
+    lds_barrier();  // every wave's reads of the block returned: the tiles may be refilled
+    if (b + 1 < nblk) issue(rb + 1);
+
+    u32x2 lop[RT], lopn[RT];
+    if constexpr (R > 0) {
+      f32x4 acc[2][RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) acc[0][t] = acc[1][t] = zero4();
+      {
+        int jj = j;  // (as for the rotation's operands)
+        asm volatile("" : "+v"(jj));
+        const u32x2 ident = identity_bop(jj, g);
+#pragma unroll
+        for (int i = 0; i < UPW; ++i)
+#pragma unroll
+          for (int p = 0; p < NP; ++p)
+            if (i < nl) project_unit<G, R>(vop[i][p], x[i][p], ident, acc[(i * NP + p) & 1]);
+      }
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        f32x4 a = acc[0][t];
+        a[0] += acc[1][t][0];
+        a[1] += acc[1][t][1];
+        a[2] += acc[1][t][2];
+        a[3] += acc[1][t][3];
+        part[(w * RT + t) * 64 + lane] = a;
+      }
+      lds_barrier();  // (the next block's partials come two barriers after these are read)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        f32x4 sum = part[t * 64 + lane];
+#pragma unroll
+        for (int w2 = 1; w2 < NW; ++w2) {
+          const f32x4 o = part[(w2 * RT + t) * 64 + lane];
+          sum[0] += o[0];
+          sum[1] += o[1];
+          sum[2] += o[2];
+          sum[3] += o[3];
+        }
+        // lane (j, g) holds L[row j][16t + 4g + v]
+        lop[t] = u32x2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+        lopn[t] = neg_bf16x4(lop[t]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint8_t* crow = codes + (int64_t)row * ldc;
+    uint16_t* qrow = qparams + (int64_t)row * ldq;
+#pragma unroll
+    for (int i = 0; i < UPW; ++i) {
+      if (i < nl) quant_unit<BITS, G, R>(x[i], vop[i], lopn, nullptr, w + NW * i, N, g, crow, qrow);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (R > 0) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        st8_pred(Lout + (int64_t)rb * 16 * ldl, (uint32_t)(16 * ldl * 2), (uint32_t)(((row - rb * 16) * ldl + 16 * t + 4 * g) * 2),
+                 lop[t], w == 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// -------------------------------------------------------------------------------------
 // Projection only (first pass of the two-pass encode).  Grid: ceil(rows / 16) workgroups
 // of 4 waves; wave w sums 32-column chunks w, w + 4, ... of the row.  Uses V^T [R, N].
 template <int R>
@@ -1399,6 +1565,50 @@ static int encode_persist_dispatch(const lrq_tensors* t, const void* x, int64_t 
   }
 }
 
+// k_encode_any: about as many workgroups as fit the CUs at once, each walking consecutive row blocks.
+// Where it does not apply (or the device refuses the LDS) returns 0 and nothing is launched.  The limits:
+// the block and the partials in 160 KB of LDS; at rank 32 the V operands of four units no longer fit the
+// registers beside the quantisation; at rank 0 the slab pass (k_quant_slab) is a single pass already and
+// the faster one, but takes even unit counts only.  ROT: the shapes the slab passes rotate.
+template <int BITS, int G, int R, bool ROT>
+static int encode_any_dispatch(const lrq_tensors* t, const void* x, int64_t ldx, hipStream_t s, int* status) {
+  if constexpr (!((BITS == 4 && G == 64) || (BITS == 8 && G == 128)) || (R == 0 && (ROT || BITS == 8))) {
+    return 0;
+  } else {
+    const int64_t U = t->hidden / 128;
+    if (t->n_outlier > 0 || U > (R == 32 ? 24 : R == 0 ? 40 : 38)) return 0;
+    if (R == 0 && U % 2 == 0) return 0;
+    if (ROT && (U % 2 != 0 || (t->hidden / (8 / BITS)) % 128 != 0)) return 0;
+    if ((int64_t)16 * t->ld_L * 2 >= ((int64_t)1 << 31) || 32 * ldx >= ((int64_t)1 << 31)) return 0;
+    auto go = [&](auto upw) __attribute__((always_inline)) {
+      constexpr int UPW = decltype(upw)::value;
+      if constexpr (R == 32 && UPW > 3) {
+        return 0;
+      } else {
+        using Ae = AnyEnc<BITS, G, R, UPW>;
+        auto kern = k_encode_any<BITS, G, R, UPW, ROT>;
+        const size_t shm = Ae::bytes((int)U);
+        if (shm > 160 * 1024) return 0;
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess) return 0;
+        const int64_t nrb = (t->rows + 15) / 16;
+        const int64_t slots = (int64_t)cu_count() * Ae::kPerCu;
+        const int rbw = (int)((nrb + slots - 1) / slots);
+        *status = launch(kern, dim3((unsigned)((nrb + rbw - 1) / rbw)), dim3(512), shm, s, (const uint16_t*)x, ldx,
+                         (int)t->rows, (int)t->hidden, (const uint16_t*)t->V, (uint16_t*)t->L, t->ld_L,
+                         (uint8_t*)t->codes, t->ld_codes, (uint16_t*)t->qparams, t->ld_qp, rbw);
+        return 1;
+      }
+    };
+    switch ((U + 7) / 8) {
+      case 1: return go(std::integral_constant<int, 1>{});
+      case 2: return go(std::integral_constant<int, 2>{});
+      case 3: return go(std::integral_constant<int, 3>{});
+      case 4: return go(std::integral_constant<int, 4>{});
+      default: return go(std::integral_constant<int, 5>{});
+    }
+  }
+}
+
 // Column-slab encode (see k_project_slab).  Rank > 0: projection partials, their reduction
 // into L, then the quantisation pass; the slab partials of L live in the codes buffer until
 // the quantisation pass overwrites it (row r's partials take the first nslab*4*R bytes of its
@@ -1506,11 +1716,13 @@ static int encode_impl(const lrq_tensors* t, const void* x, int64_t ldx, hipStre
     // rotated format: the single-pass tile kernel, or the column-slab passes, rotate X in LDS
     // as they read it
     if (!force_twopass && encode_tiles_dispatch<BITS, G, R, true>(t, x, ldx, s, &st)) return st;
+    if (!force_twopass && encode_any_dispatch<BITS, G, R, true>(t, x, ldx, s, &st)) return st;
     if (R > 0 && t->Vt == nullptr) return LRQ_ERR_NULL;
     if (encode_slabs<BITS, G, R, true>(t, x, ldx, s, &st)) return st;
     return LRQ_ERR_UNSUPPORTED;
   }
   if (!force_twopass && encode_persist_dispatch<BITS, G, R>(t, x, ldx, s, &st)) return st;
+  if (!force_twopass && encode_any_dispatch<BITS, G, R, false>(t, x, ldx, s, &st)) return st;
   if (R > 0 && t->Vt == nullptr) return LRQ_ERR_NULL;  // the two-pass projection reads V^T
   return encode_twopass<BITS, G, R>(t, x, ldx, s);
 }
