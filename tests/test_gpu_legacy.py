@@ -190,6 +190,29 @@ def test_legacy_dequant_gemm(pkg, dev, B, M, N, K, bits, n, s_rows):
     assert_fp_close(bits16(out), ref, f"legacy dequant-GEMM {bits}-bit K={K} n={n}")
 
 
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("M,K,n", [(100, 16, 32), (33, 32, 16), (8200, 16, 32), (16400, 32, 32)])  # 1, 1, 2, 4 blocks
+def test_legacy_dequant_gemm_picks_the_decode(pkg, dev, bits, M, K, n):
+    """A y that picks one column per output returns the dense decode's x_hat exactly, also from items
+    whose scales (2^101) or l @ r (about 2^120) take the element-by-element form."""
+    B, N = 1, 1024
+    l, r, x, s = _inputs(7400 + bits, B, M, N, K, 1, outlier_cols=0)
+    s[0, 130], s[0, 131] = 2.0 ** 101, -(2.0 ** 101)
+    l[20, 3], r[3, 700], r[3, 701] = 2.0 ** 60, 2.0 ** 60, -(2.0 ** 61)
+    g = torch.Generator().manual_seed(74)
+    q = torch.randint(0, 256, (B, M, N * bits // 8), generator=g, dtype=torch.uint8).to(dev)
+    cols = torch.randperm(N, generator=g)[:n]
+    cols[:6] = torch.tensor([130, 131, 129, 700, 701, 1023])
+    y = torch.zeros((B, N, n), dtype=torch.bfloat16)
+    y[0, cols, torch.arange(n)] = 1.0
+    args = [t.to(dev) for t in (l, r, s, y)]
+    out = pkg.triton_matmul_decompress(q, args[0], args[1], args[2], args[3], quantize_bit=bits)
+    o = torch.zeros((B, M, N), dtype=torch.bfloat16, device=dev)
+    xh = pkg.low_rank_addition_fuse_decompression_dequantization(args[0], args[1], q, o, args[2], bits, 0.0)
+    assert torch.isfinite(xh).all()
+    assert bool((out == xh[:, :, cols.to(dev)]).all())
+
+
 def test_legacy_dequant_gemm_strided_y_and_empty(pkg, dev):
     """A non-contiguous y (a transposed view) gives the same bits as its contiguous copy, and
     zero rows or zero output columns return empty results."""

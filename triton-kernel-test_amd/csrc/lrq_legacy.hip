@@ -831,7 +831,7 @@ __global__ __launch_bounds__(256) void k_legacy_apply(LegacyArgs a, int RBW, int
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const float sv = bf_lo(srow[unit_base(p, u, N, NP, G) + lane]);
-    s_ok &= fabsf(sv) < 0x1p100f;  // (NaN fails)
+    s_ok &= (__float_as_uint(sv) & 0x7fffffffu) < 0x71800000u;  // |s| < 2^100 (as bits: a NaN is above)
     // bf16(s) | bf16(16 s) << 16: the second term serves the high nibble at 8 bits
     stab[p * 64 + ((lane >> 4) * 4 + (lane & 3)) * 4 + ((lane >> 2) & 3)] = pack_bf16x2(sv, 16.f * sv);
   }
@@ -894,7 +894,10 @@ __global__ __launch_bounds__(256) void k_legacy_apply(LegacyArgs a, int RBW, int
 #pragma unroll
     for (int k = 0; k < RT; ++k) lt = pk_max_u16(lt, pk_max_u16(lop[k][0] & 0x7fff7fffu, lop[k][1] & 0x7fff7fffu));
     const float lmax = __uint_as_float(max(lt & 0xffff0000u, lt << 16));
-    const bool fast = unit_ok && __builtin_amdgcn_ballot_w64(!(lmax * rbound < 0x1p120f) || big) == 0;  // wave-uniform
+    // (as bits: an infinity or a NaN in either is above)
+    const uint32_t lrb = __float_as_uint(lmax * rbound) & 0x7fffffffu;
+    const bool lr_big = lrb >= 0x7b800000u || __float_as_uint(lmax) >= 0x7f800000u || __float_as_uint(rbound) >= 0x7f800000u;
+    const bool fast = unit_ok && __builtin_amdgcn_ballot_w64(lr_big || big) == 0;  // wave-uniform
     __builtin_amdgcn_sched_barrier(0);
     static_for<0, NP>([&](auto pc) {
       constexpr int p = decltype(pc)::value;
@@ -1351,109 +1354,185 @@ struct LegacyGemmArgs {
 // workgroups of 8 waves; a workgroup owns RB 16-row blocks of one batch.  Work items are
 // (unit, plane) pairs, unit-major, so the waves that run together share a unit's code rows in
 // L2; wave w takes items w, w + 8, ...  An item's operands (rt and y rows of the plane's 64
-// columns in the reconstruction layout, the lane's 16 scales, the RB blocks' code vectors) sit in
-// one of two register slots, loaded while the other item is computed.  Per item the y operands are
-// transposed once (identity MFMA); per row block the reconstruction MFMA gives bf16(l @ r) in the
-// lane's 16 columns, the decode's roundings give x_hat, and x_hat (bf16, exact) is the B operand of
-// the product MFMA.  The 8 waves' partial tiles are then summed through LDS in wave order.
+// columns in the reconstruction layout, the scales, the RB blocks' code vectors) sit in
+// one of two register slots, loaded while the other item is computed (wave-uniform bases and 32-bit lane
+// offsets).  Per item the y operands are transposed once (identity MFMA); per row block x_hat is formed on
+// the matrix pipe by diagonal 4x4x4 steps as in k_legacy_apply (the -s (128 + h) term once per item), and
+// x_hat (bf16, exact) is the B operand of the product MFMA.  The 8 waves' partial tiles are then summed
+// through LDS in wave order.
+// An item whose scales or l r could overflow inside a diagonal step (the limits of k_legacy_apply) is
+// formed element by element.
+// Bound by the operands' loads (every CU reads all of y and rt through L2: 512 KB at [4096, 32] each,
+// against 64 KB of codes) and their latency, two waves a SIMD: [4, 4096, 4096] 2 bits @ [4, 4096, 32], K = 32:
+// 32.9 -> 28.8 us.  Of that, x_hat on the matrix pipe (about 2 vector instructions per element for 7) gave
+// 2.7, y as one 16-byte load per lane and row 2.5 (with the scales as vectors and whole-wave addresses).
 template <int BITS, int K, int NOUT, int RB>
 __global__ __launch_bounds__(512) void k_legacy_gemm(LegacyGemmArgs a) {
   constexpr int NP = 8 / BITS, G = 64, E = 16, RT = K / 16, TO = NOUT / 16, NW = 8;
-  constexpr uint32_t kMask = BITS == 8 ? 0xffu : (1u << BITS) - 1u;
+  constexpr uint32_t kMask = (BITS == 8 ? 0x0fu : (1u << BITS) - 1u) * 0x01010101u;
+  constexpr int kHalf = 1 << (BITS - 1);
   __shared__ f32x4 part[NW][TO][64];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
   const int M = (int)a.M, N = (int)a.N;
   const int nrb = (M + 15) / 16, gx = (nrb + RB - 1) / RB;
-  const int b = blockIdx.x / gx;
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / gx);
   const int rb0 = (blockIdx.x - b * gx) * RB;
   const int nu = N / NP / G, ni = nu * NP;
   const int64_t NB = N / NP;
   const uint16_t* srow = a.s + (a.s_rows == 1 ? 0 : (int64_t)b * N);
   const uint16_t* yb = a.y + (int64_t)b * N * a.ldy;
-  const uint8_t* qb = a.q + (int64_t)b * M * NB;
+  const uint8_t* qb = a.q + ((int64_t)b * M + rb0 * 16) * NB;  // the workgroup's first code row
   const u32x2 ident = identity_bop(j, g);
-  const float zero[E] = {};
+  const u32x2 ida = diag4_aop(lane, 0x3f80u), dmask = diag4_aop(lane, 0xffffu);
+  const uint32_t koff = pack_bf16x2_exact(-(float)(BITS == 8 ? 2304 : 128 + kHalf), -(float)(BITS == 8 ? 2304 : 128 + kHalf));
 
   f32x4 acc[RB][TO];
   u32x2 lop[RB][RT];
+  uint32_t qoff[RB];  // the lane's code rows
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
-    const int64_t row = min(min(rb0 + i, nrb - 1) * 16 + j, M - 1);
+    const int row = min(min(rb0 + i, nrb - 1) * 16 + j, M - 1);
+    qoff[i] = (uint32_t)(row - rb0 * 16) * (uint32_t)NB + (uint32_t)(E * g);
 #pragma unroll
     for (int t = 0; t < TO; ++t) acc[i][t] = zero4();
 #pragma unroll
-    for (int t = 0; t < RT; ++t) lop[i][t] = ld8(a.l + row * K + 16 * t + 4 * g);
+    for (int t = 0; t < RT; ++t) lop[i][t] = ld8(a.l + (int64_t)row * K + 16 * t + 4 * g);
   }
+  // byte offsets of the lane's rt and y rows (row q of the layout is 4 q rows on)
+  const uint32_t voff = (uint32_t)(2 * (vrow_res<G>(0, j, 0) * K + 4 * g));
+  const uint32_t ldy2 = 2u * (uint32_t)a.ldy, yoff = (uint32_t)vrow_res<G>(0, j, 0) * ldy2 + (uint32_t)(8 * TO * g);
+  const uint32_t soff = (uint32_t)(2 * E * g);
   struct Item {
-    u32x2 vop[G / 16][RT];  // rt rows of the item's columns (reconstruction A operand)
-    u32x2 ya[G / 16][TO];   // y rows of the item's columns, same layout
-    u32x4 sc[2];            // the lane's 16 scales (bf16)
     u32x4 cb[RB];           // the lane's 16 code bytes of each row block
+    u32x2 ya[G / 16][TO];   // y rows of the item's columns (reconstruction layout): columns 4 TO g .. + 4 TO - 1
+    u32x2 vop[G / 16][RT];  // rt rows of the item's columns (reconstruction A operand)
+    u32x4 sw[2];            // the lane's 16 scales (bf16)
   };
   auto load_item = [&](int it, Item& d) __attribute__((always_inline)) {
     const int u = it / NP, p = it % NP;
     const int base = unit_base(p, u, N, NP, G);
-    load_vops<G, K>(a.rt, base, j, g, d.vop);
+    const uint8_t* qu = qb + u * G;
+    const unsigned char* yu = reinterpret_cast<const unsigned char*>(yb + (int64_t)base * a.ldy);
+    const unsigned char* vu = reinterpret_cast<const unsigned char*>(a.rt + (int64_t)base * K);
+    const unsigned char* su = reinterpret_cast<const unsigned char*>(srow + base);
+#pragma unroll
+    for (int i = 0; i < RB; ++i) d.cb[i] = ld16_stream(qu + qoff[i]);
 #pragma unroll
     for (int q = 0; q < G / 16; ++q)
 #pragma unroll
-      for (int t = 0; t < TO; ++t) d.ya[q][t] = ld8(yb + (int64_t)vrow_res<G>(base, j, q) * a.ldy + 16 * t + 4 * g);
-    d.sc[0] = ld16(srow + base + E * g);
-    d.sc[1] = ld16(srow + base + E * g + 8);
+      for (int t = 0; t < TO; ++t) d.ya[q][t] = ld8(yu + (yoff + (uint32_t)(4 * q) * ldy2) + 8 * t);
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
-      const int64_t row = min(min(rb0 + i, nrb - 1) * 16 + j, M - 1);
-      d.cb[i] = ld16_stream(qb + row * NB + u * G + E * g);
-    }
+    for (int q = 0; q < G / 16; ++q)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) d.vop[q][t] = ld8(vu + voff + (8 * q * K + 32 * t));
+    d.sw[0] = ld16(su + soff);
+    d.sw[1] = ld16(su + soff + 16);
   };
-  // x_hat = bf16(a + bf16(l @ r)) with a = bf16((code - 2^(b-1)) * s), as legacy_value, two columns
-  // at a time: (code - 2^(b-1)) * s is fma(code, s, -2^(b-1) s), exact in fp32 (an integer of at
-  // most 8 bits times a bf16), and already a bf16 value for 1 and 2 bits (|code - 2^(b-1)| <= 2);
-  // each bf16 rounding is one v_cvt_pk_bf16_f32 (round to nearest even, as bf16r) per pair, and
-  // the last one leaves the pair packed as the product's operand.
-  auto compute_item = [&](const Item& d, int p) __attribute__((always_inline)) {
-    u32x4 yt[G / 32][TO];
-    transpose_vops<G, NOUT>(d.ya, ident, yt);
-    float sc[E], zb[E];
-    unpack8(d.sc[0], sc);
-    unpack8(d.sc[1], sc + 8);
-#pragma unroll
-    for (int e = 0; e < E; ++e) zb[e] = -(float)(1 << (BITS - 1)) * sc[e];
-    const int sh = BITS * p;
-#pragma unroll
-    for (int i = 0; i < RB; ++i) {
-      float lr[E];
-      residual_unit<G, K>(d.vop, lop[i], zero, lr);
-      u32x4 xb[G / 32];
-#pragma unroll
-      for (int e = 0; e < E; e += 2) {
-        const uint32_t lp = pack_bf16x2(lr[e], lr[e + 1]);  // bf16(l @ r) of both columns
-        float av[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const uint32_t code = (d.cb[i][(e + h) >> 2] >> (8 * ((e + h) & 3) + sh)) & kMask;
-          av[h] = __builtin_fmaf((float)code, sc[e + h], zb[e + h]);
-        }
-        if constexpr (BITS > 2) {
-          const uint32_t ap = pack_bf16x2(av[0], av[1]);
-          av[0] = bf_lo(ap);
-          av[1] = bf_hi(ap);
-        }
-        xb[e / 8][(e / 2) % 4] = pack_bf16x2(av[0] + bf_lo(lp), av[1] + bf_hi(lp));
-      }
-      project_unit_vt<G, NOUT>(yt, xb, acc[i]);
-    }
-  };
-  // Items w, w + NW, ... through the two slots.  The loop body has no condition (a compute under
-  // a branch made the compiler wait for every outstanding load, the other slot's included, at the
-  // join); an odd last item runs after the loop.  NW is a multiple of NP, so every item of a wave
-  // is in plane w % NP.
-  static_assert(NW % NP == 0, "one plane per wave");
-  const int nit = w < ni ? (ni - w + NW - 1) / NW : 0, pw = w % NP;
   Item ring[2];
 #pragma unroll
   for (int sl = 0; sl < 2; ++sl) load_item(min(w + sl * NW, ni - 1), ring[sl]);
+  __builtin_amdgcn_sched_barrier(0);
+  uint32_t ltop = 0;  // the largest |l| of the workgroup's rows (bf16 bits)
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+      ltop = pk_max_u16(pk_max_u16(ltop, lop[i][t][0] & 0x7fff7fffu), lop[i][t][1] & 0x7fff7fffu);
+  uint32_t lmax = max(ltop >> 16, ltop & 0xffffu);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) lmax = max(lmax, (uint32_t)__shfl_xor((int)lmax, d));
+  const float lbound = (float)K * __uint_as_float(lmax << 16);  // infinite or NaN when an operand is
+  auto compute_item = [&](const Item& d, int p) __attribute__((always_inline)) {
+    // (the scales are the item's last loads: every load of the item has landed before the branch)
+    uint32_t rtop = 0, stop = 0, sc[4];  // sc: the scales of columns 4q + j % 4 / 2 * 2 and the next
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      sc[q] = (j & 2) ? d.sw[q >> 1][2 * (q & 1) + 1] : d.sw[q >> 1][2 * (q & 1)];
+      stop = pk_max_u16(stop, sc[q] & 0x7fff7fffu);
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        rtop = pk_max_u16(pk_max_u16(rtop, d.vop[q][t][0] & 0x7fff7fffu), d.vop[q][t][1] & 0x7fff7fffu);
+    }
+    // |s| < 2^100 and K max |l| |r| < 2^120, as bits (a NaN or an infinity is above)
+    const float rmax = __uint_as_float(max(rtop & 0xffff0000u, rtop << 16));
+    const bool big = max(stop & 0xffff0000u, stop << 16) >= 0x71800000u || __float_as_uint(rmax) >= 0x7f800000u ||
+                     __float_as_uint(lbound) >= 0x7f800000u ||
+                     (__float_as_uint(lbound * rmax) & 0x7fffffffu) >= 0x7b800000u;
+    const bool fast = __builtin_amdgcn_ballot_w64(big) == 0;  // wave-uniform
+    u32x4 yt[G / 32][TO];
+    transpose_vops<G, NOUT>(d.ya, ident, yt);
+    if (fast) {
+      u32x2 sa[4], sb[4];
+      f32x4 off[4];  // -(128 + h) s
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        sa[q] = u32x2{sc[q] & dmask[0], sc[q] & dmask[1]};
+        if constexpr (BITS == 8) {  // 16 s for the codes' high nibbles
+          const uint32_t s16 = pack_bf16x2(16.f * bf_lo(sc[q]), 16.f * bf_hi(sc[q]));
+          sb[q] = u32x2{s16 & dmask[0], s16 & dmask[1]};
+        }
+        off[q] = mfma_4x4x4(sa[q], u32x2{koff, koff}, zero4());
+      }
+      auto rounded = [&](f32x4 v) __attribute__((always_inline)) {
+        return u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      };
+      auto code_op = [&](uint32_t m) __attribute__((always_inline)) {  // 128 + code as bf16 (bytes code, 0x43)
+        return u32x2{__builtin_amdgcn_perm(0x43434343u, m, 0x04010400u), __builtin_amdgcn_perm(0x43434343u, m, 0x04030402u)};
+      };
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        f32x4 tl[4], tv[4];
+        legacy_lowrank_mfma<K>(d.vop, lop[i], tl);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t c = d.cb[i][q];
+          tv[q] = mfma_4x4x4(sa[q], code_op(BITS == 8 ? c & kMask : (c >> (BITS * p)) & kMask), off[q]);
+          if constexpr (BITS == 8) tv[q] = mfma_4x4x4(sb[q], code_op((c >> 4) & kMask), tv[q]);
+        }
+        if constexpr (BITS > 2) {  // (already a bf16 value at 1 and 2 bits)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) tv[q] = mfma_4x4x4(ida, rounded(tv[q]), zero4());
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) tv[q] = mfma_4x4x4(ida, rounded(tl[q]), tv[q]);
+        u32x4 xb[G / 32];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x2 r = rounded(tv[q]);
+          xb[q >> 1][2 * (q & 1)] = r[0];
+          xb[q >> 1][2 * (q & 1) + 1] = r[1];
+        }
+        project_unit_vt<G, NOUT>(yt, xb, acc[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        f32x4 tl[4];
+        legacy_lowrank_mfma<K>(d.vop, lop[i], tl);
+        u32x4 xb[G / 32];
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+          float v[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint32_t code = (d.cb[i][(e + h) >> 2] >> (8 * ((e + h) & 3) + BITS * p)) & ((1u << BITS) - 1u);
+            const uint32_t sw = d.sw[e >> 3][(e >> 1) & 3];
+            const float sv = h ? bf_hi(sw) : bf_lo(sw);
+            v[h] = legacy_value<BITS, false>(code, sv, 0.f, bf16r(tl[e >> 2][(e + h) & 3]));
+          }
+          xb[e / 8][(e / 2) % 4] = pack_bf16x2_exact(v[0], v[1]);
+        }
+        project_unit_vt<G, NOUT>(yt, xb, acc[i]);
+      }
+    }
+  };
+  // Items w, w + NW, ... through the two slots.  The loop body requests and computes unconditionally (an
+  // item's loads that land under a branch make the compiler wait for every outstanding load, the other
+  // slot's included, at the join); an odd last item runs after the loop.  NW is a multiple of NP, so every item of a wave
+  // is in plane w % NP.
+  static_assert(NW % NP == 0, "one plane per wave");
+  const int nit = w < ni ? (ni - w + NW - 1) / NW : 0, pw = w % NP;
   int i0 = 0;
   for (; i0 + 1 < nit; i0 += 2) {
     compute_item(ring[0], pw);
@@ -1467,7 +1546,7 @@ __global__ __launch_bounds__(512) void k_legacy_gemm(LegacyGemmArgs a) {
   }
   if (i0 < nit) compute_item(ring[0], pw);  // wave-uniform
 
-  // acc[i][t] in lane (j, g), component v: out[row j][16t + 4g + v] (partial over this wave's items)
+  // acc[i][t] in lane (j, g), component v: out[row j][4 TO g + 4t + v] (partial over this wave's items)
   constexpr int F = TO * 256 / NW, S = 64 / F, PPL = NW / S;
   static_assert(F >= 1 && F <= 64 && 64 % F == 0 && NW % S == 0, "out reduction split");
   const float* partf = reinterpret_cast<const float*>(&part[0][0][0]);
@@ -1487,7 +1566,7 @@ __global__ __launch_bounds__(512) void k_legacy_gemm(LegacyGemmArgs a) {
 #pragma unroll
     for (int m = F; m < 64; m <<= 1) s += __shfl_xor(s, m);
     const int row = (rb0 + i) * 16 + (src & 15);
-    const int col = 16 * t + 4 * (src >> 4) + v;
+    const int col = 4 * TO * (src >> 4) + 4 * t + v;
     if (pg == 0 && row < M) ob[(int64_t)row * a.ldo + col] = (uint16_t)pack_bf16x2(s, 0.f);
     __syncthreads();
   }
@@ -1880,7 +1959,8 @@ extern "C" int lrq_legacy_dequant_gemm(const void* l, const void* rt, int32_t K,
   a.s_rows = s_rows, a.y = (const uint16_t*)y, a.ldy = ldy, a.out = (uint16_t*)out, a.ldo = ldo, a.M = M, a.N = N;
   a.n_out = n_out;
   const int64_t NB = N / (8 / bits);
-  const bool mfma_ok = vec_ok({l, rt, q, s}) && NB % 64 == 0 && n_out % 16 == 0 && aligned(y, 8) && ldy % 4 == 0;
+  const bool mfma_ok = vec_ok({l, rt, q, s}) && NB % 64 == 0 && n_out % 16 == 0 && aligned(y, 8) && ldy % 4 == 0 &&
+                       NB <= (int64_t)1 << 24 && ldy <= (int64_t)1 << 23;  // (32-bit lane offsets)
   hipStream_t hs = (hipStream_t)stream;
   switch (bits) {
     case 1: return legacy_gemm_bits<1>(a, K, B, mfma_ok, hs);
