@@ -1364,8 +1364,8 @@ struct LegacyGemmArgs {
 // formed element by element.
 // Bound by the operands' loads (every CU reads all of y and rt through L2: 512 KB at [4096, 32] each,
 // against 64 KB of codes) and their latency, two waves a SIMD: [4, 4096, 4096] 2 bits @ [4, 4096, 32], K = 32:
-// 32.9 -> 28.8 us.  Of that, x_hat on the matrix pipe (about 2 vector instructions per element for 7) gave
-// 2.7, y as one 16-byte load per lane and row 2.5 (with the scales as vectors and whole-wave addresses).
+// 32.9 -> 28.8 us, a call 36.9 -> 31.7: x_hat on the matrix pipe (about 2 vector instructions per element for
+// 7) with wave-uniform address bases gave 2.7 of that, y and the scales as 16-byte loads 2.5.
 template <int BITS, int K, int NOUT, int RB>
 __global__ __launch_bounds__(512) void k_legacy_gemm(LegacyGemmArgs a) {
   constexpr int NP = 8 / BITS, G = 64, E = 16, RT = K / 16, TO = NOUT / 16, NW = 8;
