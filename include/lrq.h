@@ -75,8 +75,9 @@ typedef struct lrq_tensors {
   void* L;
   int64_t ld_L;
   const void* V;  /* bf16 [hidden, rank] */
-  const void* Vt; /* bf16 [rank, hidden]; read only by the two-pass encode (rank 32 and hidden
-                     sizes without a single-pass kernel); lrq_transpose_bf16 builds it */
+  const void* Vt; /* bf16 [rank, hidden]; read only by an encode whose width or rank has no kernel
+                     of its own (other than rank 16 and 8, 16, 32 or 40 units of 128
+                     elements, roughly); lrq_transpose_bf16 builds it */
   void* codes;
   int64_t ld_codes;
   void* qparams;  /* fp16 [rows, U, NP, 2], see above */

@@ -91,7 +91,7 @@ def test_encode_decode_formats(pkg, dev, rows, hidden, rank, bits, group):
     (9000, 384, 16, 4, 64),    # several row blocks per workgroup, two workgroups per CU
     (5003, 3072, 16, 4, 64),   # 24 units, ragged rows
     (64, 3072, 32, 4, 64),     # the widest at rank 32
-    (47, 4864, 16, 4, 64),     # 38 units: the widest
+    (47, 4864, 16, 4, 64),     # 38 units
     (4100, 2176, 16, 4, 64),   # 17 units: plane 1 starts in the middle of a tile
     (50, 1152, 0, 4, 64),      # rank 0, odd
     (70, 4992, 0, 4, 64),      # rank 0, 39 units
@@ -105,6 +105,27 @@ def test_encode_any_width(pkg, dev, rows, hidden, rank, bits, group):
     x = pkg.inputs.activation(rows, hidden, n_outlier=2, outlier_scale=20.0, seed=rows + hidden)
     V = pkg.inputs.basis(hidden, rank, seed=9) if rank else None
     _check_encode(pkg, dev, x, V, bits, group)
+
+
+@pytest.mark.parametrize("hadamard", [False, True])
+@pytest.mark.parametrize("rows,hidden,rank,bits,group", [
+    # even unit counts: one chain, fewer and as many chains as waves, more (V^T registers and LDS), V^T from L2
+    (1, 256, 16, 4, 64), (9000, 768, 16, 4, 64), (700, 2304, 16, 4, 64), (5003, 3072, 16, 4, 64), (33, 3328, 16, 4, 64),
+    (4100, 3584, 16, 4, 64), (33, 3840, 16, 4, 64), (300, 512, 32, 4, 64), (4500, 1536, 32, 4, 64), (40, 2304, 32, 4, 64),
+    (4200, 1280, 16, 8, 128), (50, 2816, 16, 8, 128), (130, 3584, 16, 8, 128),
+    # odd ones: one unit, one to three batches of steps, V^T from L2; a few row blocks and many
+    (33, 128, 16, 4, 64), (5003, 1152, 16, 4, 64), (200, 2944, 16, 4, 64), (4100, 3968, 16, 4, 64), (150, 4736, 16, 4, 64),
+    (40, 896, 32, 4, 64), (150, 1920, 32, 4, 64), (4200, 1152, 32, 4, 64), (5003, 1152, 0, 4, 64), (2200, 3712, 0, 4, 64),
+])
+def test_encode_any_width_is_the_two_pass_encode(pkg, dev, rows, hidden, rank, bits, group, hadamard):
+    """The single pass gives the bits of the passes that it takes the place of: the same L (products
+    summed in the same chains and order), codes, scales and zeros."""
+    x = pkg.inputs.activation(rows, hidden, n_outlier=2, outlier_scale=20.0, seed=rows + hidden).to(dev)
+    V = pkg.inputs.basis(hidden, rank, seed=9).to(dev) if rank else None
+    a = pkg.encode(x, V, bits=bits, group_size=group, hadamard=hadamard)
+    b = pkg.encode(x, V, bits=bits, group_size=group, hadamard=hadamard, _twopass=True)
+    assert torch.equal(a.codes, b.codes) and torch.equal(a.qparams, b.qparams)
+    assert rank == 0 or torch.equal(a.L, b.L)
 
 
 @pytest.mark.parametrize("rows,hidden,rank,bits,group", [(50, 2304, 16, 4, 64), (4100, 3584, 16, 4, 64), (33, 1536, 32, 4, 64),

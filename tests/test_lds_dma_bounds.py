@@ -273,32 +273,66 @@ def test_wht_rows_direct_loads_stay_in_bounds(cus):
 
 
 # ----------------------------------------------------------------------------- k_encode_any
-def encode_any_replay(M, N, ldx, cus, bits, per_cu):
-    """k_encode_any as encode_any_dispatch() launches it, and the read-back of every unit's columns."""
-    TILE, NP, U = 4096, 8 // bits, N // 128
-    alloc = U * TILE
+def encode_any_replay(M, N, ldx, cus, bits, rank):
+    """k_encode_any as encode_any_dispatch() launches it: X's and V^T's tiles, and the read-back of every
+    unit's columns and of every projection step's operands (which cover the columns in the chains of the
+    two-pass encode)."""
+    TILE, NP, U, NW = 4096, 8 // bits, N // 128, 8
+    even, upw, RT = U % 2 == 0, (U + 7) // 8, max(1, rank // 16)
+    nch = 0 if rank == 0 else U // 2 if even else 4
+    QR = 8 if (upw == 3 if rank == 16 else rank == 32 and upw == 2) else 0
+    vlds = rank > 0 and (upw <= 2 or (rank == 16 and upw == 3))
+    t0 = 0 if QR == 0 else 16 if even else QR
+    nv = max(0, U - t0) * RT if vlds else 0
+    vbase = U * TILE + nch * RT * 1024
+    alloc = vbase + nv * TILE
+    assert alloc <= LDS_BYTES and nv >= 0
     nrb = (M + 15) // 16
-    rbw, grid = _rows_per_wg(nrb, cus * per_cu)
+    rbw, grid = _rows_per_wg(nrb, cus * (2 if upw == 1 and rank <= 16 else 1))
     lane = np.arange(64)
     lr, lq, j, g = lane >> 4, lane & 15, lane & 15, lane >> 4
     checked = 0
+    # V^T tiles: chunk held at each (tile, rank row, position)
+    vheld = np.full((max(nv, 1), 16, 16), -1, dtype=np.int64)
+    for v in range(nv):
+        for k in range(4):
+            r = 4 * k + lr
+            src = (v % RT) * 16 * N * 2 + 256 * (t0 + v // RT) + (r * N + 8 * (lq ^ r)) * 2
+            dst = vbase + v * TILE + 1024 * k + 16 * lane
+            _check(src, dst, gbytes=rank * N * 2, lds_alloc=alloc, lo=vbase + v * TILE, hi=vbase + (v + 1) * TILE,
+                   what=f"k_encode_any V^T {N} rank {rank}")
+            vheld[v, r, lq] = src % (2 * N) // 16  # 16-byte chunk of the V^T row
+    # the projection: wave w's steps in order; the chains cover every 32 columns once, as the two passes do
+    chains = {}
+    for w in range(NW):
+        nq = 0 if w >= nch else (nch - w + NW - 1) // NW * 8 if even else U
+        for q in range(nq):
+            col = 256 * (w + NW * (q >> 3)) + 32 * (q & 7) if even else 32 * w + 128 * q
+            chains.setdefault(w + 8 * (q >> 3) if even else w, []).append(col)
+            c = col >> 5
+            if vlds and q >= QR:
+                for t in range(RT):
+                    v = ((c >> 2) - t0) * RT + t
+                    assert (vheld[v, j, (4 * (c & 3) + g) ^ j] == (col + 8 * g) // 8).all()
+    if rank:
+        want = {c: [256 * c + 32 * k for k in range(8)] for c in range(U // 2)} if even else \
+            {c: [32 * k for k in range(c, 4 * U, 4)] for c in range(4)}
+        assert chains == want
     for rbs in _blocks(grid, rbw, nrb):
         for rb in rbs:
             lim = M - 1 - rb * 16
-            where = {}  # (tile, row, position) -> chunk of the row
+            held = np.full((U, 16, 16), -1, dtype=np.int64)  # (tile, row, position) -> chunk of the row
             dsts = []
-            for w in range(8):
-                for t in range(w, U, 8):
-                    for k in range(4):
-                        r = 4 * k + lr
-                        gsrc = (rb * 16 * ldx) * 2 + 256 * t + np.minimum(r, lim) * ldx * 2 + 16 * (lq ^ r)
-                        ldst = t * TILE + 1024 * k + 16 * lane
-                        _check(gsrc, ldst, gbytes=((M - 1) * ldx + N) * 2, lds_alloc=alloc, lo=t * TILE, hi=(t + 1) * TILE,
-                               what=f"k_encode_any {M}x{N}")
-                        dsts.append(ldst)
-                        checked += 64
-                        for ll in range(0, 64, 7):
-                            where[(t, int(r[ll]), int(lq[ll]))] = int(lq[ll] ^ r[ll])
+            for t in range(U):
+                for k in range(4):
+                    r = 4 * k + lr
+                    gsrc = (rb * 16 * ldx) * 2 + 256 * t + np.minimum(r, lim) * ldx * 2 + 16 * (lq ^ r)
+                    ldst = t * TILE + 1024 * k + 16 * lane
+                    _check(gsrc, ldst, gbytes=((M - 1) * ldx + N) * 2, lds_alloc=alloc, lo=t * TILE, hi=(t + 1) * TILE,
+                           what=f"k_encode_any {M}x{N}")
+                    dsts.append(ldst)
+                    checked += 64
+                    held[t, r, lq] = (gsrc - np.minimum(rb * 16 + r, M - 1) * ldx * 2) // 16
             d = np.concatenate(dsts)
             assert np.unique(d).size == d.size
             for u in range(U):
@@ -306,13 +340,10 @@ def encode_any_replay(M, N, ldx, cus, bits, per_cu):
                     c = p * U + u if NP == 2 else 2 * u
                     for k in range(4 // NP):
                         chunk = 8 * (c & 1) + (4 // NP) * g + k
-                        col = 128 * (c // 2) + 8 * chunk
                         want = p * (N // NP) + u * (128 // NP) + (32 // NP) * g + 8 * k
-                        assert (col == want).all()
-                        for ll in range(0, 64, 5):
-                            key = (c // 2, int(j[ll]), int(chunk[ll] ^ j[ll]))
-                            if key in where:
-                                assert where[key] == chunk[ll]
+                        assert (held[c // 2, j, chunk ^ j] == want // 8).all()
+            for c in range(4 * U if rank else 0):  # a projection step's 32 columns
+                assert (held[c >> 2, j, (4 * (c & 3) + g) ^ j] == (32 * c + 8 * g) // 8).all()
     return checked
 
 
@@ -320,8 +351,10 @@ def encode_any_replay(M, N, ldx, cus, bits, per_cu):
 @pytest.mark.parametrize("cus", CU_COUNTS)
 def test_encode_any_direct_loads_stay_in_bounds(cus, bits):
     n = 0
-    for M, N, extra, per in [(1, 128, 0, 2), (33, 896, 8, 2), (40, 1152, 0, 1), (100, 3072, 0, 1), (47, 4864, 0, 1)]:
-        n += encode_any_replay(M, N, N + extra, cus, bits, per)
+    for M, N, extra, rank in [(1, 128, 0, 16), (33, 896, 8, 16), (40, 1152, 0, 32), (33, 1024, 0, 32), (40, 2048, 0, 32),
+                              (40, 1920, 0, 32), (100, 3072, 0, 16), (20, 2944, 0, 16), (33, 2048, 0, 16), (47, 3584, 0, 16),
+                              (47, 4736, 0, 16), (50, 4992, 0, 0)]:
+        n += encode_any_replay(M, N, N + extra, cus, bits, rank)
     assert n > 0
 
 

@@ -11,9 +11,13 @@
 //     through LDS; each wave sums a 1/NW slice of the tile and writes it as bf16, and every
 //     wave reads back its rows of L (two barriers per row block, neither of which waits for
 //     the prefetch).
-//   * k_project + k_quant — two passes for other shapes (rank 32, hidden sizes without a
-//     persistent instantiation); X is read twice.  k_quant alone is the whole rank-0 encode
-//     (with optional outlier channels).
+//   * k_encode_rows, k_encode_tiles — the same for rows of 16, 32 or 40 units, streamed
+//     through LDS.
+//   * k_encode_any — one pass for the other widths whose 16-row block fits the LDS, with the
+//     two-pass encode's L bit for bit.
+//   * k_project_slab + k_reduce_slabs + k_quant_slab, k_project + k_quant — two passes for what
+//     is left; X is read twice.  k_quant_slab or k_quant alone is the rank-0 encode (with
+//     optional outlier channels).
 #include "lrq_common.h"
 #include "lrq_host.h"
 #include "lrq_quant.h"
@@ -812,33 +816,48 @@ __global__ __launch_bounds__(512) void k_encode_tiles(const uint16_t* __restrict
 }
 
 // -------------------------------------------------------------------------------------
-// Single-pass encode for any width whose 16-row block fits the LDS (int4/g64 and int8/g128 at rank 16 up
-// to 38 units of 128 elements, int4/g64 at rank 32 up to 24 units and, for odd unit counts, at rank 0).
+// Single-pass encode for any width whose 16-row block fits the LDS (the range: encode_any_dispatch).
 //
 // As in k_encode_tiles the block lives in LDS as N/128 tiles of 16 rows x 128 columns (row r's 16-byte
 // chunk c at position c ^ r), wave w loads (and with ROT rotates) tiles w, w + 8, ... and quantises units
 // w, w + 8, ... (a wave has UPW or UPW - 1 of them); unit u of plane p is the 64-column half (p U + u) % 2
 // of tile (p U + u) / 2 at int4, tile u at int8.  Per block: own tiles landed (and rotated) | barrier |
-// the units' columns into registers | barrier | the next block's tiles requested | projection partials,
-// barrier, L summed in wave order | units quantised.  Up to 8 units two workgroups share a CU (one's
-// loads under the other's work).
-// Against the two slab passes and the slab reduction, which read X twice: [5003, 3072] int4 rank 16
-// 10.2 + 4.0 + 11.9 us.
-template <int BITS, int G, int R, int UPW>
+// projection partials, the units' columns into registers | barrier | the next block's tiles requested | L
+// summed | units quantised.  Up to 8 units two workgroups share a CU (one's loads under the other's work).
+//
+// L is the two-pass encode's bit for bit, so that a width's codes do not depend on the path: the same
+// 16x16x32 steps over the same 32 consecutive columns, in the same chains, added in the same order.
+//   even unit counts (k_project_slab, k_reduce_slabs): chain c = the 8 steps of columns 256c .. 256c + 255;
+//     chains 8s .. 8s + 7 added in order are slab s, the slabs are added in order;
+//   odd ones (k_project): chain c < 4 = steps c, c + 4, c + 8, ..., the four added in order.
+// Wave w takes chains w, w + 8, ...  V^T stays on the CU where it fits (AnyEnc): in LDS, as tiles laid out like
+// X's (16 ranks for 16 rows), or with two or more units a wave a wave's first eight steps in registers and
+// the others in LDS; else it comes from L2, eight steps ahead, for every block.  (EVEN: the unit count is
+// even.)
+template <int BITS, int G, int R, int UPW, bool EVEN>
 struct AnyEnc {
-  static constexpr int NW = 8, TILE = 16 * 256, RT = R > 0 ? R / 16 : 1, PART = R > 0 ? NW * RT * 64 * 16 : 0;
+  static constexpr int NW = 8, TILE = 16 * 256, RT = R > 0 ? R / 16 : 1;
   static constexpr int kPerCu = UPW == 1 && R <= 16 ? 2 : 1;  // workgroups per CU (two would spill from two units a wave up)
-  static size_t bytes(int U) { return (size_t)U * TILE + PART; }
+  static constexpr int chains(int U) { return R == 0 ? 0 : EVEN ? U / 2 : 4; }
+  // a wave's first QR projection steps keep their V^T operands in registers; with VLDS the LDS holds the
+  // V^T tiles of the others, vtile0() .. U - 1
+  static constexpr int QR = R > 0 && (R == 16 ? UPW == 3 : UPW == 2) ? 8 : 0;
+  static constexpr bool VLDS = R > 0 && (UPW <= 2 || (R == 16 && UPW == 3));
+  static constexpr int vtile0() { return QR == 0 ? 0 : EVEN ? 2 * NW : QR; }
+  static constexpr size_t part_bytes(int U) { return (size_t)chains(U) * RT * 64 * 16; }
+  static size_t bytes(int U) {
+    return (size_t)U * TILE + part_bytes(U) + (VLDS && U > vtile0() ? (size_t)(U - vtile0()) * RT * TILE : 0);
+  }
   static_assert(G * (8 / BITS) == 128, "a unit is 128 elements of a row");
 };
 
-template <int BITS, int G, int R, int UPW, bool ROT>
-__global__ __launch_bounds__(512, (2 * AnyEnc<BITS, G, R, UPW>::kPerCu)) void k_encode_any(
+template <int BITS, int G, int R, int UPW, bool ROT, bool EVEN>
+__global__ __launch_bounds__(512, (2 * AnyEnc<BITS, G, R, UPW, EVEN>::kPerCu)) void k_encode_any(
     const uint16_t* __restrict__ X, int64_t ldx, int M, int N, const uint16_t* __restrict__ V,
-    uint16_t* __restrict__ Lout, int64_t ldl, uint8_t* __restrict__ codes, int64_t ldc, uint16_t* __restrict__ qparams,
-    int64_t ldq, int RBW) {
-  using Ae = AnyEnc<BITS, G, R, UPW>;
-  constexpr int NP = 8 / BITS, CPG = G / 32, RT = Ae::RT, NW = Ae::NW, TILE = Ae::TILE;
+    const uint16_t* __restrict__ Vt, uint16_t* __restrict__ Lout, int64_t ldl, uint8_t* __restrict__ codes, int64_t ldc,
+    uint16_t* __restrict__ qparams, int64_t ldq, int RBW) {
+  using Ae = AnyEnc<BITS, G, R, UPW, EVEN>;
+  constexpr int NP = 8 / BITS, CPG = G / 32, RT = Ae::RT, NW = Ae::NW, TILE = Ae::TILE, VB = 8, QR = Ae::QR;
   extern __shared__ __attribute__((aligned(16))) unsigned char shm[];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
@@ -847,7 +866,7 @@ __global__ __launch_bounds__(512, (2 * AnyEnc<BITS, G, R, UPW>::kPerCu)) void k_
   if (rb0 >= nrb) return;  // whole workgroup (no barrier reached)
   const int nblk = min(RBW, nrb - rb0);
   const int nl = U <= w ? 0 : (U - w + NW - 1) / NW;  // this wave's tiles and units (wave-uniform): UPW or UPW - 1
-  f32x4* part = reinterpret_cast<f32x4*>(shm + (size_t)U * TILE);  // [NW][RT][64]
+  f32x4* part = reinterpret_cast<f32x4*>(shm + (size_t)U * TILE);  // [chains][RT][64]
 
   // tile i of this wave: rows 4k .. 4k + 3 per load; lane l covers row 4k + l / 16, chunk (l % 16) ^ row,
   // landing at position l % 16 (rows past the end clamp to the last row)
@@ -878,30 +897,129 @@ __global__ __launch_bounds__(512, (2 * AnyEnc<BITS, G, R, UPW>::kPerCu)) void k_
       for (int p = 0; p < NP; ++p)
         if (i < nl) load_vops<G, R>(V, unit_base(p, w + NW * i, N, NP, G), j, g, vop[i][p]);
   }
+  // The wave's nq projection steps, chain after chain; step q's 32 columns start at step_col(q).
+  const int nch = Ae::chains(U);
+  const int nq = w >= nch ? 0 : EVEN ? (nch - w + NW - 1) / NW * 8 : U;  // (uniform)
+  auto step_col = [&](int q) __attribute__((always_inline)) -> int {
+    return EVEN ? 256 * ((nq > 0 ? w : 0) + NW * (q >> 3)) + 32 * (q & 7) : 32 * (w & 3) + 128 * q;
+  };
+  // the lane's part of a step's V^T operand: Vt[16t + j][column + 8g .. +7]
+  auto vt_at = [&](int q, int t, uint32_t off) __attribute__((always_inline)) {
+    return ld16(reinterpret_cast<const unsigned char*>(Vt + step_col(q) + (int64_t)16 * t * N) + off);
+  };
+  u32x4 vr[QR > 0 ? QR : 1][RT];
+  unsigned char* const vl = shm + (size_t)U * TILE + Ae::part_bytes(U);  // V^T tiles [U - vtile0()][RT]
+  if constexpr (R > 0) {
+    if constexpr (Ae::VLDS) {
+      // tiles vtile0() + w, + 8, ..., as issue() loads X's (rank r in the place of row r)
+#pragma unroll 1
+      for (int v = w; v < (U - Ae::vtile0()) * RT; v += NW) {
+        const uint16_t* base = Vt + (int64_t)(v % RT) * 16 * N + 128 * (Ae::vtile0() + v / RT);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int r = 4 * k + lr;
+          ld16_to_lds(base + (uint32_t)(r * N + 8 * (lq ^ r)), vl + (size_t)v * TILE + 1024 * k);
+        }
+      }
+    }
+    const uint32_t off = 2u * (uint32_t)(j * N + 8 * g);
+    // (unconditionally: a wave without a chain loads chain 0's, unused)
+#pragma unroll
+    for (int k = 0; k < QR; ++k)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) vr[k][t] = vt_at(min(k, max(nq - 1, 0)), t, off);
+  }
 
 #pragma unroll 1
   for (int b = 0; b < nblk; ++b) {
     const int rb = __builtin_amdgcn_readfirstlane(rb0 + b);
     const int row = min(rb * 16 + j, M - 1);
-    // Own tiles landed: after their loads this wave issued the previous block's stores (each unit's, and
-    // the L rows'), which need not complete here; memory operations retire in issue order.
+    constexpr bool kL2 = R > 0 && !Ae::VLDS;
+    u32x4 vt[kL2 ? VB : 1][RT];  // the next steps' operands from L2
+    int jj = j;  // (the empty asm hides that the lane's offset is loop-invariant: it would stay live)
+    auto first_vt = [&]() __attribute__((always_inline)) {
+      asm volatile("" : "+v"(jj));
+      if constexpr (kL2) {
+#pragma unroll
+        for (int k = 0; k < VB; ++k)
+#pragma unroll
+          for (int t = 0; t < RT; ++t) vt[k][t] = vt_at(min(QR + k, max(nq - 1, 0)), t, 2u * (uint32_t)(jj * N + 8 * g));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if constexpr (!ROT) first_vt();  // (with ROT after the rotation, which needs the registers)
+    // Own tiles landed: after their loads this wave issued at least the previous block's stores (each
+    // unit's, and the L rows'), which need not complete here; memory operations retire in issue order.
     constexpr int kUnit = quant_unit_stores<G>(), kL = R > 0 ? RT : 0;
-    if (b == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    if (b == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // (V^T's tiles too)
     else if (nl == UPW) __builtin_amdgcn_s_waitcnt(vmcnt_imm(UPW * kUnit + kL));
     else __builtin_amdgcn_s_waitcnt(vmcnt_imm((UPW - 1) * kUnit + kL));
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (ROT) {
-      // the sign operands, formed per block (the empty asm hides that they are loop-invariant, so they
-      // do not stay live across the quantisation)
-      int jj = j;
+      // the sign operands, formed per block (as the offset above)
       asm volatile("" : "+v"(jj));
       u32x4 op[2][2];
       wht_operands_from_pair(wht_sign_dword(jj, g, 0, false, 0), wht_sign_dword(jj, g, 0, false, 1), op);
 #pragma unroll
       for (int i = 0; i < UPW; ++i)
         if (i < nl) wht128_lds_swz(shm + (size_t)(w + NW * i) * TILE + 256 * j, g, j, op);
+      __builtin_amdgcn_sched_barrier(0);
+      first_vt();
     }
-    lds_barrier();  // every tile landed and rotated
+    lds_barrier();  // every tile landed and rotated; every wave has read the previous block's partials
+    if constexpr (R > 0) {
+      f32x4 acc[RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) acc[t] = zero4();
+      auto lane_at = [&](int c) __attribute__((always_inline)) { return 256 * jj + 16 * ((4 * (c & 3) + g) ^ jj); };
+      // steps q0 .. q0 + 7 (those below nq), and the chain's partial at its end
+      auto steps = [&](int q0, const u32x4 (&v)[VB][RT]) __attribute__((always_inline)) {
+        u32x4 xv[VB];
+#pragma unroll
+        for (int k = 0; k < VB; ++k) {
+          const int c = step_col(min(q0 + k, nq - 1)) >> 5;  // 32-column group: quarter c % 4 of tile c / 4
+          xv[k] = *reinterpret_cast<const u32x4*>(shm + (size_t)(c >> 2) * TILE + lane_at(c));
+        }
+#pragma unroll
+        for (int k = 0; k < VB; ++k) {
+          if (EVEN || q0 + k < nq) {  // (uniform)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) acc[t] = mfma_16x16x32(v[k][t], xv[k], acc[t]);
+          }
+        }
+        if (EVEN || q0 + VB >= nq) {
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            part[((EVEN ? w + q0 : w) * RT + t) * 64 + lane] = acc[t];  // (chain w + 8 (q0 / 8))
+            acc[t] = zero4();
+          }
+        }
+      };
+      if constexpr (QR > 0) {
+        if (nq > 0) steps(0, vr);
+      }
+#pragma unroll 1
+      for (int q0 = QR; q0 < nq; q0 += VB) {
+        if constexpr (kL2) {
+          steps(q0, vt);
+          if (q0 + VB < nq) {
+#pragma unroll
+            for (int k = 0; k < VB; ++k)
+#pragma unroll
+              for (int t = 0; t < RT; ++t) vt[k][t] = vt_at(min(q0 + VB + k, nq - 1), t, 2u * (uint32_t)(jj * N + 8 * g));
+          }
+        } else {
+          u32x4 v[VB][RT];
+#pragma unroll
+          for (int k = 0; k < VB; ++k) {
+            const int c = step_col(min(q0 + k, nq - 1)) >> 5;
+#pragma unroll
+            for (int t = 0; t < RT; ++t) v[k][t] = *reinterpret_cast<const u32x4*>(vl + (size_t)(((c >> 2) - Ae::vtile0()) * RT + t) * TILE + lane_at(c));
+          }
+          steps(q0, v);
+        }
+      }
+    }
     u32x4 x[UPW][NP][CPG];
 #pragma unroll
     for (int i = 0; i < UPW; ++i)
@@ -915,44 +1033,36 @@ __global__ __launch_bounds__(512, (2 * AnyEnc<BITS, G, R, UPW>::kPerCu)) void k_
             x[i][p][k] = *reinterpret_cast<const u32x4*>(tr + 16 * ((8 * (c & 1) + CPG * g + k) ^ j));
         }
       }
-    lds_barrier();  // every wave's reads of the block returned: the tiles may be refilled
+    lds_barrier();  // every wave's reads of the block returned (the tiles may be refilled), the partials are written
     if (b + 1 < nblk) issue(rb + 1);
 
     u32x2 lop[RT], lopn[RT];
     if constexpr (R > 0) {
-      f32x4 acc[2][RT];
-#pragma unroll
-      for (int t = 0; t < RT; ++t) acc[0][t] = acc[1][t] = zero4();
-      {
-        int jj = j;  // (as for the rotation's operands)
-        asm volatile("" : "+v"(jj));
-        const u32x2 ident = identity_bop(jj, g);
-#pragma unroll
-        for (int i = 0; i < UPW; ++i)
-#pragma unroll
-          for (int p = 0; p < NP; ++p)
-            if (i < nl) project_unit<G, R>(vop[i][p], x[i][p], ident, acc[(i * NP + p) & 1]);
-      }
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        f32x4 a = acc[0][t];
-        a[0] += acc[1][t][0];
-        a[1] += acc[1][t][1];
-        a[2] += acc[1][t][2];
-        a[3] += acc[1][t][3];
-        part[(w * RT + t) * 64 + lane] = a;
-      }
-      lds_barrier();  // (the next block's partials come two barriers after these are read)
+        f32x4 sum = zero4();
+#pragma unroll 1
+        for (int s = 0; s < nch; s += NW) {
+          f32x4 v = part[(s * RT + t) * 64 + lane];
 #pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        f32x4 sum = part[t * 64 + lane];
-#pragma unroll
-        for (int w2 = 1; w2 < NW; ++w2) {
-          const f32x4 o = part[(w2 * RT + t) * 64 + lane];
-          sum[0] += o[0];
-          sum[1] += o[1];
-          sum[2] += o[2];
-          sum[3] += o[3];
+          for (int w2 = 1; w2 < NW; ++w2) {
+            // (chains past the last are the slab kernel's idle waves: a zero)
+            const f32x4 o = s + w2 < nch ? part[((s + w2) * RT + t) * 64 + lane] : zero4();
+            if (EVEN || w2 < 4) {
+              v[0] += o[0];
+              v[1] += o[1];
+              v[2] += o[2];
+              v[3] += o[3];
+            }
+          }
+          if (s == 0) {
+            sum = v;
+          } else {
+            sum[0] += v[0];
+            sum[1] += v[1];
+            sum[2] += v[2];
+            sum[3] += v[3];
+          }
         }
         // lane (j, g) holds L[row j][16t + 4g + v]
         lop[t] = u32x2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
@@ -1565,47 +1675,86 @@ static int encode_persist_dispatch(const lrq_tensors* t, const void* x, int64_t 
   }
 }
 
+// Whether encode_slabs serves the shape.  ROT: every wave's columns start on a 128-column block of their
+// plane.
+template <int BITS, int G, int R, bool ROT>
+static bool slabs_fit(const lrq_tensors* t) {
+  constexpr int NP = 8 / BITS;
+  const int N = (int)t->hidden;
+  const int units = N / (G * NP);
+  const int nslab = (N + 2047) / 2048;
+  const bool outl = t->n_outlier > 0;
+  if (units % 2 != 0 || N % 32 != 0) return false;
+  if (ROT && ((N / NP) % 128 != 0 || (2 * G) % 128 != 0 || (NP == 2 && G == 128))) return false;
+  if (outl && (t->n_outlier > 32767 || t->side == nullptr || t->outlier_idx == nullptr)) return false;
+  if (NP == 2 ? (t->ld_qp % 8 != 0 || !aligned(t->qparams, 16)) : (t->ld_qp % 4 != 0 || !aligned(t->qparams, 8))) return false;
+  if ((int64_t)16 * t->ld_qp * 2 >= ((int64_t)1 << 31)) return false;
+  if (outl && (int64_t)16 * t->ld_side * 2 >= ((int64_t)1 << 31)) return false;
+  if ((outl ? QuantSlab<BITS, G, R, true>::bytes(N) : QuantSlab<BITS, G, R, false>::bytes(N)) > 160 * 1024) return false;
+  if constexpr (R > 0) {
+    if ((int64_t)nslab * 4 * R > (int64_t)N * BITS / 8 || t->ld_codes % 16 != 0 || !aligned(t->codes, 16)) return false;
+    if (t->ld_L % 4 != 0 || !aligned(t->L, 8)) return false;
+  }
+  return true;
+}
+
 // k_encode_any: about as many workgroups as fit the CUs at once, each walking consecutive row blocks.
-// Where it does not apply (or the device refuses the LDS) returns 0 and nothing is launched.  The limits:
-// the block and the partials in 160 KB of LDS; at rank 32 the V operands of four units no longer fit the
-// registers beside the quantisation; at rank 0 the slab pass (k_quant_slab) is a single pass already and
-// the faster one, but takes even unit counts only.  ROT: the shapes the slab passes rotate.
+// Where it does not apply (or the device refuses the LDS) returns 0 and nothing is launched.  ROT: the
+// shapes the slab passes rotate.  At rank > 0 an even unit count must be one that the slab passes serve (its
+// L is theirs), an odd one has k_project's.  The lines lie where it stops being the faster one (int4, the
+// kernels alone, µs of the two passes / of this; int8 and rotated alike):
+// - even unit counts at rank 16: [16, 3072] 10.3 / 9.1, [5003, 3072] 20.9 / 16.6, [16384, 3072] 49.7 / 35.1;
+//   above 26 units V^T comes from L2: 28 units 10.5 / 10.5 and 55.3 / 49.6, 30 units 10.2 / 11.4 at 16 rows,
+//   rotated 32 units 62.0 / 64.1;
+// - rank 32: 12 units 12.3 / 10.2 and 32.8 / 21.9 (V^T in registers); above 16 units neither registers nor
+//   LDS hold it: [16384, 3072] 55.6 / 64.3;
+// - odd unit counts (k_project reads X in the MFMA layout): [16384, 2944] 63.1 / 34.7, [16384, 4736] 102 / 73.8;
+//   with V^T from L2 (above 24 units), or 4 waves of 9 or more rank-32 steps, one row block a CU alone takes
+//   longer than the passes over all CUs: [128, 4480] 14.4 / 15.7, [256, 4480] 20.0 / 16.0;
+// - rank 0: the slab pass is a single pass already and the faster one, but takes even unit counts only;
+//   against k_quant [16384, 2944] 31.1 / 25.3, [128, 2944] 5.0 / 5.4; [2000, 3968] 6.4 / 7.0,
+//   [5003, 3968] 15.9 / 13.3.
 template <int BITS, int G, int R, bool ROT>
 static int encode_any_dispatch(const lrq_tensors* t, const void* x, int64_t ldx, hipStream_t s, int* status) {
   if constexpr (!((BITS == 4 && G == 64) || (BITS == 8 && G == 128)) || (R == 0 && (ROT || BITS == 8))) {
     return 0;
   } else {
     const int64_t U = t->hidden / 128;
-    if (t->n_outlier > 0 || U > (R == 32 ? 24 : R == 0 ? 40 : 38)) return 0;
-    if (R == 0 && U % 2 == 0) return 0;
-    if (ROT && (U % 2 != 0 || (t->hidden / (8 / BITS)) % 128 != 0)) return 0;
+    const int64_t nrb = (t->rows + 15) / 16;
+    if (t->n_outlier > 0 || U > (R == 32 ? 16 : U % 2 == 0 ? 28 : R == 0 ? 40 : 38)) return 0;
+    if (R == 0 && (U % 2 == 0 || nrb <= (U > 24 ? 128 : 8))) return 0;
+    if (R > 0 && U % 2 != 0 && U > (R == 32 ? 8 : 24) && nrb <= 8) return 0;
+    if (R > 0 && (t->Vt == nullptr || ((ROT || U % 2 == 0) && !slabs_fit<BITS, G, R, ROT>(t)))) return 0;
     if ((int64_t)16 * t->ld_L * 2 >= ((int64_t)1 << 31) || 32 * ldx >= ((int64_t)1 << 31)) return 0;
-    auto go = [&](auto upw) __attribute__((always_inline)) {
+    auto go = [&](auto upw, auto even) __attribute__((always_inline)) {
       constexpr int UPW = decltype(upw)::value;
-      if constexpr (R == 32 && UPW > 3) {
+      constexpr bool EVEN = decltype(even)::value;
+      if constexpr ((R == 32 && UPW > 2) || (EVEN ? R == 0 || UPW > 4 : ROT)) {
         return 0;
       } else {
-        using Ae = AnyEnc<BITS, G, R, UPW>;
-        auto kern = k_encode_any<BITS, G, R, UPW, ROT>;
+        using Ae = AnyEnc<BITS, G, R, UPW, EVEN>;
+        auto kern = k_encode_any<BITS, G, R, UPW, ROT, EVEN>;
         const size_t shm = Ae::bytes((int)U);
         if (shm > 160 * 1024) return 0;
         if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess) return 0;
-        const int64_t nrb = (t->rows + 15) / 16;
         const int64_t slots = (int64_t)cu_count() * Ae::kPerCu;
         const int rbw = (int)((nrb + slots - 1) / slots);
         *status = launch(kern, dim3((unsigned)((nrb + rbw - 1) / rbw)), dim3(512), shm, s, (const uint16_t*)x, ldx,
-                         (int)t->rows, (int)t->hidden, (const uint16_t*)t->V, (uint16_t*)t->L, t->ld_L,
-                         (uint8_t*)t->codes, t->ld_codes, (uint16_t*)t->qparams, t->ld_qp, rbw);
+                         (int)t->rows, (int)t->hidden, (const uint16_t*)t->V, (const uint16_t*)t->Vt, (uint16_t*)t->L,
+                         t->ld_L, (uint8_t*)t->codes, t->ld_codes, (uint16_t*)t->qparams, t->ld_qp, rbw);
         return 1;
       }
     };
-    switch ((U + 7) / 8) {
-      case 1: return go(std::integral_constant<int, 1>{});
-      case 2: return go(std::integral_constant<int, 2>{});
-      case 3: return go(std::integral_constant<int, 3>{});
-      case 4: return go(std::integral_constant<int, 4>{});
-      default: return go(std::integral_constant<int, 5>{});
-    }
+    auto pick = [&](auto even) __attribute__((always_inline)) {
+      switch ((U + 7) / 8) {
+        case 1: return go(std::integral_constant<int, 1>{}, even);
+        case 2: return go(std::integral_constant<int, 2>{}, even);
+        case 3: return go(std::integral_constant<int, 3>{}, even);
+        case 4: return go(std::integral_constant<int, 4>{}, even);
+        default: return go(std::integral_constant<int, 5>{}, even);
+      }
+    };
+    return U % 2 == 0 ? pick(std::true_type{}) : pick(std::false_type{});
   }
 }
 
@@ -1617,25 +1766,16 @@ static int encode_any_dispatch(const lrq_tensors* t, const void* x, int64_t ldx,
 template <int BITS, int G, int R, bool ROT>
 static int encode_slabs(const lrq_tensors* t, const void* x, int64_t ldx, hipStream_t s, int* status) {
   constexpr int NP = 8 / BITS;
+  if (!slabs_fit<BITS, G, R, ROT>(t)) return 0;
   const int M = (int)t->rows, N = (int)t->hidden;
   const int units = N / (G * NP);
   const int nslab = (N + 2047) / 2048;
   const bool outl = t->n_outlier > 0;
-  if (units % 2 != 0 || N % 32 != 0) return 0;
-  // rotated input: every wave's columns start on a 128-column block of their plane
-  if (ROT && ((N / NP) % 128 != 0 || (2 * G) % 128 != 0 || (NP == 2 && G == 128))) return 0;
-  if (outl && (t->n_outlier > 32767 || t->side == nullptr || t->outlier_idx == nullptr)) return 0;
-  if (NP == 2 ? (t->ld_qp % 8 != 0 || !aligned(t->qparams, 16)) : (t->ld_qp % 4 != 0 || !aligned(t->qparams, 8))) return 0;
-  if ((int64_t)16 * t->ld_qp * 2 >= ((int64_t)1 << 31)) return 0;
-  if (outl && (int64_t)16 * t->ld_side * 2 >= ((int64_t)1 << 31)) return 0;
   const size_t shm = outl ? QuantSlab<BITS, G, R, true>::bytes(N) : QuantSlab<BITS, G, R, false>::bytes(N);
-  if (shm > 160 * 1024) return 0;
   const int cus = cu_count();
   const int nrb = (M + 15) / 16;
   if constexpr (R > 0) {
     const int64_t ldp = t->ld_codes;  // bytes
-    if ((int64_t)nslab * 4 * R > (int64_t)N * BITS / 8 || ldp % 16 != 0 || !aligned(t->codes, 16)) return 0;
-    if (t->ld_L % 4 != 0 || !aligned(t->L, 8)) return 0;
     // pass 1: about one workgroup per CU over (row groups, slabs)
     const int per1 = std::max(1, cus / nslab);
     const int rbw1 = (nrb + per1 - 1) / per1;

@@ -76,7 +76,7 @@ static inline int launch(void (*k)(P...), dim3 grid, dim3 block, size_t shm, hip
     if (lrq_try_status_ != LRQ_OK) return lrq_try_status_; \
   } while (0)
 
-// Validates a group-mode descriptor (Vt is checked by the two-pass encode, its only reader).
+// Validates a group-mode descriptor (Vt is checked by the encodes that read it).
 static inline int validate_tensors(const lrq_tensors* t) {
   if (t == nullptr) return LRQ_ERR_NULL;
   if (t->rows < 0 || t->hidden <= 0 || t->rows > INT32_MAX || t->hidden > INT32_MAX) return LRQ_ERR_SHAPE;
