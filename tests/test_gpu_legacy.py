@@ -655,6 +655,29 @@ def test_legacy_encode_non_finite_and_huge(pkg, dev, bits):
         assert np.array_equal(O.bf16_to_f32(og), O.bf16_to_f32(ref_o))
 
 
+@pytest.mark.parametrize("tau", [0.0, -0.0, -1e-42])  # the last rounds to -0 in bf16
+@pytest.mark.parametrize("bits,N", [(1, 512), (2, 1024), (4, 1024), (8, 512), (4, 72)])  # (the last: scalar path)
+def test_legacy_encode_zero_threshold(pkg, dev, bits, N, tau):
+    """A threshold of zero of either sign makes every nonzero residual an outlier, from the dense and the
+    staged encode alike; a residual of exactly zero is none."""
+    B, M, K = 1, 40, 16
+    l, r, x, s = _inputs(300 + bits, B, M, N, K, 1)
+    l[7], x[0, 7, ::3] = 0.0, 0.0
+    o_ref, q_ref = O.legacy_encode(bits16(l), bits16(r), bits16(x), bits16(s), bits, tau)
+    nz = O.bf16_to_f32(o_ref) != 0
+    ld, rd, xd, sd = l.to(dev), r.to(dev), x.to(dev), s.to(dev)
+    oc, q = pkg.legacy_encode_coo(ld, rd, xd, sd, bits, tau, capacity=x.numel())
+    assert int(oc.nnz.item()) == int(nz.sum())
+    assert np.array_equal(q.cpu().numpy(), q_ref)
+    assert np.array_equal(bits16(oc.to_sparse().to_dense())[nz], o_ref[nz])
+    l2, rt, kp = pkg.legacy._factors(ld, rd)
+    o, q = torch.empty_like(xd), torch.empty_like(q)
+    pkg._lib.call("lrq_legacy_encode", l2.data_ptr(), rt.data_ptr(), kp, xd.data_ptr(), B, M, N, M * N, N,
+                  sd.data_ptr(), 1, bits, tau, o.data_ptr(), q.data_ptr(), pkg.api._stream(xd.device))
+    assert np.array_equal(q.cpu().numpy(), q_ref)
+    assert np.array_equal(O.bf16_to_f32(bits16(o)), O.bf16_to_f32(o_ref))
+
+
 # the MFMA decode (k_legacy_apply) where it can go wrong: units that do not fill a group of four, one
 # row, ragged last blocks, several runs; densities below and above the entries requested ahead; every
 # bit width and rank

@@ -171,7 +171,7 @@ __device__ __forceinline__ uint32_t bf16_at(const u32x4& w0, const u32x4& w1, ui
 // value is the one the VALU forms above give.  The bf16 tests and masks are packed 16-bit integer
 // operations (two elements each).  An infinite or NaN x would spread over its 4 elements through the
 // zeros of A, and a residual so large that a r2 overflows would meet a r1's infinity: the wave redoes
-// a plane with such a magnitude (mag_limit) with legacy_code_mfma2.  tau >= 0 here.
+// a plane with such a magnitude (mag_limit) with legacy_code_mfma2.  tau >= +0 here (legacy_tau).
 // (The packed operations are asm: written as vector code the compiler splits a saturated difference
 // and its test into per-half compares and selects.)
 __device__ __forceinline__ uint32_t pk_sub_sat_u16(uint32_t a, uint32_t b) {
@@ -1790,6 +1790,13 @@ static int legacy_bits(const LegacyArgs& a, int K, int64_t B, int bits, bool mfm
   }
 }
 
+// The outlier threshold as the kernels compare with it: rounded to bf16, and -0 (also what a tiny negative
+// threshold rounds to) as +0, which compares alike but whose bits the encode's packed-integer test can take.
+static float legacy_tau(float outlier) {
+  const uint16_t h = bf16_bits_host(outlier);
+  return bf16_value_host(h == 0x8000u ? (uint16_t)0 : h);
+}
+
 // Shape / argument checks common to every legacy entry point.
 static int legacy_check(const void* l, const void* rt, int32_t K, int64_t B, int64_t M, int64_t N, int32_t bits,
                         const void* s, int64_t s_rows, bool need_s) {
@@ -1827,7 +1834,7 @@ extern "C" int lrq_legacy_encode(const void* l, const void* rt, int32_t K, const
   LegacyArgs a{};
   a.l = (const uint16_t*)l, a.rt = (const uint16_t*)rt, a.x = (const uint16_t*)x, a.ldx_b = ldx_b, a.ldx_m = ldx_m;
   a.s = (const uint16_t*)s, a.s_rows = s_rows, a.oout = (uint16_t*)o, a.qout = (uint8_t*)q, a.M = M, a.N = N;
-  a.tau = bf16_value_host(bf16_bits_host(outlier));
+  a.tau = legacy_tau(outlier);
   const bool mfma_ok = vec_ok({l, rt, x, s, o, q}) && ldx_b % 8 == 0 && ldx_m % 8 == 0 && N % 8 == 0;
   return legacy_bits<kEncode, 0>(a, K, B, bits, mfma_ok, (hipStream_t)stream);
 }
@@ -1851,7 +1858,7 @@ extern "C" int lrq_legacy_encode_coo(const void* l, const void* rt, int32_t K, c
   const int NP = 8 / bits;
   const bool mfma_ok = vec_ok({l, rt, x, s, o, q}) && ldx_b % 8 == 0 && ldx_m % 8 == 0 && N % 8 == 0;
   const int64_t NB = N / NP;
-  const float tau = bf16_value_host(bf16_bits_host(outlier));
+  const float tau = legacy_tau(outlier);
   // (with tau >= 0 an element's |xr| > tau is exactly "an entry"; a negative threshold keeps every
   // element but the +-0 ones, counted by the compaction's own pass)
   const bool counted = mfma_ok && NB % 64 == 0 && NB / 64 <= 65535 && B <= 65535 && aligned(o, 16) && tau >= 0.f;
