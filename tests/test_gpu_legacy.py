@@ -678,6 +678,31 @@ def test_legacy_encode_zero_threshold(pkg, dev, bits, N, tau):
     assert np.array_equal(O.bf16_to_f32(bits16(o)), O.bf16_to_f32(o_ref))
 
 
+@pytest.mark.parametrize("bits,K", [(1, 16), (2, 32), (4, 16), (8, 32)])
+def test_legacy_encode_non_finite_scales(pkg, dev, bits, K):
+    """A NaN scale changes no code but its own column's (the encode's matrix steps sum over four columns),
+    and outliers do not depend on the scale; infinite and zero scales give the oracle's codes.  One unit
+    holds a NaN alone, others the other scales, so that none sends the NaN's unit to the element form."""
+    B, M, N, tau = 2, 50, 1024, 5.0
+    NB = N * bits // 8
+    l, r, x, s = _inputs(90 + bits, B, M, N, K, B)
+    r[:, 70] = 0.0
+    x[:, :, 70] = 1.0  # no column's residual is zero where its scale is
+    s[0, 5], s[1, 70] = float("nan"), -float("nan")  # units 0 and 1 of plane 0, one batch each
+    s[0, NB - 1], s[1, NB - 2], s[0, 70] = float("inf"), -float("inf"), 2.0 ** 110
+    if NB > 192:
+        s[1, 130] = 0.0
+    with np.errstate(all="ignore"):
+        o_ref, q_ref = O.legacy_encode(bits16(l), bits16(r), bits16(x), bits16(s), bits, tau)
+    o_sp, q = pkg.low_rank_addition_fuse_compression_quantization(l.to(dev), r.to(dev), x.to(dev), s.to(dev), bits, tau)
+    qg, og = q.cpu().numpy(), bits16(o_sp.to_dense())
+    own = (1 << bits) - 1  # plane 0's bits
+    for b, c in ((0, 5), (1, 70)):
+        q_ref[b, :, c] = (q_ref[b, :, c] & (0xFF ^ own)) | (qg[b, :, c] & own)
+    assert np.array_equal(qg, q_ref)
+    assert np.array_equal(O.bf16_to_f32(og), O.bf16_to_f32(o_ref))
+
+
 # the MFMA decode (k_legacy_apply) where it can go wrong: units that do not fill a group of four, one
 # row, ragged last blocks, several runs; densities below and above the entries requested ahead; every
 # bit width and rank

@@ -285,10 +285,11 @@ __device__ __forceinline__ bool legacy_codes_mfma(uint32_t (&w)[8], uint32_t tau
   return (top >> 16) >= mag_limit || (top & 0xffffu) >= mag_limit;
 }
 
-// Scales whose reciprocal estimate gives legacy_code's codes (NaN fails the test).
+// Scales whose two-term reciprocal gives legacy_code's codes, 2^-100 <= |sc| <= 2^100: compared as bits, so
+// that a NaN is above (this build's float comparisons take no NaN).
 __device__ __forceinline__ bool rc_scale_ok(float sc) {
-  const float m = fabsf(sc);
-  return m >= 0x1p-100f && m <= 0x1p100f;
+  const uint32_t m = __float_as_uint(sc) & 0x7fffffffu;
+  return m >= 0x0d800000u && m <= 0x71800000u;
 }
 
 // Decode of one element: bf16(bf16(bf16((code - 2^(b-1)) * s) + o) + lr); with !HAS_O the add
