@@ -257,7 +257,9 @@ int64_t lrq_coo_workspace(int64_t B, int64_t M, int64_t N);
 /* piece_ptr (as lrq_coo_compact writes it, int64 [B*M*ceil(N/64) + 1]) of a coalesced COO tensor
  * from elsewhere: indices int64 [ndim, n_entries], rows ld_idx apart, the last ndim of (b, m, n) in
  * row-major order (1 <= ndim <= 3; a missing dimension is 0).  Every pointer lies in [0, n_entries]
- * whatever the indices hold; entries outside the tensor belong to no piece. */
+ * whatever the indices hold.  Of entries outside the tensor, a column past N counts in its row's last
+ * piece and a row past M in its batch's last piece, where lrq_legacy_decode_coo skips every column
+ * outside the piece; a batch past B counts in none. */
 int lrq_coo_pieces(const int64_t* indices, int64_t ld_idx, int32_t ndim, int64_t n_entries, int64_t B, int64_t M,
                    int64_t N, int64_t* piece_ptr, void* stream);
 

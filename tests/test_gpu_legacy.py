@@ -597,6 +597,30 @@ def test_coo_pieces_of_a_sparse_tensor(pkg, dev, shape, n):
         assert cnt == n and torch.equal(ptr.cpu(), want) and torch.equal(cols.cpu(), ind[2])
 
 
+@pytest.mark.parametrize("B,M,N,bits", [(1, 2, 64, 8), (2, 40, 512, 2), (2, 33, 70, 8), (1, 50, 1000, 4), (3, 200, 256, 4)])
+@pytest.mark.parametrize("more", [(0, 0, 6), (0, 0, 300), (0, 5, 0), (2, 0, 0), (1, 3, 130), (0, -1, -2)])
+def test_sparse_outliers_of_another_shape(pkg, dev, B, M, N, bits, more):
+    """Sparse outliers with more (or fewer) batches, rows or columns than the activation: the decode reads
+    the entries inside it and no other."""
+    shape = (B + more[0], M + more[1], N + more[2])
+    g = torch.Generator().manual_seed(N + sum(more))
+    o = torch.randn(shape, generator=g) * (torch.rand(shape, generator=g) < 0.1)
+    o[0, 0, :8] = torch.arange(8) + 1.0
+    o[:, -1, -3:] = 7.0
+    o = o.to(torch.bfloat16).to(dev)
+    l, r, s, q, _ = _decode_operands(dev, B, M, N, 16, bits, 0.0, N)
+    inside = torch.zeros((B, M, N), dtype=torch.bfloat16, device=dev)
+    cut = o[:B, :M, :N]
+    inside[:, : cut.shape[1], : cut.shape[2]] = cut
+    dec = pkg.low_rank_addition_fuse_decompression_dequantization
+    want = dec(l, r, q, inside, s, quantize_bit=bits)
+    assert torch.equal(dec(l, r, q, o.to_sparse(), s, quantize_bit=bits), want)
+    if shape[0] == 1 and B == 1:
+        assert torch.equal(dec(l, r, q, o[0].to_sparse(), s, quantize_bit=bits), want)
+    ptr, _, _, n = pkg.legacy._coo_pieces(o.to_sparse(), B, M, N)
+    assert int(ptr[0]) == 0 and int(ptr[-1]) <= n and bool((ptr[1:] >= ptr[:-1]).all())
+
+
 @pytest.mark.parametrize("nd,at,row,value", [(3, 4, 2, 64), (3, 0, 0, -1), (3, 70_000, 1, 500), (3, 9, 2, 0),
                                               (2, 5, 1, 500), (1, 3, 2, 64), (1, 4, 2, -3)])
 def test_sparse_outliers_are_checked(pkg, dev, nd, at, row, value):

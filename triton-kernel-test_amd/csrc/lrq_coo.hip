@@ -550,8 +550,7 @@ __global__ __launch_bounds__(kScatterThreads) void k_coo_scatter_staged(
 // 590 k pieces and 200 k entries it takes the place of a dozen elementwise passes over the
 // indices and a searchsorted per piece (with k_coo_check below, the reference-named encode + decode
 // of [4, 3072, 3072] at 2 bits: 371 -> 156 us a pass).  Bound by the entry reads (24 bytes each) and the
-// 8-byte pointers.  An entry outside [0, B) x [0, M) x [0, N) is counted nowhere, and every pointer lies in
-// [0, n], whatever the indices hold.
+// 8-byte pointers.  Every pointer lies in [0, n], whatever the indices hold.
 constexpr int kPtrChunk = 2048, kPtrThreads = 512;
 
 struct CooIndex {
@@ -561,13 +560,16 @@ struct CooIndex {
   int64_t B, M, N, npc;
 };
 
-// The piece of entry e, -1 when the entry lies outside the tensor.
+// The piece that entry e counts in, in the order of the entries also where they lie outside the tensor (the
+// search and the prefix sums need that): a column past N in its row's last piece, a row past M in its
+// batch's last piece (the readers drop an entry by its column), a batch past B after every piece.
 __device__ __forceinline__ int64_t coo_entry_piece(const CooIndex& c, int64_t e) {
   const int64_t col = c.idx[(c.nd - 1) * c.ld + e];
   const int64_t m = c.nd > 1 ? c.idx[(c.nd - 2) * c.ld + e] : 0;
   const int64_t b = c.nd > 2 ? c.idx[e] : 0;
-  const bool in = (uint64_t)col < (uint64_t)c.N && (uint64_t)m < (uint64_t)c.M && (uint64_t)b < (uint64_t)c.B;
-  return in ? (b * c.M + m) * c.npc + col / kPiece : -1;
+  if (b >= c.B) return c.B * c.M * c.npc;
+  if (m >= c.M) return (max(b, (int64_t)0) + 1) * c.M * c.npc - 1;
+  return (max(b, (int64_t)0) * c.M + max(m, (int64_t)0)) * c.npc + min(max(col, (int64_t)0) / kPiece, c.npc - 1);
 }
 
 __global__ __launch_bounds__(kPtrThreads) void k_coo_pieces(CooIndex c, int64_t npieces, int64_t* __restrict__ piece_ptr) {

@@ -237,7 +237,11 @@ def _coo_pieces(o, B: int, M: int, N: int):
         ind = ind.contiguous()
     ptr = torch.empty((B * M * ((N + 63) // 64) + 1,), dtype=torch.int64, device=ind.device)
     call("lrq_coo_pieces", _p(ind), ind.stride(0), ind.shape[0], ind.shape[1], B, M, N, _p(ptr), _stream(ind.device))
-    return ptr, ind[-1], o.values().to(torch.bfloat16).contiguous(), int(ind.shape[1])
+    cols = ind[-1]
+    if ind.shape[0] > 1 and o.shape[-2] > M:
+        # rows past the decode's (a column past N is skipped by the decode)
+        cols = torch.where(ind[-2] < M, cols, torch.full_like(cols, N))
+    return ptr, cols, o.values().to(torch.bfloat16).contiguous(), int(ind.shape[1])
 
 
 def _encode_coo(l, r, x, s, bits: int, outlier: float, capacity: Optional[int]):
