@@ -8,6 +8,7 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 ROOT = Path(__file__).resolve().parents[1]
 HEADERS = sorted((ROOT / "include").glob("*.h"))
@@ -312,3 +313,17 @@ def test_row_offset_clamp_stays_in_32_bits():
             wrapped = min((r * ld) & mask, ((M - 1 - r0) * ld) & mask) // ld
             if r0 == 0 and r == 15:
                 assert wrapped != want       # the uncapped form fails here
+
+
+def test_sparse_outliers_respect_the_invariant_checks(pkg, monkeypatch):
+    """A program that has torch check sparse invariants gets the check on the outliers' tensor too, also
+    where the device check has passed; without it the tensor is built unchecked."""
+    ind = torch.tensor([[0, 0], [0, 0], [5, 99]])  # column 99 of 64
+    o = pkg.LegacyOutliers(ind, torch.ones(2, dtype=torch.bfloat16), torch.tensor([2]), torch.zeros(2, dtype=torch.int64),
+                           (1, 1, 64))
+    with pytest.raises(RuntimeError):
+        o.to_sparse()  # host tensors: torch checks
+    monkeypatch.setattr(pkg.LegacyOutliers, "_count_valid", lambda self: (2, True))
+    assert o.to_sparse()._nnz() == 2
+    with torch.sparse.check_sparse_tensor_invariants(enable=True), pytest.raises(RuntimeError):
+        o.to_sparse()

@@ -134,11 +134,12 @@ class LegacyOutliers:
 
     def _sparse(self, n: int, valid: Optional[bool]) -> torch.Tensor:
         nd = len(self.shape)
-        # (what _count_valid could not check on the device, torch checks)
+        # (what _count_valid could not check on the device, torch checks; None: as the program has set
+        # torch.sparse.check_sparse_tensor_invariants)
         if valid is False:
             raise RuntimeError("the outlier indices are not a coalesced COO tensor's: outside the shape or out of order")
         return torch.sparse_coo_tensor(self.indices[3 - nd:, :n], self.values[:n], self.shape, is_coalesced=True,
-                                       check_invariants=valid is None)
+                                       check_invariants=True if valid is None else None)
 
     def _overflow(self, n: int):
         raise RuntimeError(f"{n} outliers exceed the capacity {self.capacity}; compact again with a larger one")
