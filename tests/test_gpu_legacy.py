@@ -785,6 +785,42 @@ def test_legacy_apply_non_finite_and_huge(pkg, dev, bits):
     assert same.all()
 
 
+@pytest.mark.parametrize("bits", [1, 2, 8])
+def test_legacy_decode_of_wide_rows(pkg, dev, bits):
+    """Rows of more than 2^20 columns give the dense decode's bits and take the matrix kernels like
+    narrower ones of as many elements (the element-by-element kernels take over twenty times as long)."""
+    dec, silu = pkg.low_rank_addition_fuse_decompression_dequantization, pkg.triton_silu_backward_fuse_extraction
+
+    def operands(M, N):
+        l, r, s, q, o = _decode_operands(dev, 1, M, N, 16, bits, 0.002, bits)
+        return l, r, s, q, o, torch.randn((1, M, N), device=dev).to(torch.bfloat16)
+
+    def best(f):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        times = []
+        for _ in range(5):
+            e[0].record()
+            f()
+            e[1].record()
+            torch.cuda.synchronize()
+            times.append(e[0].elapsed_time(e[1]))
+        return min(times)
+
+    wide, narrow = operands(17, (1 << 21) + 512), operands(17 * 512, 4096 + 512)
+    times = []
+    for l, r, s, q, o, y in (wide, narrow):
+        oc = pkg.compact_outliers(o)
+        x = dec(l, r, q, oc.check(), s, quantize_bit=bits)
+        assert torch.equal(x, dec(l, r, q, o, s, quantize_bit=bits))
+        plain = dec(l, r, q, None, s, quantize_bit=bits)
+        assert torch.equal(plain, dec(l, r, q, torch.zeros_like(o), s, quantize_bit=bits))
+        assert torch.equal(silu(l, r, q, s, y, bits), pkg.triton_silu_backward(plain, y))
+        times.append([best(lambda: dec(l, r, q, oc, s, quantize_bit=bits)), best(lambda: dec(l, r, q, None, s, quantize_bit=bits)),
+                      best(lambda: silu(l, r, q, s, y, bits))])
+    for w, n in zip(*times):
+        assert w < 8 * n, times
+
+
 @pytest.mark.parametrize("bits,K", [(2, 16), (4, 32), (8, 16)])
 def test_legacy_rows_largest_dense_coo(pkg, dev, bits, K):
     """Dense COO outliers at 2^27 elements (the row-tile decode) give the dense decode's bits."""

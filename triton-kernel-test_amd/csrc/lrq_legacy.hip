@@ -688,6 +688,7 @@ struct LegacyApply {
   static constexpr int OFF_TAB = HASY ? RING * SLOT : 0, OFF_OUT = OFF_TAB + TAB, OFF_O = OFF_OUT + SLOT;
   static constexpr int WAVE = OFF_O + (COO ? NP * SLOT : 0);  // bytes per wave
   static constexpr int kStepOps = 4;                          // with y: two loads, two stores per step
+  static constexpr int64_t kWindow = (int64_t)1 << 27;        // entries of a block within reach of its first
   static constexpr int LPP = NREC <= 64 ? 64 / NREC : 1, PPL = NREC <= 64 ? 1 : NREC / 64;
   // entries of a piece per lane and round (2 bits, 16 % outliers: [4, 3072, 3072] 49.7 us at 8, 58.5 at
   // 12, 61.3 at 20)
@@ -761,9 +762,9 @@ __global__ __launch_bounds__(256) void k_legacy_apply(LegacyArgs a, int RBW, int
     }
   };
   // entries s0 + LPP * (SL * round + k) + lane % LPP, k < SL, of the lane's pieces; an entry past the
-  // piece (or 2^24 entries past the block's first) is outside the range and reads as column 0, value 0
+  // piece (or kWindow entries past the block's first) is outside the range and reads as column 0, value 0
   auto load_entries = [&](const Bnd (&d)[PPL], int round, Ent (&en)[PPL]) __attribute__((always_inline)) {
-    const int64_t left = max(min(a.ncap - ebase, (int64_t)1 << 24), (int64_t)0);
+    const int64_t left = max(min(a.ncap - ebase, La::kWindow), (int64_t)0);
     const __amdgpu_buffer_rsrc_t rc = uniform_rsrc(const_cast<int64_t*>(a.ocol + ebase), (uint32_t)(left * 8));
     const __amdgpu_buffer_rsrc_t rv = uniform_rsrc(const_cast<uint16_t*>(a.oval + ebase), (uint32_t)(left * 2));
 #pragma unroll
@@ -790,7 +791,7 @@ __global__ __launch_bounds__(256) void k_legacy_apply(LegacyArgs a, int RBW, int
         const int64_t e = d[h].s0 + LPP * (SL * round + k) + lane % LPP;
         const int64_t rel = e - ebase;
         const uint32_t c = en[h].col[k] - (uint32_t)cbase;
-        if (e < d[h].s1 && rel >= 0 && rel < (1 << 24) && c < 64u) {
+        if (e < d[h].s1 && rel >= 0 && rel < La::kWindow && c < 64u) {
           // (chunk c / 8 of row r at position (c / 8) ^ (r % 8))
           uint16_t* o = reinterpret_cast<uint16_t*>(otile + pi * 128 + 16 * ((c >> 3) ^ (pi & 7)));
           o[c & 7u] = clear ? (uint16_t)0 : (uint16_t)en[h].val[k];
@@ -1735,10 +1736,13 @@ static int legacy_launch(const LegacyArgs& a, int K, int64_t B, bool mfma_ok, hi
   const int64_t NB = a.N / NP;
   const int rb = legacy_rows_per_wg(a.M, NB / 64 * B);
   const int64_t nwg = (a.M + 64 * rb - 1) / (64 * rb) * (NB / 64) * B;
-  // (the MFMA decode's store and entry ranges cover 16 rows)
+  // k_legacy_apply's store range covers 16 rows of fewer than 2^26 columns (32-bit offsets, past which a
+  // dropped lane's offset lies), its entry range kWindow entries of those.  Other shapes take the scalar
+  // kernel (at [64, 2^21] 2 bits 140 us against 3.8 ms)
   constexpr bool kApply = (MODE == kDecode && OSRC != 1) || MODE == kFusedStore || MODE == kFusedSilu ||
                           MODE == kFusedMul;
-  const bool fits = !kApply || 16 * a.N <= ((int64_t)1 << 24);
+  constexpr int64_t kWindow = LegacyApply<kDecode, BITS, 1>::kWindow;
+  const bool fits = !kApply || (32 * a.N <= 0x7ffffff0 && (OSRC == 0 || 16 * a.N <= kWindow || a.ncap <= kWindow));
   if (mfma_ok && fits && NB % 64 == 0 && nwg <= INT32_MAX) {
     // 4 row blocks per workgroup, fewer where that would leave under two workgroups per CU
     LegacyArgs la = a;
@@ -1968,7 +1972,7 @@ extern "C" int lrq_legacy_dequant_gemm(const void* l, const void* rt, int32_t K,
   a.n_out = n_out;
   const int64_t NB = N / (8 / bits);
   const bool mfma_ok = vec_ok({l, rt, q, s}) && NB % 64 == 0 && n_out % 16 == 0 && aligned(y, 8) && ldy % 4 == 0 &&
-                       NB <= (int64_t)1 << 24 && ldy <= (int64_t)1 << 23;  // (32-bit lane offsets)
+                       NB <= (int64_t)1 << 26 && ldy <= (int64_t)1 << 25;  // (32-bit lane offsets: 63 rows)
   hipStream_t hs = (hipStream_t)stream;
   switch (bits) {
     case 1: return legacy_gemm_bits<1>(a, K, B, mfma_ok, hs);
