@@ -359,6 +359,18 @@ def test_encode_any_direct_loads_stay_in_bounds(cus, bits):
 
 
 # ----------------------------------------------------------------------------- k_legacy_encode
+def _legacy_run_blocks(groups, nrb, cus):
+    """legacy_run_blocks(): row blocks per run."""
+    best, least = 1, None
+    for r in range(1, 17):
+        per_cu = -(-groups * -(-nrb // r) // cus)
+        if r > 1 and per_cu < (3 if groups * nrb >= 24 * cus else 2):
+            break
+        if least is None or per_cu * (4 * r + 3) < least:
+            best, least = r, per_cu * (4 * r + 3)
+    return best
+
+
 def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits):
     """k_legacy_encode<bits, ...> as legacy_launch() launches it: every request of every wave, and the
     read-back of every slot (lane (j, g): columns 16g .. 16g + 15 of row j)."""
@@ -368,7 +380,7 @@ def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits):
     WAVE = RING * SLOT + NP * 64 * 4 + 16 * NP * 8
     nrb, nu = (M + 15) // 16, NB // 64
     ug = (nu + 3) // 4
-    rbw = max(1, min(16, B * ug * nrb // (4 * cus)))
+    rbw = _legacy_run_blocks(B * ug, nrb, cus)
     nrun = (nrb + rbw - 1) // rbw
     lane = np.arange(64)
     j, g = lane & 15, lane >> 4
@@ -412,6 +424,18 @@ def test_legacy_encode_direct_loads_stay_in_bounds(cus, bits):
     for B, M, N, extra in [(1, 1, 512, 0), (2, 100, 1024, 8), (1, 40, 1536, 0), (3, 37, 2048, 0), (1, 2100, 512, 0)]:
         n += legacy_encode_replay(B, M, N, N + extra, M * (N + extra), cus, bits)
     assert n > 0
+
+
+@pytest.mark.parametrize("B,M,N,bits", [(4, 3072, 3072, 1), (4, 3072, 3072, 2), (4, 3072, 3072, 4), (4, 3072, 3072, 8),
+                                        (2, 5253, 2560, 1), (2, 5253, 2560, 8), (4, 1024, 1024, 8), (4, 8192, 8192, 1)])
+def test_legacy_runs_spread_over_the_cus(B, M, N, bits):
+    """The run length of k_legacy_encode and k_legacy_apply leaves the busiest of 256 CUs at most half more
+    than the mean number of row blocks, a run's set-up counted as 3/4 of one (lengths from the mean alone
+    came to 1.75 times)."""
+    groups, nrb = B * ((N * bits // 8 // 64 + 3) // 4), (M + 15) // 16
+    r = _legacy_run_blocks(groups, nrb, 256)
+    busiest = -(-groups * -(-nrb // r) // 256) * (r + 0.75)
+    assert 1 <= r <= 16 and busiest <= 1.5 * groups * nrb / 256
 
 
 def test_replay_catches_a_planted_overrun():

@@ -1694,6 +1694,27 @@ static int legacy_rows_per_wg(int64_t M, int64_t wg_cols) {
   return 1;
 }
 
+// Row blocks per run of k_legacy_encode and k_legacy_apply (up to 16): the length that gives the busiest CU
+// the fewest blocks, a run's set-up (operands, tables, the first loads) counted as 3/4 of one, with at least
+// two workgroups per CU where there is the work (three from 24 blocks a CU up: at [4, 8192, 8192], 1 bit,
+// runs of 16 leave two, SiLU gradient 223 -> 232 us).  A length taken from the mean alone left CUs with one run
+// more than the others: [4, 3072, 3072], us with the mean's length -> with this one (before the streamed
+// kernels): staged encode + compaction 8 bits 55.0 -> 47.2 (42.4), 4 bits 46.7 -> 42.3 (44.3), 1 bit of rank
+// 32 77.1 -> 58.7 (61.3), 2 bits 44.1 -> 39.6 (52.5); SiLU gradient 1 bit 44.7 -> 36.4 (39.5).
+static int64_t legacy_run_blocks(int64_t B, int64_t ug, int64_t nrb) {
+  const int64_t cus = cu_count();
+  int64_t best = 1, least = INT64_MAX;
+  for (int64_t r = 1; r <= 16; ++r) {
+    const int64_t per_cu = (B * ug * ((nrb + r - 1) / r) + cus - 1) / cus;
+    if (r > 1 && per_cu < (B * ug * nrb >= 24 * cus ? 3 : 2)) break;
+    if (per_cu * (4 * r + 3) < least) {
+      least = per_cu * (4 * r + 3);
+      best = r;
+    }
+  }
+  return best;
+}
+
 // The row-tile decode (k_legacy_rows) for dense COO outliers at 2, 4 and 8 bits from 2^27 elements up,
 // where the COO entries outgrow the caches and their longer contiguous ranges pay (16 % outliers, 2
 // bits: [4, 8192, 8192] 340 us against 352 - 370 us for k_legacy_apply; [4, 3072, 3072] 60 against 50).
@@ -1749,9 +1770,8 @@ static int legacy_launch(const LegacyArgs& a, int K, int64_t B, bool mfma_ok, hi
     la.rb = rb;
     const dim3 grid((unsigned)nwg);
     if constexpr (MODE == kEncode) {
-      // runs of up to 16 row blocks, shorter where that would leave under four workgroups per CU
       const int64_t ug = (NB / 64 + 3) / 4, nrb = (a.M + 15) / 16;
-      const int64_t rbw = std::max<int64_t>(1, std::min<int64_t>(16, B * ug * nrb / (4 * (int64_t)cu_count())));
+      const int64_t rbw = legacy_run_blocks(B, ug, nrb);
       const int64_t wgs = (nrb + rbw - 1) / rbw * ug * B;
       if (wgs > INT32_MAX) return LRQ_ERR_SHAPE;
       const dim3 eg((unsigned)wgs);
@@ -1759,7 +1779,7 @@ static int legacy_launch(const LegacyArgs& a, int K, int64_t B, bool mfma_ok, hi
       return launch((k_legacy_encode<BITS, 32, OSRC == 1>), eg, dim3(256), 0, st, a, (int)rbw, (int)ug);
     } else if constexpr (kApply) {
       const int64_t ug = (NB / 64 + 3) / 4, nrb = (a.M + 15) / 16;
-      const int64_t rbw = std::max<int64_t>(1, std::min<int64_t>(16, B * ug * nrb / (4 * (int64_t)cu_count())));
+      const int64_t rbw = legacy_run_blocks(B, ug, nrb);
       const int64_t wgs = (nrb + rbw - 1) / rbw * ug * B;
       if (wgs > INT32_MAX) return LRQ_ERR_SHAPE;
       const dim3 eg((unsigned)wgs);
