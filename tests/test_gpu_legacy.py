@@ -727,6 +727,23 @@ def test_legacy_encode_non_finite_scales(pkg, dev, bits, K):
     assert np.array_equal(O.bf16_to_f32(og), O.bf16_to_f32(o_ref))
 
 
+@pytest.mark.parametrize("B,M,N", [(1, 16, 512), (2, 37, 1536), (1, 700, 2560)])
+def test_legacy_encode_one_bit_rank_32(pkg, dev, B, M, N):
+    """The 1-bit rank-32 encode (the last planes' operands in LDS): units that do not fill a group of four,
+    several row blocks per run, a plane in the element form."""
+    tau = 5.0
+    l, r, x, s = _inputs(600 + N, B, M, N, 32, B)
+    x[0, M // 2, N - 1], s[0, N - 64] = float("inf"), 2.0 ** 110
+    with np.errstate(all="ignore"):
+        o_ref, q_ref = O.legacy_encode(bits16(l), bits16(r), bits16(x), bits16(s), 1, tau)
+    o_sp, q = pkg.low_rank_addition_fuse_compression_quantization(l.to(dev), r.to(dev), x.to(dev), s.to(dev), 1, tau)
+    qg, og = q.cpu().numpy(), bits16(o_sp.to_dense())
+    q_ref[0, M // 2, N // 8 - 1] = qg[0, M // 2, N // 8 - 1]  # (its own code comes of inf - inf)
+    assert _frac_mismatch(qg, q_ref) <= TIE_BUDGET
+    nz = (O.bf16_to_f32(o_ref) != 0) | (O.bf16_to_f32(og) != 0)
+    assert _frac_mismatch(og[nz], o_ref[nz]) <= TIE_BUDGET
+
+
 # the MFMA decode (k_legacy_apply) where it can go wrong: units that do not fill a group of four, one
 # row, ragged last blocks, several runs; densities below and above the entries requested ahead; every
 # bit width and rank

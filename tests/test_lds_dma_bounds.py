@@ -371,13 +371,13 @@ def _legacy_run_blocks(groups, nrb, cus):
     return best
 
 
-def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits):
-    """k_legacy_encode<bits, ...> as legacy_launch() launches it: every request of every wave, and the
+def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits, K):
+    """k_legacy_encode<bits, K, ...> as legacy_launch() launches it: every request of every wave, and the
     read-back of every slot (lane (j, g): columns 16g .. 16g + 15 of row j)."""
     NP = 8 // bits
     NB = N // NP
     RING, SLOT = 4, 16 * 128
-    WAVE = RING * SLOT + NP * 64 * 4 + 16 * NP * 8
+    WAVE = RING * SLOT + NP * 64 * 4 + 16 * NP * 8 + (2 * 4 * 64 * 16 if bits == 1 and K == 32 else 0)
     nrb, nu = (M + 15) // 16, NB // 64
     ug = (nu + 3) // 4
     rbw = _legacy_run_blocks(B * ug, nrb, cus)
@@ -422,7 +422,8 @@ def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits):
 def test_legacy_encode_direct_loads_stay_in_bounds(cus, bits):
     n = 0
     for B, M, N, extra in [(1, 1, 512, 0), (2, 100, 1024, 8), (1, 40, 1536, 0), (3, 37, 2048, 0), (1, 2100, 512, 0)]:
-        n += legacy_encode_replay(B, M, N, N + extra, M * (N + extra), cus, bits)
+        for K in (16, 32) if bits == 1 else (16,):  # (the rank changes the layout at 1 bit only)
+            n += legacy_encode_replay(B, M, N, N + extra, M * (N + extra), cus, bits, K)
     assert n > 0
 
 

@@ -446,17 +446,21 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
 // pieces it cannot hold; else the dense outliers.  A block's 16 NP records are gathered in LDS, each
 // lane writing the entries it holds (usually none or one: the or of its masked values), and leave
 // as one 8-byte store per record.
-template <int BITS>
+// At 1 bit and rank 32 the r^T operands of eight planes (128 registers) spilled inside the loop, and the
+// reloads waited in the ring's memory queue: the last LP planes' live in LDS (with 3 one workgroup per CU
+// would be left).  With the compaction [4, 4096, 4096] 82.5 -> 59.6 us, [4, 8192, 8192] 229 -> 186 us.
+template <int BITS, int K>
 struct LegacyEnc {
   static constexpr int NP = 8 / BITS, NW = 4, RING = 4, SLOT = 16 * 128, NREC = 16 * NP;
-  static constexpr int TAB = NP * 64 * 4, WAVE = RING * SLOT + TAB + NREC * 8;  // bytes per wave
+  static constexpr int LP = BITS == 1 && K == 32 ? 2 : 0;
+  static constexpr int TAB = NP * 64 * 4, WAVE = RING * SLOT + TAB + NREC * 8 + LP * 4 * 64 * 16;  // bytes per wave
   static constexpr int kStepOps = 4;  // memory operations per step: two loads, two (dense outlier) stores
 };
 template <int BITS, int K, bool STAGED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1 : BITS >= 2 && K == 16 ? 3 : 2))) void k_legacy_encode(
     LegacyArgs a, int RBW, int ug) {
-  using Le = LegacyEnc<BITS>;
-  constexpr int NP = Le::NP, G = 64, E = 16, RT = K / 16, RING = Le::RING, SLOT = Le::SLOT, NREC = Le::NREC;
+  using Le = LegacyEnc<BITS, K>;
+  constexpr int NP = Le::NP, G = 64, E = 16, RT = K / 16, RING = Le::RING, SLOT = Le::SLOT, NREC = Le::NREC, VREG = NP - Le::LP;
   __shared__ __attribute__((aligned(16))) unsigned char lds[Le::NW][Le::WAVE];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int j = lane & 15, g = lane >> 4;
@@ -491,9 +495,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1
     for (int k = 0; k < RT; ++k) nl[k] = ld8(a.l + rn * K + 16 * k + 4 * g);
   };
   fetch_l(0);
-  u32x2 vop[NP][4][RT];
+  u32x2 vop[VREG][4][RT];
 #pragma unroll
-  for (int p = 0; p < NP; ++p) load_vops<G, K>(a.rt, unit_base(p, u, N, NP, G), j, g, vop[p]);
+  for (int p = 0; p < VREG; ++p) load_vops<G, K>(a.rt, unit_base(p, u, N, NP, G), j, g, vop[p]);
+  u32x4* const vlds = reinterpret_cast<u32x4*>(ring + RING * SLOT + Le::TAB + NREC * 8) + lane;  // [LP][4][64]
+  if constexpr (Le::LP > 0) {
+#pragma unroll 1
+    for (int p = 0; p < Le::LP; ++p) {
+      u32x2 v[4][RT];
+      load_vops<G, K>(a.rt, unit_base(VREG + p, u, N, NP, G), j, g, v);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) vlds[(p * 4 + q) * 64] = u32x4{v[q][0][0], v[q][0][1], v[q][RT - 1][0], v[q][RT - 1][1]};
+    }
+  }
+  auto lowrank = [&](auto pc, const u32x2* lo, f32x4 (&t)[4]) __attribute__((always_inline)) {  // plane pc's fp32(l r)
+    constexpr int p = decltype(pc)::value;
+    if constexpr (p < VREG) {
+      legacy_lowrank_mfma<K>(vop[p], lo, t);
+    } else {
+      u32x2 v[4][RT];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 d = vlds[((p - VREG) * 4 + q) * 64];
+        v[q][0] = u32x2{d[0], d[1]};
+        v[q][RT - 1] = u32x2{d[2], d[3]};
+      }
+      legacy_lowrank_mfma<K>(v, lo, t);
+    }
+  };
   // fast: the estimate serves every scale of the unit and the threshold is not negative
   int ok = a.tau >= 0.f ? 1 : 0;
   float smin = INFINITY;
@@ -550,7 +579,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1
       const u32x4 x1 = *reinterpret_cast<const u32x4*>(xs + 16 * ((2 * g + 1) ^ (j & 7)));
       const u32x4 rc = *reinterpret_cast<const u32x4*>(rtab + p * 64 + (g * 4 + (j & 3)) * 4);
       f32x4 tl[4], tx[4];
-      legacy_lowrank_mfma<K>(vop[p], lop, tl);
+      lowrank(pc, lop, tl);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slot is read
       __builtin_amdgcn_sched_barrier(0);
       // (past the run the last block is requested again: unused)
@@ -581,7 +610,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1
         const uint16_t* xp = a.x + (int64_t)b * a.ldx_b + rr * a.ldx_m + c0;
         unpack8(ld16(xp), xv);
         unpack8(ld16(xp + 8), xv + 8);
-        legacy_lowrank_mfma<K>(vop[p], lop, tl);
+        lowrank(pc, lop, tl);
         hm = 0;
 #pragma unroll
         for (int e = 0; e < E; ++e) lr[e] = tl[e >> 2][e & 3];
@@ -1700,7 +1729,7 @@ static int legacy_rows_per_wg(int64_t M, int64_t wg_cols) {
 // runs of 16 leave two, SiLU gradient 223 -> 232 us).  A length taken from the mean alone left CUs with one run
 // more than the others: [4, 3072, 3072], us with the mean's length -> with this one (before the streamed
 // kernels): staged encode + compaction 8 bits 55.0 -> 47.2 (42.4), 4 bits 46.7 -> 42.3 (44.3), 1 bit of rank
-// 32 77.1 -> 58.7 (61.3), 2 bits 44.1 -> 39.6 (52.5); SiLU gradient 1 bit 44.7 -> 36.4 (39.5).
+// 32 77.1 -> 58.7 (61.3; 50.2 without its spills), 2 bits 44.1 -> 39.6 (52.5); SiLU gradient 1 bit 44.7 -> 36.4 (39.5).
 static int64_t legacy_run_blocks(int64_t B, int64_t ug, int64_t nrb) {
   const int64_t cus = cu_count();
   int64_t best = 1, least = INT64_MAX;
