@@ -854,6 +854,23 @@ def test_legacy_rows_largest_dense_coo(pkg, dev, bits, K):
     assert torch.equal(dec(l, r, q, oc.check(), s, quantize_bit=bits), dec(l, r, q, o, s, quantize_bit=bits))
 
 
+@pytest.mark.parametrize("M,N,K,share", [(16400, 4096, 16, 0.04), (8200, 8192, 32, 0.035), (16400, 2048, 16, 0.2), (16400, 2048, 32, 0.1)])
+def test_legacy_decode_four_bits_by_density(pkg, dev, M, N, K, share):
+    """Four-bit decodes on both sides of the line between the two COO decodes (elements, entries) give the
+    dense decode's bits."""
+    dec = pkg.low_rank_addition_fuse_decompression_dequantization
+    g = torch.Generator(device=dev).manual_seed(N)
+    l = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    r = torch.randn(K, N, generator=g, device=dev).to(torch.bfloat16)
+    s = (torch.randn(1, N, generator=g, device=dev) + 2).to(torch.bfloat16)
+    q = torch.randint(0, 256, (1, M, N // 2), generator=g, device=dev, dtype=torch.uint8)
+    o = torch.randn(1, M, N, generator=g, device=dev) * (torch.rand(1, M, N, generator=g, device=dev) < share)
+    o = o.to(torch.bfloat16)
+    want = dec(l, r, q, o, s, quantize_bit=4)
+    for cap in (int((o != 0).sum()), o.numel() // 4):
+        assert torch.equal(dec(l, r, q, pkg.compact_outliers(o, capacity=cap), s, quantize_bit=4), want), cap
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 1, 1), (65, 8, 63), (64, 16, 64), (130, 17, 1000), (3, 32, 65), (200, 31, 8), (5, 0, 70)])
 def test_legacy_factors(pkg, dev, M, K, N):
     """r transposed and l, r zero-padded to 16 or 32 ranks."""

@@ -1744,10 +1744,22 @@ static int64_t legacy_run_blocks(int64_t B, int64_t ug, int64_t nrb) {
   return best;
 }
 
-// The row-tile decode (k_legacy_rows) for dense COO outliers at 2, 4 and 8 bits from 2^27 elements up,
-// where the COO entries outgrow the caches and their longer contiguous ranges pay (16 % outliers, 2
-// bits: [4, 8192, 8192] 340 us against 352 - 370 us for k_legacy_apply; [4, 3072, 3072] 60 against 50).
-// Runs of whole ring rounds (PD blocks).  Returns false where it does not apply.
+// Whether k_legacy_rows decodes n COO entries in E elements faster than k_legacy_apply: where the codes and
+// entries come from HBM, its longer contiguous entry ranges pay.  Times in us of both, inputs that are not
+// in the caches / inputs of the pass before (rank 16):
+//   4 bits  [4, 4096, 4096] 2 %: 56 and 59 / 57 and 36;  5 %: 57 and 71 / 59 and 44;  16 %: 70 and 79 / 69 and 63
+//           [4, 8192, 8192] 2 %: 198 and 216 / 202 and 128;  3.5 %: 203 and 230 / 206 and 222
+//           [4, 2048, 4096] 8 %: 34 and 36 / 34 and 28;  30 %: 54 and 65 / 47 and 57
+//   2 bits  [4, 4096, 4096] 16 %: 89 and 94 / 77 and 68;  [4, 8192, 4096] 8 %: 139 and 132 / 122 and 90;
+//           16 %: 169 and 181 / 148 and 168
+//   8 bits  [4, 8192, 4096] 8 %: 139 and 134 / 144 and 128;  16 %: 151 and 155 / 143 and 155
+static bool legacy_rows_pays(int bits, int64_t E, int64_t n) {
+  if (bits == 4) return (E >= ((int64_t)1 << 26) && n * 32 > E) || (E >= ((int64_t)1 << 25) && n * 6 > E);
+  return (bits == 2 || bits == 8) && E >= ((int64_t)1 << 27) && n * 8 > E;
+}
+
+// The row-tile decode (k_legacy_rows), in runs of whole ring rounds (PD blocks).  Returns false where it does
+// not apply.
 template <int MODE, int BITS, int OSRC>
 static bool legacy_rows_launch(const LegacyArgs& a, int K, int64_t B, hipStream_t st, int* status) {
   if constexpr (MODE != kDecode || OSRC != 3 || BITS == 1) {
@@ -1755,7 +1767,7 @@ static bool legacy_rows_launch(const LegacyArgs& a, int K, int64_t B, hipStream_
   } else {
     using Lr = LegacyRows<BITS>;
     const int64_t NB = a.N / Lr::NP, nu = NB / 64, nrb = (a.M + 15) / 16;
-    if (B * a.M * a.N < ((int64_t)1 << 27) || a.ncap == 0) return false;
+    if (!legacy_rows_pays(BITS, B * a.M * a.N, a.ncap)) return false;
     if (NB % 64 != 0 || nu < Lr::NW || 16 * a.N * 2 >= ((int64_t)1 << 31)) return false;
     const int64_t ug = (nu + Lr::NW - 1) / Lr::NW, tiles = B * ug;
     const int64_t want = 2 * (int64_t)cu_count();
@@ -2062,8 +2074,8 @@ extern "C" int lrq_legacy_decode_coo(const void* l, const void* rt, int32_t K, c
   a.optr = piece_ptr, a.ocol = cols, a.oval = (const uint16_t*)vals, a.npc = (N + 63) / 64, a.ncap = n_entries;
   const bool mfma_ok = vec_ok({l, rt, q, s, out}) && N % 8 == 0;
   // more than about 4 entries per 64-column piece (1/16 of the elements): more of a piece's entries are
-  // requested ahead (k_legacy_apply), or the row-tile decode (legacy_rows_launch)
-  if (mfma_ok && n_entries * 16 > B * M * N) return legacy_bits<kDecode, 3>(a, K, B, bits, mfma_ok, (hipStream_t)stream);
+  // requested ahead (k_legacy_apply), or the row-tile decode (legacy_rows_pays)
+  if (mfma_ok && (n_entries * 16 > B * M * N || legacy_rows_pays(bits, B * M * N, n_entries))) return legacy_bits<kDecode, 3>(a, K, B, bits, mfma_ok, (hipStream_t)stream);
   return legacy_bits<kDecode, 2>(a, K, B, bits, mfma_ok, (hipStream_t)stream);
 }
 
