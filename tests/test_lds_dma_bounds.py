@@ -1,9 +1,9 @@
 """CPU replay of the direct global-to-LDS loads (ld16_to_lds, csrc/lrq_common.h).
 
-Six kernels move 16 bytes per lane from global memory straight into LDS with
+Seven kernels move 16 bytes per lane from global memory straight into LDS with
 __builtin_amdgcn_global_load_lds: k_encode_rows, k_encode_tiles and k_encode_any (csrc/lrq_encode.hip),
-k_softmax_rows (csrc/lrq_rowops.hip), k_wht_rows (csrc/lrq_wht.hip) and k_legacy_encode
-(csrc/lrq_legacy.hip).  This file restates, in numpy, the
+k_softmax_rows (csrc/lrq_rowops.hip), k_wht_rows (csrc/lrq_wht.hip), k_legacy_encode and
+k_legacy_apply (csrc/lrq_legacy.hip).  This file restates, in numpy, the
 host launch arithmetic (grid, row blocks per workgroup) and each kernel's source and
 destination address arithmetic, and checks for every instance and launch shape that the
 library's callers use (bench.py's configurations and the GPU tests' shapes) that
@@ -13,9 +13,8 @@ library's callers use (bench.py's configurations and the GPU tests' shapes) that
     region (encode) or the block's tile (softmax, rotation),
   * no two lanes of one workgroup write the same LDS bytes for one row block.
 
-For k_encode_tiles, whose tiles are swizzled (chunk c of tile row r at position c ^ r), the
-replay also checks that the read-back (projection / quantisation layout and the rotation's
-layout) finds every column where the loads put it.
+For the kernels whose LDS is swizzled (k_encode_tiles, k_encode_any, k_legacy_encode and
+k_legacy_apply) the replay also checks that every read-back finds every column where the loads put it.
 
 No GPU is needed; a change to any of these kernels' addressing must be mirrored here.
 """
@@ -371,13 +370,13 @@ def _legacy_run_blocks(groups, nrb, cus):
     return best
 
 
-def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits, K):
-    """k_legacy_encode<bits, K, ...> as legacy_launch() launches it: every request of every wave, and the
-    read-back of every slot (lane (j, g): columns 16g .. 16g + 15 of row j)."""
+def legacy_ring_replay(B, M, N, ldx_m, ldx_b, cus, bits, WAVE, what):
+    """k_legacy_encode (its x) and k_legacy_apply (its y) as legacy_launch() launches them, WAVE bytes of
+    LDS per wave with the ring first: every request of every wave, and the read-back of every slot (lane
+    (j, g): columns 16g .. 16g + 15 of row j) from what the slot holds at that step."""
     NP = 8 // bits
     NB = N // NP
     RING, SLOT = 4, 16 * 128
-    WAVE = RING * SLOT + NP * 64 * 4 + 16 * NP * 8 + (2 * 4 * 64 * 16 if bits == 1 and K == 32 else 0)
     nrb, nu = (M + 15) // 16, NB // 64
     ug = (nu + 3) // 4
     rbw = _legacy_run_blocks(B * ug, nrb, cus)
@@ -398,32 +397,58 @@ def legacy_encode_replay(B, M, N, ldx_m, ldx_b, cus, bits, K):
             steps = [(min(st // NP, nblk - 1), st % NP, st) for st in range(RING)]
             steps += [(min(i + (p + RING) // NP, nblk - 1), (p + RING) % NP, (i * NP + p) % RING)
                       for i in range(nblk) for p in range(NP)]
-            held = {}
+            held = {}  # slot -> (block, plane, first column, chunk held at each position of each row)
+
+            def read_back(i, p, slot):
+                hi, hp, col0, col = held[slot]
+                assert (hi, hp) == (i, p) and col0 == u * 64 + p * NB, "the slot holds another step"
+                for h in range(2):
+                    assert (col[j, (2 * g + h) ^ (j & 7)] == 2 * g + h).all()
+
             for n, (i, p, slot) in enumerate(steps):
+                if n >= RING:  # (each step reads its slot, then requests it again)
+                    read_back((n - RING) // NP, (n - RING) % NP, slot)
                 col = np.empty((16, 8), dtype=np.int64)  # chunk held at each position of each row
                 for k in range(2):
                     r = 8 * k + lane // 8
                     row = np.minimum((rb0 + i) * 16 + r, M - 1)
                     c = u * 64 + 8 * ((lane & 7) ^ (lane >> 3)) + p * NB
                     gsrc = (b * ldx_b + row * ldx_m + c) * 2
+                    assert (gsrc % 16 == 0).all()
                     ldst = w * WAVE + slot * SLOT + 1024 * k + 16 * lane
                     _check(gsrc, ldst, gbytes=((B - 1) * ldx_b + (M - 1) * ldx_m + N) * 2, lds_alloc=4 * WAVE,
-                           lo=w * WAVE + slot * SLOT, hi=w * WAVE + (slot + 1) * SLOT, what=f"k_legacy_encode {M}x{N} {bits}")
+                           lo=w * WAVE + slot * SLOT, hi=w * WAVE + (slot + 1) * SLOT, what=f"{what} {M}x{N} {bits}")
                     col[r, lane & 7] = (c - u * 64 - p * NB) // 8
                     checked += 64
-                held[slot] = (n, col)
-                for h in range(2):
-                    assert (col[j, (2 * g + h) ^ (j & 7)] == 2 * g + h).all()
+                held[slot] = (i, p, u * 64 + p * NB, col)
     return checked
+
+
+# (batches, rows, columns, row padding): one row, ragged blocks, unit counts that are no multiple of four,
+# several blocks per run
+RING_SHAPES = [(1, 1, 512, 0), (2, 100, 1024, 8), (1, 40, 1536, 0), (3, 37, 2048, 0), (1, 2100, 512, 0), (2, 5003, 512, 8)]
 
 
 @pytest.mark.parametrize("bits", [1, 2, 4, 8])
 @pytest.mark.parametrize("cus", CU_COUNTS)
 def test_legacy_encode_direct_loads_stay_in_bounds(cus, bits):
     n = 0
-    for B, M, N, extra in [(1, 1, 512, 0), (2, 100, 1024, 8), (1, 40, 1536, 0), (3, 37, 2048, 0), (1, 2100, 512, 0)]:
+    NP = 8 // bits
+    for B, M, N, extra in RING_SHAPES:
         for K in (16, 32) if bits == 1 else (16,):  # (the rank changes the layout at 1 bit only)
-            n += legacy_encode_replay(B, M, N, N + extra, M * (N + extra), cus, bits, K)
+            wave = 4 * 2048 + NP * 64 * 4 + 16 * NP * 8 + (2 * 4 * 64 * 16 if bits == 1 and K == 32 else 0)
+            n += legacy_ring_replay(B, M, N, N + extra, M * (N + extra), cus, bits, wave, "k_legacy_encode")
+    assert n > 0
+
+
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("cus", CU_COUNTS)
+def test_legacy_apply_direct_loads_stay_in_bounds(cus, bits):
+    """The consumers' y (contiguous rows and batches) through the ring; behind it the scale table and the
+    result tile."""
+    n = 0
+    for B, M, N, _ in RING_SHAPES:
+        n += legacy_ring_replay(B, M, N, N, M * N, cus, bits, 4 * 2048 + 8 // bits * 64 * 4 + 2048, "k_legacy_apply")
     assert n > 0
 
 
