@@ -7,10 +7,12 @@
  *        b = 1:        q >= -(0.5 + 2^-9)  (one compare, no rounding), and
  *        b = 2, 4, 8:  clamp(bits(d + 1.5 * 2^23), B - 2^(b-1), B + 2^(b-1) - 1) - B + 2^(b-1),
  *                      d = bf16(q), B = bits(1.5 * 2^23) (legacy_code_biased);
- *   2. for every finite bf16 a and bf16 sc with 2^-100 <= |sc| <= 2^100 (the scales the
- *      estimate serves) the quotient estimate a * RN32(1/sc) in place of RN32(a / sc): its code is
- *      the same at b = 1, 2, 4 and 8 (a / sc never comes near a code boundary within the
- *      estimate's error).
+ *   2. for every finite bf16 a and bf16 sc with 2^-100 <= |sc| <= 2^100 (rc_scale_ok) the two-term
+ *      quotient in place of RN32(a / sc): 1/sc = r1 + r2, r1 = bf16(RN32(1/sc)), r2 = bf16(RN32(1/sc) - r1)
+ *      (legacy_rc_split), a r1 (exact) and then a r2 added with one rounding; at b = 1 the threshold
+ *      0.5 + 2^-9 is added to a r1 first, and the sum's sign bit is the code's complement.  Magnitudes from
+ *      2^118 |sc| up take the division (mag_limit).  The codes are the same at b = 1, 2, 4 and 8: a / sc,
+ *      a quotient of two bf16 values, is at least 2^-17 (relative) from a code boundary.
  * Prints the number of quotients checked and of mismatches of part 1 per bit width, then the
  * number of (a, sc) pairs checked and of mismatches of part 2 per bit width. */
 #include <math.h>
@@ -67,13 +69,19 @@ int main(void) {
     const float sc = from_bits((uint32_t)s << 16);
     const float m = fabsf(sc);
     if (!(m >= 0x1p-100f && m <= 0x1p100f)) continue;
-    const float rc = 1.0f / sc;
+    const float rc = 1.0f / sc, r1 = bf16_round(rc), r2 = bf16_round(rc - r1);
+    const float lim = m * 0x1p118f;
+    uint32_t limit;
+    memcpy(&limit, &lim, 4);
+    limit >>= 16;
     for (int h = 0; h < 65536; ++h) {
       const float a = from_bits((uint32_t)h << 16);
       if (!isfinite(a)) continue;
       ++pairs;
-      const float est = a * rc, q = a / sc;
-      e1 += code(est, 1) != code(q, 1);
+      if (((uint32_t)h & 0x7fffu) >= limit) continue; /* the division */
+      const float est = fmaf(a, r2, a * r1), q = a / sc;
+      const float one = fmaf(a, r2, fmaf(a, r1, 0.5f + 0x1p-9f));
+      e1 += (signbit(one) ? 0 : 1) != code(q, 1);
       e2 += code(est, 2) != code(q, 2);
       e4 += code(est, 4) != code(q, 4);
       e8 += code(est, 8) != code(q, 8);

@@ -7,10 +7,10 @@ torch form: `(x - o) / s`, bf16, then round and clamp), exhaustively on the host
   bits the clamped bits of bf16(q) + 1.5 * 2^23; both equal clamp(rint(bf16(q))) + 2^(b-1) for
   every fp32 quotient but NaN;
 * the quotient: for every finite bf16 numerator and every bf16 scale with
-  2^-100 <= |s| <= 2^100, the estimate a * RN32(1/s) gives the IEEE quotient's code at 1, 2, 4
-  and 8 bits.
+  2^-100 <= |s| <= 2^100, the two-term product a r1 + a r2, 1/s = r1 + r2 in bf16, gives the IEEE
+  quotient's code at 1, 2, 4 and 8 bits (magnitudes of 2^118 |s| and more are divided).
 
-The check fails for a threshold of -0.5, a bias of 2^23, or an estimate off by 10^-4."""
+The check fails for a threshold of -0.5, a bias of 2^23, or a quotient of the first term alone."""
 
 from __future__ import annotations
 
@@ -33,7 +33,7 @@ def test_code_step_forms_give_the_reference_codes(tmp_path):
     checked, bad1, bad2, bad4, bad8, pairs, e1, e2, e4, e8 = map(int, out)
     assert checked == 2 ** 32 - 2 * (2 ** 23 - 1)  # every bit pattern but the NaNs
     assert (bad1, bad2, bad4, bad8) == (0, 0, 0, 0)
-    # scales: the 200 binades 2^-100 .. 2^99 (128 each) and 2^100, both signs; numerators: the
+    # two-term quotients.  Scales: the 200 binades 2^-100 .. 2^99 (128 each) and 2^100, both signs; numerators: the
     # 65280 finite bf16 values
     assert pairs == 2 * (200 * 128 + 1) * 65280
     assert (e1, e2, e4, e8) == (0, 0, 0, 0)
@@ -47,13 +47,13 @@ def _bf16(f: np.ndarray) -> np.ndarray:
 
 
 def test_two_term_quotient_gives_the_reference_codes():
-    """The encode's matrix-step quotient: 1/s as two bf16 terms r1 + r2, a r1 (exact) and then a r2
+    """The same without a compiler, at scales from the smallest to the largest served: 1/s as two bf16 terms r1 + r2, a r1 (exact) and then a r2
     added with one fp32 rounding (at 1 bit the threshold 0.5 + 2^-9 enters with a r1, and the sign is
     the code): its code is the IEEE quotient's for every pair of bf16 mantissas and signs at every
     exponent difference that can reach a code boundary (|q| from 2^-4 to 2^9; beyond, both clamp)."""
     man = np.arange(128, 256, dtype=np.float32)
     a0 = np.concatenate([man, -man])[:, None]
-    for es in (-100, -7, 0, 3, 92):
+    for es in (-107, -100, -93, -60, -31, -7, 0, 3, 24, 55, 92):  # (times 128 .. 255: 2^-100 .. 2^100)
         for sg in (1.0, -1.0):
             s = (sg * man * 2.0 ** es).astype(np.float32)[None, :]
             rc = (np.float32(1.0) / s).astype(np.float32)
