@@ -22,8 +22,10 @@
 // (what an fp32-accumulating GEMM returns up to the order of its additions).
 //
 // Two implementations with identical results:
-//   * k_legacy_encode / k_legacy_mfma — when every plane is a whole number of 64-column units and the
-//     operands are 16-byte aligned.  The unit layout of lrq_common.h (lane (j, g) owns 16 consecutive
+//   * on MFMA — when every plane is a whole number of 64-column units and the operands are 16-byte
+//     aligned: k_legacy_encode (encode), k_legacy_apply (decode with sparse or no outliers, fused
+//     consumers), k_legacy_rows (decode, denser sparse outliers of large tensors), k_legacy_mfma
+//     (decode from dense outliers, add, histogram), k_legacy_gemm (the product).  The unit layout of lrq_common.h (lane (j, g) owns 16 consecutive
 //     columns of its row in every plane) with l @ r rebuilt on MFMA exactly like the
 //     group-mode reconstruction (V = rt).
 //   * k_legacy_scalar — any shape: one thread per packed byte, l @ r summed in fp64 (the
@@ -96,9 +98,9 @@ __device__ __forceinline__ uint32_t legacy_code(float x, float lr, float sc, flo
 // - at 1 bit the code is 1 exactly when bf16(q) >= -0.5, i.e. when q >= -(0.5 + 2^-9) (below
 //   -0.5 the bf16 spacing is 2^-8, and the tie at -0.5 - 2^-9 rounds to the even -0.5): one
 //   compare of the quotient, no rounding.
-// The host checks compare the code forms with the reference's over every fp32 quotient but NaN
-// (tests/legacy_code_check.c) and the two-term product's codes with the IEEE quotient's over every pair
-// of bf16 mantissas (tests/test_legacy_division.py).
+// The host check tests/legacy_code_check.c compares the code forms with the reference's over every fp32
+// quotient but NaN, and the two-term product's codes with the IEEE quotient's over every finite bf16
+// numerator and every scale served.
 constexpr uint32_t kCodeBias = 0x4B400000u;  // bits of 1.5 * 2^23
 template <int BITS>
 __device__ __forceinline__ uint32_t legacy_code_biased(float d) {
@@ -235,8 +237,8 @@ __device__ __forceinline__ void legacy_lowrank_mfma(const u32x2 (&vop)[4][K / 16
 // The plane's outlier test and codes from the packed residuals w (w[k]: elements 2k, 2k + 1): hm bit e =
 // element e is an outlier, w becomes the outlier values (0 elsewhere), code[16] the codes
 // (legacy_code_biased; at 1 bit a word whose sign bit is the code's complement).  Returns whether some
-// magnitude of the lane reaches mag_limit (bf16 bits): hm, w and code are then unspecified.  aq: the LDS table of the plane's quotient operands (step q's two terms at aq[128 q],
-// aq[128 q + 64]).
+// magnitude of the lane reaches mag_limit (bf16 bits): hm, w and code are then unspecified.
+// rc[q]: r1 | r2 << 16 of column 4q + lane % 4 (legacy_rc_split), the two diagonals' bf16 bits in this lane's row.
 template <int BITS>
 __device__ __forceinline__ bool legacy_codes_mfma(uint32_t (&w)[8], uint32_t tau2, uint32_t mag_limit, u32x4 rc, int lane,
                                                   uint32_t (&code)[16], uint32_t& hm) {
@@ -1103,7 +1105,7 @@ __global__ __launch_bounds__(256) void k_legacy_scalar(LegacyArgs a, int K, int6
 }
 
 // ------------------------------------------------------------------ row-tile decode
-// Decode from dense COO outliers for the largest shapes (2, 4 or 8 bits), staged through an LDS
+// Decode from denser COO outliers of large tensors (2, 4 or 8 bits; legacy_rows_pays), staged through an LDS
 // tile so that the output leaves as whole row segments.  A workgroup of 4 waves owns 4 units
 // (wave w: unit u0 + w, i.e. 64 columns in every plane) of one batch over a run of RBW 16-row
 // blocks, with the unit's r^T operands in registers and the units' scales in LDS for the whole
