@@ -443,7 +443,8 @@ __global__ __launch_bounds__(256) void k_legacy_mfma(LegacyArgs a) {
 // accesses and stores moves the 604 MB of [4, 8192, 8192] at 2 bits in 126 us; loads in the MFMA
 // layout, four row blocks of one unit per workgroup, took 162 - 176 us.  The encode itself runs 152 us
 // there (218 us in that layout with the element work on the VALU; 184 us with it on the matrix pipe),
-// 155 us at 1 bit (202 us).
+// 155 us at 1 bit (202 us); 13.4 vector instructions per element at 1 bit, matrix steps included (22.4
+// before, without any).
 // STAGED: each 64-column piece's record (lrq_coo.h) goes to a.pcnt and the dense outliers only of the
 // pieces it cannot hold; else the dense outliers.  A block's 16 NP records are gathered in LDS, each
 // lane writing the entries it holds (usually none or one: the or of its masked values), and leave
@@ -700,8 +701,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!STAGED ? 1
 // - Element work on the matrix pipe (diagonal 4x4x4 steps, see legacy_codes_mfma): the codes enter as
 //   the bf16 values 128 + c (a byte permute, no conversion), a = s (128 + c) - s (128 + h) is exact in
 //   fp32 (h = 2^(b-1); at 8 bits c = 16 hi + lo takes two steps); then a's bf16 rounding (4 and 8 bits),
-//   + o and + bf16(l r) are identity steps with one rounding each, as in legacy_value.  About 3.5 vector
-//   instructions per element for x_hat, 11 - 16 before.
+//   + o and + bf16(l r) are identity steps with one rounding each, as in legacy_value.  The 2-bit COO
+//   decode issues 8.4 vector instructions per element, matrix steps included (row-tile decode 15.7).
 //   2-bit decode of [4, 8192, 8192] with 0.6 % outliers 209 -> 114 us, 1-bit 319 -> 115 us; SiLU gradient
 //   at [4, 4096, 4096] 97 -> 57.6 us a call.
 // - COO: the block's pieces (one per (row, plane)) take LPP lanes each; a lane's piece bounds are
@@ -1397,8 +1398,8 @@ struct LegacyGemmArgs {
 // formed element by element.
 // Bound by the operands' loads (every CU reads all of y and rt through L2: 512 KB at [4096, 32] each,
 // against 64 KB of codes) and their latency, two waves a SIMD: [4, 4096, 4096] 2 bits @ [4, 4096, 32], K = 32:
-// 32.9 -> 28.8 us, a call 36.9 -> 31.7: x_hat on the matrix pipe (about 2 vector instructions per element for
-// 7) with wave-uniform address bases gave 2.7 of that, y and the scales as 16-byte loads 2.5.
+// 32.9 -> 28.8 us, a call 36.9 -> 31.7: x_hat on the matrix pipe (5.5 vector instructions per element in all,
+// matrix steps included) with wave-uniform address bases gave 2.7 of that, y and the scales as 16-byte loads 2.5.
 template <int BITS, int K, int NOUT, int RB>
 __global__ __launch_bounds__(512) void k_legacy_gemm(LegacyGemmArgs a) {
   constexpr int NP = 8 / BITS, G = 64, E = 16, RT = K / 16, TO = NOUT / 16, NW = 8;
