@@ -250,8 +250,11 @@ constexpr int dma_units_after() {
 // projection is that of Y with those columns zeroed (the same products and sums) and their
 // residuals are zeroed before the group statistics; their bf16 values go to the fp16 side
 // columns from the slice in LDS.  LDS: Re::LDS + N/32 mask words + N slot entries.
+// Aligned to 2 KB: the same instructions at an odd multiple of 256 B took 61.7 us instead of 60.6
+// for a [16384, 4096] 4-bit rank-16 encode and decode in turn (each alone: within 0.1 us), so the
+// place does not depend on what is compiled before it.
 template <int BITS, int G, int R, int NW, int UPW, bool OUTL>
-__global__ __launch_bounds__(NW * 64) void k_encode_rows(
+__global__ __launch_bounds__(NW * 64) __attribute__((aligned(2048))) void k_encode_rows(
     const uint16_t* __restrict__ X, int64_t ldx, int M, int N, const uint16_t* __restrict__ V,
     uint16_t* __restrict__ Lout, int64_t ldl, uint8_t* __restrict__ codes, int64_t ldc,
     uint16_t* __restrict__ qparams, int64_t ldq, int RBW, const int32_t* __restrict__ oidx, int nout,
